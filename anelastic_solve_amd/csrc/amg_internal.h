@@ -23,13 +23,10 @@ namespace amg {
 // Coefficient table of one level (precision T): 3*nx + 3*ny + 3*nz values,
 //   [wxm | wxp | dx] [wym | wyp | dy] [wzm | wzp | dz]
 // with (A u)_ijk = wxm_i u_{i-1} + wxp_i u_{i+1} + ... + (dx_i+dy_j+dz_k) u_ijk.
+// The first 128 bytes are what nearly every kernel needs of a level, read in
+// one go (level_head in amg_kernels.hip).
 struct DevLevel {
   int nx, ny, nz, hx;
-  int px, py, pz;            // periodic flags
-  int inst;                  // instance id (batched/served runs)
-  int ncell;                 // nx*ny*nz
-  int link;                  // FP64 finest entry: index of the FP32 finest level (mixed)
-  int nullsp;                // the operator is singular (periodic/Neumann): constants in the null space
   // the instance's solve state, written by the device (the gate at the end
   // of every cycle) on every level of the instance:
   int stop;                  // the stop rule held: the instance's kernels return at once
@@ -37,13 +34,27 @@ struct DevLevel {
                              //   of a pair): the finest level's first sweep reads the iterate
   int skipc;                 // this cycle is the first of a pair: no FP64 correction after it
   int pcur;                  // FP64 pressure buffers of a mixed solve: 1 when u2 holds the current
+  unsigned gmhx, gmny;       // division of any 32-bit index by hx, ny: multiplier and
+  int gshx, gsny;            // shifts (s1 | s2 << 8) of gm_magic
+  int px, py, pz;            // periodic flags
+  int ncell;                 // nx*ny*nz
+  void* u;                   // solution / correction (chequer layout)
+  void* f;                   // right-hand side (chequer layout)
+  void* u2;                  // FP64 finest: ping-pong partner of u
+  const double* co64;        // coefficient table, FP64
+  const float* co32;         // coefficient table, FP32
+  const float* zt;           // FP32 z-line table of a level whose columns share one matrix
+                             // (k_zline_table), or null
+  const double* vol;         // [dxc(nx) | dyc(ny) | dzc(nz)] interior widths
+  const double* rho;         // rho(z) interior, nz values
+  int inst;                  // instance id (batched/served runs)
+  int link;                  // FP64 finest entry: index of the FP32 finest level (mixed)
+  int nullsp;                // the operator is singular (periodic/Neumann): constants in the null space
   int pairok;                // the instance may pair cycles (mixed, residual stop rule)
   int gslot;                 // the instance's slot in the per-instance gate array
   unsigned mhx, mny;         // ceil(2^32/hx), ceil(2^32/ny) (0 for a divisor of 1): e/hx = umulhi(e, mhx)
                              // exactly while e*hx < 2^32 (the coarse tail's small levels)
-  unsigned gmhx, gmny;       // division of any 32-bit index by hx, ny: multiplier and
-  int gshx, gsny;            // shifts (s1 | s2 << 8) of gm_magic
-  unsigned gmzp;             // the same for nz rounded up to a multiple of 16 (the direct
+  unsigned gmzp;             // gm_magic of nz rounded up to a multiple of 16 (the direct
   int gszp;                  // solve's padded z extent)
   int bcx0, bcx1, bcy0, bcy1, bcz0, bcz1;   // boundary codes (prolongation ghosts)
   double vsum;               // finest: sum of cell volumes
@@ -51,16 +62,9 @@ struct DevLevel {
   double bshift;             // mixed FP64 finest: the compatibility shift sum V b / sum V, which
                              // the outer step subtracts from b as it loads it (a state word:
                              // written by the first defect)
-  const double* co64;        // coefficient table, FP64
-  const float* co32;         // coefficient table, FP32
-  const double* vol;         // [dxc(nx) | dyc(ny) | dzc(nz)] interior widths
-  const double* rho;         // rho(z) interior, nz values
   const double* bcfold;      // [x(nx) | y(ny) | z(nz)] boundary-value RHS shifts (finest only)
   const double* minvT;       // coarsest level: transposed dense (pseudo-)inverse, ncell^2
   const double* minv;        // the same, row-major, when the coarse solve is its own kernel
-  void* u;                   // solution / correction (chequer layout)
-  void* u2;                  // FP64 finest: ping-pong partner of u
-  void* f;                   // right-hand side (chequer layout)
   void* scr;                 // z-line scratch: nz * hx * ny values
   // separable direct solve of a coarse level (amg_direct.cpp, k_direct_*)
   // the direct level's tables, in its compute type (FP64 for an FP64
@@ -243,6 +247,14 @@ constexpr int kZMaxSegs = 16;
 // form.  Both forms give the same bits.
 void launch_zline(bool fp64, const DevLevel* L, const LaunchList& ll, int parity,
                   int zero_guess, int segs, hipStream_t s, int form = 0);
+// The FP32 half-sweep of levels that hold a z-line table (DevLevel::zt), the
+// same bits as launch_zline's; 'segs' is the exact segment count of every
+// item.  The table's bytes, and its computation from the level's FP32
+// coefficient table.
+void launch_zline_shared(const DevLevel* L, const LaunchList& ll, int parity, int zero_guess, int segs,
+                         hipStream_t s);
+size_t zline_table_bytes(int nz);
+void launch_zline_table(const float* co32, int nx, int ny, int nz, float* zt, hipStream_t s);
 void launch_restrict(bool fp64, const DevLevel* L, const DevXfer* X, const LaunchList& ll,
                      hipStream_t s);
 // Residual + restriction marching in z, for a transfer with factor 2 in every

@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 
 namespace amg {
 namespace {
@@ -39,6 +40,40 @@ __device__ __forceinline__ int find_item(const int* prefix, int n, int b) {
     if (prefix[mid] <= b) lo = mid; else hi = mid - 1;
   }
   return lo;
+}
+
+// Keeps values in scalar registers from here on.  The compiler loads a
+// descriptor field where it is first used and waits for each: a kernel's
+// start was a chain of up to ten dependent scalar loads.  Pinning the fields
+// after reading them together leaves one round trip.
+template <class A, class... V> __device__ __forceinline__ void pin_s(A& a, V&... v);
+template <class A, class B, class C, class D, class E, class F, class G, class H, class... V>
+__device__ __forceinline__ void pin_s8(A& a, B& b, C& c, D& d, E& e, F& f, G& g, H& h, V&... v) {
+  asm("" : "+s"(a), "+s"(b), "+s"(c), "+s"(d), "+s"(e), "+s"(f), "+s"(g), "+s"(h));
+  if constexpr (sizeof...(V) > 0) pin_s(v...);
+}
+template <class A, class... V> __device__ __forceinline__ void pin_s(A& a, V&... v) {
+  if constexpr (sizeof...(V) >= 7) {
+    pin_s8(a, v...);
+  } else {
+    asm("" : "+s"(a));
+    if constexpr (sizeof...(V) > 0) pin_s(v...);
+  }
+}
+
+__device__ __forceinline__ int xcd_swizzle(int b, int n);
+// The item of this block and the block's number within it (blocks swizzled
+// over the XCDs).  A launch of one item (a single solve) reads no list.
+struct Work {
+  int t, idx, lb;
+};
+__device__ __forceinline__ Work work_item(const LaunchList& ll) {
+  int n = ll.nitems, nb = ll.nblocks, i0 = ll.items[0];
+  pin_s(n, nb, i0);
+  const int b = xcd_swizzle(blockIdx.x, nb);
+  if (n == 1) return {0, i0, b};
+  const int t = find_item(ll.prefix, n, b);
+  return {t, ll.items[t], b - ll.prefix[t]};
 }
 
 // A gated cycle has stopped (DevLevel::stop): the kernel returns at once.
@@ -67,6 +102,11 @@ __device__ __forceinline__ int xcd_swizzle(int b, int n) {
 // correctly rounded division in FP64.
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ double rcp(double x) { return 1.0 / x; }
+
+// Fused multiply-add a*b + c, written out where several kernels have to
+// round alike.
+__device__ __forceinline__ float fm(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fm(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
 // a / d in the point smoother: times the hardware reciprocal in FP32 (an
 // IEEE division is about a dozen instructions), a division in FP64.
@@ -379,6 +419,12 @@ template <class T> __device__ __forceinline__ T ld_row_nt(sp<kG, const T> row, u
   return __builtin_nontemporal_load((const T*)(sp<kG, const T>)((sp<kG, const char>)row + boff));
 }
 
+// The four in-plane neighbours' part of a row's stencil sum.
+template <class T>
+__device__ __forceinline__ T zline_nbr(T wxl, T wxr, T wys, T wyn, T xl, T xr, T ys, T yn) {
+  return fm(wyn, yn, fm(wys, ys, fm(wxr, xr, wxl * xl)));
+}
+
 // NBR false: the other colour is zero (zero_guess bit 0, the first
 // half-sweep from u = 0) and is not read.  LEAN: the register-lean form of
 // the segment elimination (below).  H: a wave holds two segments of 32
@@ -488,10 +534,7 @@ __device__ __forceinline__ void zline_group(const DevLevel& L, int parity, int z
 #pragma unroll
     for (int qq = 0; qq < C; ++qq) {
       if constexpr (NBR) {
-        T sn = wxl * xl[qq] + wxr * xr[qq];
-        sn += wys * ys[qq];
-        sn += wyn * yn[qq];
-        g[q0 + qq] = fv[qq] - sn;
+        g[q0 + qq] = fv[qq] - zline_nbr(wxl, wxr, wys, wyn, xl[qq], xr[qq], ys[qq], yn[qq]);
       } else {
         g[q0 + qq] = fv[qq];
       }
@@ -527,13 +570,13 @@ __device__ __forceinline__ void zline_group(const DevLevel& L, int parity, int z
       if (q < len) {
         if (q == len - 1) g[q] -= lagt;                    // row nz-1 (last segment)
         const T a = (q == 0) ? T(0) : A(q);
-        const T rd = rcp(D(q) - a * cq);
-        y = (g[q] - a * y) * rd;
+        const T rd = rcp(fm(-a, cq, D(q)));
+        y = fm(-a, y, g[q]) * rd;
         v = (q == 0) ? a_first * rd : -(a * rd) * v;
         cq = E(q) * rd;
         g[q] = y;
         if (q == 0) { y0 = y; v0 = v; }
-        else { y0 += pi * y; v0 += pi * v; }
+        else { y0 = fm(pi, y, y0); v0 = fm(pi, v, v0); }
         if (q == len - 1) { yl = y; vl = v; wl = cq; w0 = pi * cq; }
         else pi = (q == 0) ? -cq : pi * -cq;
         if constexpr (LEAN) {
@@ -579,18 +622,18 @@ __device__ __forceinline__ void zline_group(const DevLevel& L, int parity, int z
       const T ab_m = hm ? abm : T(0), cb_m = hm ? cbm : T(0), rb_m = hm ? rbm : T(0);
       const T at_p = hp ? atp : T(0), ct_p = hp ? ctp : T(0), rt_p = hp ? rtp : T(0);
       if (kZBuf == 1) __syncthreads();   // every read done before the next writes
-      const T m11 = T(1) - at * cb_m, m12 = -ct * at_p;
-      const T m21 = -ab * cb_m, m22 = T(1) - cb * at_p;
-      const T id = rcp(m11 * m22 - m12 * m21);
-      const T qt = rt - at * rb_m - ct * rt_p, qb = rb - ab * rb_m - cb * rt_p;
+      const T m11 = fm(-at, cb_m, T(1)), m12 = -ct * at_p;
+      const T m21 = -ab * cb_m, m22 = fm(-cb, at_p, T(1));
+      const T id = rcp(fm(m11, m22, -(m12 * m21)));
+      const T qt = fm(-ct, rt_p, fm(-at, rb_m, rt)), qb = fm(-cb, rt_p, fm(-ab, rb_m, rb));
       const T lt = -at * ab_m, lb = -ab * ab_m;     // couplings to b_{p-2d}
       const T ut = -ct * ct_p, ub = -cb * ct_p;     // couplings to t_{p+2d}
-      at = id * (m22 * lt - m12 * lb);
-      ab = id * (m11 * lb - m21 * lt);
-      ct = id * (m22 * ut - m12 * ub);
-      cb = id * (m11 * ub - m21 * ut);
-      rt = id * (m22 * qt - m12 * qb);
-      rb = id * (m11 * qb - m21 * qt);
+      at = id * fm(m22, lt, -(m12 * lb));
+      ab = id * fm(m11, lb, -(m21 * lt));
+      ct = id * fm(m22, ut, -(m12 * ub));
+      cb = id * fm(m11, ub, -(m21 * ut));
+      rt = id * fm(m22, qt, -(m12 * qb));
+      rb = id * fm(m11, qb, -(m21 * qt));
     }
     T* W = lds + buf * 6 * PS;
     W[sl] = rt;
@@ -610,7 +653,7 @@ __device__ __forceinline__ void zline_group(const DevLevel& L, int parity, int z
         for (int q = 0; q < S; ++q) {
           if (q < len) {
             v = (q == 0) ? a_first * rdv[q] : -(A(q) * rdv[q]) * v;
-            g[q] -= v * bprev;
+            g[q] = fm(-v, bprev, g[q]);
           }
         }
       }
@@ -621,10 +664,10 @@ __device__ __forceinline__ void zline_group(const DevLevel& L, int parity, int z
       if (q < len) {
         if constexpr (LEAN) {
           const T cq = E(q) * rdv[q];
-          x = (q == len - 1) ? g[q] - cq * tnext : g[q] - cq * x;
+          x = fm(-cq, (q == len - 1) ? tnext : x, g[q]);
         } else {
-          const T gq = g[q] - vv[q] * bprev;
-          x = (q == len - 1) ? gq - cp[q] * tnext : gq - cp[q] * x;
+          const T gq = fm(-vv[q], bprev, g[q]);
+          x = fm(-cp[q], (q == len - 1) ? tnext : x, gq);
         }
         if (live) st_row<T>(u + (ks + q) * plane, bown, x);
       }
@@ -664,6 +707,299 @@ __global__ __launch_bounds__(H ? 512 : 1024, H ? 2 : ((LEAN && sizeof(T) == 4) ?
     zline_group<T, S, C, NBR, LEAN, false>(L, parity, zero_flags(L, zero_guess),
                                            (b - ll.prefix[t]) * 64 + threadIdx.x, seg, threadIdx.x,
                                            blockDim.y, reinterpret_cast<T*>(lds_raw), true);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The FP32 half-sweep of a level whose columns all have the same x/y diagonal
+// share (both horizontal axes uniform, no wall in them): every column then
+// has the same matrix, so the pivots, the segments' coupling solutions and
+// the whole cyclic reduction of the interface matrix are the same numbers in
+// every column.  They are computed once, when the level is built
+// (k_zline_table), with the operations of zline_group, and the sweep keeps
+// only the right-hand side's own arithmetic: the results are those of
+// zline_group bit for bit.
+//
+// Table (DevLevel::zt): one record of kZRec words per segment,
+//   [0, 32)    A | RD, kZSeg words each: the sub-diagonal within the segment
+//              (0 in its first row) and the pivot's reciprocal
+//   [64, 112)  V | CQ | PI: the coupling solution v, the eliminated
+//              super-diagonal and the weight of the row's y in the segment's
+//              first value
+//   [128, 164) kZStep words per reduction step: at ab ct cb m11 m12 m21 m22 id.
+// Rows past nz are zero: they leave the carried values zero; so is the record
+// past an odd count of segments (the half-wave form's spare segment).
+constexpr int kZRec = 192, kZRecBack = 64, kZRecStep = 128, kZStep = 9;
+
+// One thread per segment.
+__global__ __launch_bounds__(64) void k_zline_table(const float* __restrict__ co, int nx, int ny, int nz,
+                                                    float* __restrict__ zt) {
+  __shared__ float st[4][64];
+  constexpr int S = kZSeg;
+  const int P = (nz + S - 1) / S, p = threadIdx.x;
+  const bool on = p < P;
+  for (int e = p; e < kZRec * ((P + 1) & ~1); e += 64) zt[e] = 0.0f;
+  __syncthreads();
+  const float* cz = co + 3 * nx + 3 * ny;
+  const float dxy = co[2 * nx] + co[3 * nx + 2 * ny];
+  const int ks = p * S, len = on ? min(S, nz - ks) : 0;
+  float* z = zt + p * kZRec;
+  float v0 = 0.0f, vl = 0.0f, w0 = 0.0f, wl = 0.0f;
+  float cq = 0.0f, v = 0.0f, pi = 1.0f;
+  if (on) {
+    const float a_first = cz[ks];
+    for (int q = 0; q < S; ++q) {
+      float a = 0.0f, rd = 0.0f, pw = 0.0f, vq = 0.0f, cw = 0.0f;
+      if (q < len) {
+        const int k = ks + q;
+        a = (q == 0) ? 0.0f : cz[k];
+        rd = rcp(fm(-a, cq, cz[2 * nz + k] + dxy));
+        v = (q == 0) ? a_first * rd : -(a * rd) * v;
+        cq = cz[nz + k] * rd;
+        if (q == 0) v0 = v;
+        else v0 = fm(pi, v, v0);
+        pw = pi;
+        vq = v;
+        cw = cq;
+        if (q == len - 1) { vl = v; wl = cq; w0 = pi * cq; }
+        else pi = (q == 0) ? -cq : pi * -cq;
+      }
+      z[q] = a;
+      z[S + q] = rd;
+      z[kZRecBack + q] = vq;
+      z[kZRecBack + S + q] = cw;
+      z[kZRecBack + 2 * S + q] = pw;
+    }
+  }
+  float at = v0, ab = vl, ct = w0, cb = wl;
+  z += kZRecStep;
+  for (int d = 1; d < P; d <<= 1, z += kZStep) {
+    st[0][p] = at; st[1][p] = ab; st[2][p] = ct; st[3][p] = cb;
+    __syncthreads();
+    const bool hm = on && p - d >= 0, hp = p + d < P;
+    const float ab_m = hm ? st[1][p - d] : 0.0f, cb_m = hm ? st[3][p - d] : 0.0f;
+    const float at_p = hp ? st[0][p + d] : 0.0f, ct_p = hp ? st[2][p + d] : 0.0f;
+    __syncthreads();
+    const float m11 = fm(-at, cb_m, 1.0f), m12 = -ct * at_p;
+    const float m21 = -ab * cb_m, m22 = fm(-cb, at_p, 1.0f);
+    const float id = rcp(fm(m11, m22, -(m12 * m21)));
+    if (on) {
+      z[0] = at; z[1] = ab; z[2] = ct; z[3] = cb;
+      z[4] = m11; z[5] = m12; z[6] = m21; z[7] = m22;
+      z[8] = id;
+    }
+    const float lt = -at * ab_m, lb = -ab * ab_m;
+    const float ut = -ct * ct_p, ub = -cb * ct_p;
+    at = id * fm(m22, lt, -(m12 * lb));
+    ab = id * fm(m11, lb, -(m21 * lt));
+    ct = id * fm(m22, ut, -(m12 * ub));
+    cb = id * fm(m11, ub, -(m21 * ut));
+  }
+}
+
+// A field as a raw buffer: a row's 32-bit byte offset is a scalar, a lane's
+// the vector offset, and an access past the field's end reads zero or is
+// dropped (a spare lane's offset is kNoLane).
+typedef __amdgpu_buffer_rsrc_t Buf;
+constexpr unsigned kNoLane = 0x80000000u;
+__device__ __forceinline__ Buf field_buf(const void* p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
+}
+__device__ __forceinline__ float buf_ld(Buf b, unsigned lane, unsigned row) {
+  return __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(b, (int)lane, (int)row, 0));
+}
+__device__ __forceinline__ void buf_st(Buf b, unsigned lane, unsigned row, float v) {
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), b, (int)lane, (int)row, 0);
+}
+
+// H false: 64 columns per workgroup, one segment per wave, whose table the
+// wave holds without a vector load per row: A and RD in scalar registers
+// (32 words; 48 spilled), the others one word per lane of two vector registers,
+// read back with readlane.  H true (launches of few column groups, to spread
+// over twice the CUs): 32 columns and two segments per wave; each wave stages
+// its two records in LDS and reads them back per half while the data is on
+// its way.  Either way the whole table is loaded with the data, before the
+// first barrier: read where it is used, each part would be a cold dependent
+// load (the sweep then took 3-10 % longer than zline_group).
+//
+// What it gives (FP32 half-sweep, zline_group -> this): 64x48x32 4.1 -> 3.1,
+// 160x112x80 6.2 -> 5.7, 128^3 5.8 -> 5.1, from zero at 256^3 15.7 -> 13.3 us.
+// The finest 256^3 sweep keeps its 20 us (100.7 MB): it is bound by the
+// memory phase and by the start of its 8192 waves, not by arithmetic.
+template <bool H>
+__global__ __launch_bounds__(H ? 512 : 1024, H ? 2 : 8) void k_zline_shared(
+    const DevLevel* __restrict__ Lt, int parity, int zero_guess, LaunchList ll) {
+  extern __shared__ float zlds[];
+  constexpr int S = kZSeg, CW = H ? 32 : 64;
+  const Work wk = work_item(ll);
+  const DevLevel& L = Lt[wk.idx];
+  int nx = L.nx, ny = L.ny, nz = L.nz, hx = L.hx, stop = L.stop, warm = L.warm, pz = L.pz;
+  unsigned gmhx = L.gmhx;
+  int gshx = L.gshx, ncell = L.ncell;
+  const void *up = L.u, *fp = L.f;
+  const float *cp = L.co32, *zp = L.zt;
+  pin_s(nx, ny, nz, hx, stop, warm, pz, gmhx, gshx, ncell, up, fp, cp, zp);
+  if (stop) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y), tx = threadIdx.x;
+  const int half = H ? tx >> 5 : 0, lane = tx & (CW - 1);
+  const int P = (nz + S - 1) / S, PA = H ? (P + 1) & ~1 : P;
+  const int p = H ? 2 * wave + half : wave;
+  const sp<kG, const float> zr = gp(zp) + (H ? 2 * wave : wave) * kZRec;
+  float* const zl = zlds + 4 * PA * CW + 2 * wave * kZRec;   // H: the wave's two records
+  float ra[S], rd[S], tback = 0.0f, tstep = 0.0f, tr[6];
+  if constexpr (H) {
+#pragma unroll
+    for (int q = 0; q < 6; ++q) tr[q] = zr[q * 64 + tx];
+  } else {
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+      ra[q] = zr[q];
+      rd[q] = zr[S + q];
+    }
+    tback = zr[kZRecBack + tx];
+    tstep = zr[kZRecStep + tx];
+  }
+  auto word = [](float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+  // word q of the segment's record, backward and step parts
+  auto rec = [&](int q) { return zl[half * kZRec + q]; };
+  auto back = [&](int q) { return H ? rec(kZRecBack + q) : word(tback, q); };
+  auto stepw = [&](int q) { return H ? rec(kZRecStep + q) : word(tstep, q); };
+  const int col0 = wk.lb * CW + lane, ncol = hx * ny;
+  const int col = min(col0, ncol - 1);
+  const int j = gm_div(col, gmhx, gshx), m = col - j * hx;
+  const int c = parity, oth = parity ^ 1;
+  const int r = (c + j) & 1, i = 2 * m + r;
+  int ml = m - 1 + r; if (ml < 0) ml = hx - 1;
+  int mr = m + r;     if (mr >= hx) mr = 0;
+  const int jm = (j == 0) ? ny - 1 : j - 1, jp = (j == ny - 1) ? 0 : j + 1;
+  const sp<kG, const float> co = gp(cp);
+  const sp<kG, const float> cy = co + 3 * nx;
+  const sp<kG, const float> cz = cy + 3 * ny;
+  const float wxl = co[i], wxr = co[nx + i], wys = cy[j], wyn = cy[ny + j];
+  constexpr unsigned W = sizeof(float);
+  const Buf u = field_buf(up, (unsigned)ncell * W), f = field_buf(fp, (unsigned)ncell * W);
+  const unsigned plane = (unsigned)(ny * 2 * hx) * W;
+  const int ks = p * S, len = max(0, min(S, nz - ks));
+  const unsigned bown = (unsigned)cidx(m, j, 0, c, hx, ny) * W;
+  const unsigned xo = (unsigned)cidx(0, j, 0, oth, hx, ny);
+  const unsigned bxl = (xo + ml) * W, bxr = (xo + mr) * W;
+  const unsigned bso = (unsigned)cidx(m, jm, 0, oth, hx, ny) * W;
+  const unsigned bno = (unsigned)cidx(m, jp, 0, oth, hx, ny) * W;
+  // the sweep from zero reads b alone; a mixed cycle's first sweep is one
+  // unless the cycle continues the previous one's iterate (kZgDyn)
+  const int zg = (zero_guess & kZgDyn) && warm ? 0 : zero_guess & 3;
+  // periodic z: the lagged wrap values, as in zline_group
+  const bool lag = pz != 0 && !(zg & 2);
+  float lagb = 0.0f, lagt = 0.0f;
+  if (lag) {
+    const float ubot = buf_ld(u, bown, (unsigned)(nz - 1) * plane), utop = buf_ld(u, bown, 0);
+    lagb = p == 0 ? cz[0] * ubot : 0.0f;
+    lagt = p == P - 1 ? cz[2 * nz - 1] * utop : 0.0f;
+  }
+  float g[S];
+  // rows at vector offset vrow(q) and scalar offset srow(q)
+  auto load = [&](auto vrow, auto srow) {
+#pragma unroll
+    for (int q = 0; q < S; ++q) g[q] = buf_ld(f, bown + vrow(q), srow(q));
+    if (!(zg & 1)) {
+      float xl[S], xr[S], ys[S], yn[S];
+#pragma unroll
+      for (int q = 0; q < S; ++q) {
+        const unsigned v = vrow(q), o = srow(q);
+        xl[q] = buf_ld(u, bxl + v, o);
+        xr[q] = buf_ld(u, bxr + v, o);
+        ys[q] = buf_ld(u, bso + v, o);
+        yn[q] = buf_ld(u, bno + v, o);
+      }
+#pragma unroll
+      for (int q = 0; q < S; ++q) g[q] -= zline_nbr(wxl, wxr, wys, wyn, xl[q], xr[q], ys[q], yn[q]);
+    }
+  };
+  if constexpr (H) {
+#pragma unroll
+    for (int q = 0; q < 6; ++q) zl[q * 64 + tx] = tr[q];
+  }
+  // rows past nz are clamped to the last one: in bounds
+  if constexpr (!H) {
+    load([](int) { return 0u; }, [&](int q) { return (unsigned)min(ks + q, nz - 1) * plane; });
+  } else if (nz == PA * S) {
+    const unsigned v0 = (unsigned)ks * plane;
+    load([=](int) { return v0; }, [=](int q) { return (unsigned)q * plane; });
+  } else {
+    load([=](int q) { return (unsigned)min(ks + q, nz - 1) * plane; }, [](int) { return 0u; });
+  }
+  if constexpr (H) {
+    // the wave's own records: written and read by its lanes alone
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+      ra[q] = rec(q);
+      rd[q] = rec(S + q);
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < S; ++q) pin_s(ra[q], rd[q]);
+  }
+  if (lag) {
+    g[0] -= lagb;
+#pragma unroll
+    for (int q = 0; q < S; ++q)
+      if (q == len - 1) g[q] -= lagt;
+  }
+  float y = 0.0f, y0 = 0.0f;
+#pragma unroll
+  for (int q = 0; q < S; ++q) {
+    y = fm(-ra[q], y, g[q]) * rd[q];
+    g[q] = y;
+    y0 = (q == 0) ? y : fm(back(2 * S + q), y, y0);
+  }
+  // the interface values, reduced as in zline_group: only the right-hand
+  // sides are exchanged, the couplings are the table's
+  float bprev = 0.0f, tnext = 0.0f;
+  if (P > 1) {
+    const int PS = PA * CW, sl = p * CW + lane;
+    float rt = y0, rb = y;
+    int buf = 0;
+    for (int d = 1, w = 0; d < P; d <<= 1, buf ^= 1, w += kZStep) {
+      const float at = stepw(w), ab = stepw(w + 1), ct = stepw(w + 2), cb = stepw(w + 3);
+      const float m11 = stepw(w + 4), m12 = stepw(w + 5), m21 = stepw(w + 6), m22 = stepw(w + 7);
+      const float id = stepw(w + 8);
+      float* B = zlds + buf * 2 * PS;
+      B[sl] = rt;
+      B[PS + sl] = rb;
+      __syncthreads();
+      const bool hm = p - d >= 0, hp = p + d < P;
+      const float rbm = B[PS + (hm ? sl - d * CW : sl)], rtp = B[hp ? sl + d * CW : sl];
+      const float rb_m = hm ? rbm : 0.0f, rt_p = hp ? rtp : 0.0f;
+      const float qt = fm(-ct, rt_p, fm(-at, rb_m, rt)), qb = fm(-cb, rt_p, fm(-ab, rb_m, rb));
+      rt = id * fm(m22, qt, -(m12 * qb));
+      rb = id * fm(m11, qb, -(m21 * qt));
+    }
+    float* B = zlds + buf * 2 * PS;
+    B[sl] = rt;
+    B[PS + sl] = rb;
+    __syncthreads();
+    const bool hm = p > 0, hp = p < P - 1;
+    const float rbm = B[PS + (hm ? sl - CW : sl)], rtp = B[hp ? sl + CW : sl];
+    bprev = hm ? rbm : 0.0f;
+    tnext = hp ? rtp : 0.0f;
+  }
+  float x = tnext;
+#pragma unroll
+  for (int q = S - 1; q >= 0; --q) {
+    x = fm(-back(S + q), x, fm(-back(q), bprev, g[q]));
+    g[q] = x;
+  }
+  const unsigned bst = col0 < ncol ? bown + (H ? (unsigned)ks * plane : 0u) : kNoLane;
+  const unsigned srow0 = H ? 0u : (unsigned)ks * plane;
+  if (nz == PA * S) {
+#pragma unroll
+    for (int q = S - 1; q >= 0; --q) buf_st(u, bst, srow0 + (unsigned)q * plane, g[q]);
+  } else {
+#pragma unroll
+    for (int q = S - 1; q >= 0; --q)
+      if (q < len) buf_st(u, bst, srow0 + (unsigned)q * plane, g[q]);
   }
 }
 
@@ -2614,6 +2950,34 @@ void launch_zline(bool fp64, const DevLevel* L, const LaunchList& ll, int parity
     return;
   }
   zline_variant(fp64, L, l2, parity, zero_guess, segs, s, form, !(zero_guess & 1), half);
+}
+size_t zline_table_bytes(int nz) { return sizeof(float) * kZRec * (((nz + kZSeg - 1) / kZSeg + 1) & ~1); }
+void launch_zline_table(const float* co32, int nx, int ny, int nz, float* zt, hipStream_t s) {
+  LAUNCH(k_zline_table, 1, 64, co32, nx, ny, nz, zt);
+}
+void launch_zline_shared(const DevLevel* L, const LaunchList& ll, int parity, int zero_guess, int segs,
+                         hipStream_t s) {
+  // More column groups than CUs, and the other colour is read: two groups
+  // share a CU, whose arithmetic hides behind the other's loads anyway, and
+  // the general sweep's smaller start is the faster (256^3: 19.5 against
+  // 20.3 us; 512x256x256: 36.0 against 37.5 us).
+  if (ll.nblocks > device_cus() && !(zero_guess & 1)) {
+    launch_zline(false, L, ll, parity, zero_guess, segs, s);
+    return;
+  }
+  if (segs >= 2 && 2 * ll.nblocks <= device_cus()) {
+    LaunchList hl = ll;
+    for (int t = 0; t <= ll.nitems; ++t) hl.prefix[t] = 2 * ll.prefix[t];
+    hl.nblocks = 2 * ll.nblocks;
+    const int wy = (segs + 1) / 2;
+    const size_t lds = (size_t)2 * wy * (4 * 32 + kZRec) * sizeof(float);
+    hipLaunchKernelGGL(k_zline_shared<true>, dim3(hl.nblocks), dim3(64, wy), lds, s, L, parity,
+                       zero_guess, hl);
+    return;
+  }
+  const size_t lds = (size_t)4 * segs * 64 * sizeof(float);
+  hipLaunchKernelGGL(k_zline_shared<false>, dim3(ll.nblocks), dim3(64, segs), lds, s, L, parity,
+                     zero_guess, ll);
 }
 void launch_zline_col(bool fp64, const DevLevel* L, const LaunchList& ll, int parity,
                       int zero_guess, hipStream_t s) {

@@ -333,6 +333,21 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
     AMG_HIP(hipMemcpy(vol, H.vol.data(), H.vol.size() * 8, hipMemcpyHostToDevice));
     AMG_HIP(hipMemcpy(rho, H.rho.data() + 1, H.nz * 8, hipMemcpyHostToDevice));
     d.co64 = c64; d.co32 = c32; d.vol = vol; d.rho = rho;
+    // FP32 z-line sweeps: one table for all columns where they share their
+    // matrix, i.e. the x and y diagonal shares are single values
+    // (fields of at most 2 GiB: the sweep's byte offsets are 32-bit)
+    if (!I->fp64 && cfg.smoother == AMG_SMOOTHER_LJ && H.ncell() <= (1ll << 29)) {
+      const float* dx = co32.data() + 2 * H.nx;
+      const float* dy = co32.data() + 3 * H.nx + 2 * H.ny;
+      if (std::all_of(dx, dx + H.nx, [&](float v) { return v == dx[0]; }) &&
+          std::all_of(dy, dy + H.ny, [&](float v) { return v == dy[0]; })) {
+        float* zt = (float*)I->mem.alloc(zline_table_bytes(H.nz));
+        if (!zt) return fail();
+        launch_zline_table(c32, H.nx, H.ny, H.nz, zt, stream);
+        AMG_HIP(hipGetLastError());
+        d.zt = zt;
+      }
+    }
     if (l == 0) {
       double* bf = (double*)I->mem.alloc(H.bcfold.size() * 8);
       if (!bf) return fail();
@@ -626,20 +641,27 @@ int Context::upload_tables() {
   return AMG_OK;
 }
 
-// z-line launches: items grouped by their segment count (blockDim.y).
+// z-line launches: items grouped by their segment count (blockDim.y) and by
+// whether their columns share one matrix (DevLevel::zt; a forced form is
+// always the general sweep).
 void Context::zline_launches(const std::vector<Item>& items, bool fp64, int parity, int zg,
                              int form) {
-  std::vector<Item> bucket[kZMaxSegs + 1];
+  std::vector<Item> bucket[2][kZMaxSegs + 1];
   for (const Item& it : items) {
-    const int nz = hL[it.idx].nz;
-    const int segs = std::min(kZMaxSegs, (nz + kZSeg - 1) / kZSeg);
-    bucket[segs].push_back(it);
+    const DevLevel& d = hL[it.idx];
+    const int segs = std::min(kZMaxSegs, (d.nz + kZSeg - 1) / kZSeg);
+    bucket[!fp64 && form == 0 && d.zt ? 1 : 0][segs].push_back(it);
   }
-  for (int sg = 1; sg <= kZMaxSegs; ++sg)
-    if (!bucket[sg].empty())
-      for_lists(bucket[sg], [&](const LaunchList& ll, int, int) {
+  for (int sg = 1; sg <= kZMaxSegs; ++sg) {
+    if (!bucket[0][sg].empty())
+      for_lists(bucket[0][sg], [&](const LaunchList& ll, int, int) {
         launch_zline(fp64, dL, ll, parity, zg, sg, stream, form);
       });
+    if (!bucket[1][sg].empty())
+      for_lists(bucket[1][sg], [&](const LaunchList& ll, int, int) {
+        launch_zline_shared(dL, ll, parity, zg, sg, stream);
+      });
+  }
 }
 
 // Point half-sweeps of the items' levels: the levels large enough march in z
