@@ -123,26 +123,26 @@ void amg::metric_ptrs(const Instance* I, const double** rho, const double** rdxc
   *rdze = m;
 }
 
-// The divergence report into `partial` (divergence_blocks * 4 values, then
-// the 4 results); copies the results to the host and fills the outputs.
+// The divergence report with its block partials in `partial`
+// (divergence_blocks * kDivVals values).  The fold writes the results to the
+// handle's pinned host buffer, so they are there when the stream is done.
 int amg::divergence_report(amg_handle h, const double* U, const double* V, const double* W,
                              double* div, double* partial, double* avg, double* maxabs,
                              int loc[3]) {
   const double *rho, *rdxc, *rdyc, *rdzc, *rdxe, *rdye, *rdze;
   metric_ptrs(h->I, &rho, &rdxc, &rdyc, &rdzc, &rdxe, &rdye, &rdze);
   const int nx = h->I->nx, ny = h->I->ny, nz = h->I->nz;
-  const int nb = divergence_blocks(nx, ny, nz);
+  const double *dxc = rdze + nz + 2, *dyc = dxc + nx + 2, *dzc = dyc + ny + 2;
   hipStream_t s = h->ctx.stream;
-  launch_divergence(U, V, W, div, rdxc, rdyc, rdzc, nx, ny, nz, partial, s);
-  launch_divergence_finalize(partial, nb, partial + 4 * (size_t)nb, s);
+  double* o = h->ctx.h_out;
+  launch_divergence(U, V, W, div, rdxc, rdyc, rdzc, dxc, dyc, dzc, nx, ny, nz, partial, s);
+  launch_divergence_finalize(partial, divergence_blocks(nx, ny, nz), o, s);
   AMG_HIP(hipGetLastError());
-  double o[4];
-  AMG_HIP(hipMemcpyAsync(o, partial + 4 * (size_t)nb, sizeof o, hipMemcpyDeviceToHost, s));
   AMG_HIP(hipStreamSynchronize(s));
-  if (avg) *avg = o[0] / o[1];
-  if (maxabs) *maxabs = o[2];
+  if (avg) *avg = o[0] / h->I->H.vol_sum;
+  if (maxabs) *maxabs = o[1];
   if (loc) {
-    const long long e = (long long)o[3];
+    const long long e = (long long)o[2];
     loc[0] = (int)(e % nx) + 2;
     loc[1] = (int)((e / nx) % ny) + 2;
     loc[2] = (int)(e / ((long long)nx * ny)) + 2;
@@ -477,7 +477,7 @@ int amg_divergence_device(amg_handle h, const double* U, const double* V, const 
   if (!h || !U || !V || !W) return fail(AMG_EINVAL, "amg_divergence_device: NULL argument");
   const int nb = divergence_blocks(h->I->nx, h->I->ny, h->I->nz);
   if (!h->d_div_partial)
-    AMG_HIP(hipMalloc((void**)&h->d_div_partial, sizeof(double) * (4 * (size_t)nb + 4)));
+    AMG_HIP(hipMalloc((void**)&h->d_div_partial, sizeof(double) * kDivVals * (size_t)nb));
   return divergence_report(h, U, V, W, div, h->d_div_partial, avg, maxabs, loc);
 }
 

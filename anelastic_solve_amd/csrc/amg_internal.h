@@ -433,13 +433,18 @@ void launch_psource(const double* U, const double* V, const double* W, double* S
 void launch_pgrad(const double* p, double* U, double* V, double* W, const double* rho,
                   const double* rdxe, const double* rdye, const double* rdze, int nx, int ny,
                   int nz, double dt, int wallmask, hipStream_t s);
-// kDivPer cells per thread: blocks = cdiv(cells, kBlock*kDivPer), each
-// writes 4 partials; the finalize writes 4 values.
-constexpr int kDivPer = 16;
+// Planes of a thread of the source and divergence kernels.
+constexpr int kProjK = 8;
+// The divergence report: at most kDivBlocks blocks, each writes kDivVals
+// partials {sum |div| V, max |div|, its cell index}; the finalize folds them
+// into the three results at out.
+constexpr int kDivBlocks = 8192;
+constexpr int kDivVals = 3;
 int divergence_blocks(int nx, int ny, int nz);
 void launch_divergence(const double* U, const double* V, const double* W, double* div,
-                       const double* rdxc, const double* rdyc, const double* rdzc, int nx,
-                       int ny, int nz, double* partial, hipStream_t s);
+                       const double* rdxc, const double* rdyc, const double* rdzc, const double* dxc,
+                       const double* dyc, const double* dzc, int nx, int ny, int nz, double* partial,
+                       hipStream_t s);
 void launch_divergence_finalize(const double* partial, int nblocks, double* out, hipStream_t s);
 
 }  // namespace amg

@@ -2,8 +2,8 @@
 //
 // amg_divergence_device (dns/Routines.F90:54-183) allocates its block
 // partials with hipMalloc on its first call.  amg_divergence_device_noalloc
-// runs the same kernels with the partials and the results in `scratch`, a
-// file-scope device array of kNoAllocDoubles doubles (256 KiB), so that it
+// runs the same kernels with the partials in `scratch`, a file-scope device
+// array of kNoAllocDoubles doubles (192 KiB), so that it
 // can be called under graph capture, from serving loops or where the
 // harness forbids allocation.  Each GPU the library runs on holds its own
 // copy of the array until the process ends.  On the host the array's name
@@ -14,8 +14,7 @@
 // Every call on one GPU shares that GPU's array and leaves the last call's
 // contents in it; calls that overlap on one GPU (two streams, two threads)
 // race.  Nothing in the array needs to start at zero: every block writes
-// its four partials and the fold writes the four results before they are
-// read.
+// its partials before the fold reads them.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -27,8 +26,8 @@
 #include "amg_solver.h"
 
 namespace {
-constexpr int kNoAllocMaxBlocks = 8192;   // grids of at most 33 554 432 cells
-constexpr size_t kNoAllocDoubles = 4 * (size_t)kNoAllocMaxBlocks + 4;
+constexpr long long kNoAllocMaxCells = 33554432;
+constexpr size_t kNoAllocDoubles = (size_t)amg::kDivVals * amg::kDivBlocks;
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
 double* g_ptr[kMaxDevices] = {};
@@ -74,11 +73,10 @@ extern "C" int amg_divergence_device_noalloc(amg_handle h, const double* U, cons
     amg::set_error("amg_divergence_device_noalloc: NULL argument");
     return AMG_EINVAL;
   }
-  const int nb = amg::divergence_blocks(h->I->nx, h->I->ny, h->I->nz);
-  if (nb > kNoAllocMaxBlocks) {
+  if ((long long)h->I->nx * h->I->ny * h->I->nz > kNoAllocMaxCells) {
     amg::set_error("amg_divergence_device_noalloc: the grid has more than " +
-                   std::to_string((long long)kNoAllocMaxBlocks * amg::kBlock * amg::kDivPer) +
-                   " cells, the limit of its static scratch; use amg_divergence_device");
+                   std::to_string(kNoAllocMaxCells) +
+                   " cells, its limit; use amg_divergence_device");
     return AMG_EBADSIZE;
   }
   double* ptr = scratch_on(h->ctx.device);

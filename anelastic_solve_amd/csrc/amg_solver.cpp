@@ -568,7 +568,6 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
   // projection metrics
   {
     const HostLevel& F = I->H.lv[0];
-    const int nx = F.nx, ny = F.ny, nz = F.nz;
     std::vector<double> m;
     m.insert(m.end(), F.rho.begin(), F.rho.end());
     auto inv = [&](const std::vector<double>& a) {
@@ -576,7 +575,7 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
     };
     inv(F.ax.dxc); inv(F.ay.dxc); inv(F.az.dxc);
     inv(F.ax.dxe); inv(F.ay.dxe); inv(F.az.dxe);
-    (void)nx; (void)ny; (void)nz;
+    for (const Axis* a : {&F.ax, &F.ay, &F.az}) m.insert(m.end(), a->dxc.begin(), a->dxc.end());
     I->d_met = (double*)I->mem.alloc(m.size() * 8);
     if (!I->d_met) return fail();
     AMG_HIP(hipMemcpy(I->d_met, m.data(), m.size() * 8, hipMemcpyHostToDevice));

@@ -66,7 +66,7 @@ struct Instance {
   int cur = 0;                   // which fine entry holds the current pressure
   std::vector<int> pre, post;
   DevArena mem;
-  // projection metrics (ghost-inclusive): rho, rdxc, rdyc, rdzc, rdxe, rdye, rdze
+  // projection metrics (ghost-inclusive): rho, rdxc, rdyc, rdzc, rdxe, rdye, rdze, dxc, dyc, dzc
   double* d_met = nullptr;
   // per-solve state
   bool converged = false, done = false;

@@ -199,7 +199,7 @@ int amg_divergence_device(amg_handle h, const double* U, const double* V, const 
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  Same arguments,
  * kernels and results as amg_divergence_device, which allocates its block
- * partials on its first call; this one keeps them in a static 256 KiB
+ * partials on its first call; this one keeps them in a static 192 KiB
  * device array per GPU instead and allocates nothing.  Limit: grids of at
  * most 33 554 432 cells (AMG_EBADSIZE beyond).  Calls that overlap on one
  * GPU share that array and race. */
