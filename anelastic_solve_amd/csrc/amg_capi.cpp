@@ -408,7 +408,7 @@ int amg_ghost_device(amg_handle h, double* var, const char* vtype, const amg_flo
   GhostPlan P;
   std::string err;
   if (plan_ghost(G, vtype, *bc, &P, &err) != 0) return fail(AMG_EINVAL, "amg_ghost_device: " + err);
-  launch_flow_ghost(var, G.nx, G.ny, G.nz, P, h->ctx.stream);
+  launch_flow_ghost(&var, &P, 1, G.nx, G.ny, G.nz, h->ctx.stream);
   AMG_HIP(hipGetLastError());
   AMG_HIP(hipStreamSynchronize(h->ctx.stream));
   return AMG_OK;
@@ -432,7 +432,7 @@ int amg_pgrad_ghost_device(amg_handle h, const double* p, double* U, double* V, 
   hipStream_t s = h->ctx.stream;
   launch_pgrad(p, U, V, W, rho, rdxe, rdye, rdze, G.nx, G.ny, G.nz, dt, wallmask, s);
   double* f[3] = {U, V, W};
-  for (int c = 0; c < 3; ++c) launch_flow_ghost(f[c], G.nx, G.ny, G.nz, P[c], s);
+  launch_flow_ghost(f, P, 3, G.nx, G.ny, G.nz, s);
   AMG_HIP(hipGetLastError());
   AMG_HIP(hipStreamSynchronize(s));
   return AMG_OK;
@@ -466,7 +466,7 @@ int amg_cn_advance_device(amg_handle h, const double* veltemp1, double* veltemp2
   metric_ptrs(h->I, &rho, &rdxc, &rdyc, &rdzc, &rdxe, &rdye, &rdze);
   launch_cn_column(veltemp1, veltemp2, p, h->d_cn, rdxe, rdye, G.nx, G.ny, G.nz, f1, f2, f3, rkdt, var,
                    s);
-  launch_flow_ghost(veltemp2, G.nx, G.ny, G.nz, P, s);
+  launch_flow_ghost(&veltemp2, &P, 1, G.nx, G.ny, G.nz, s);
   AMG_HIP(hipGetLastError());
   AMG_HIP(hipStreamSynchronize(s));
   return AMG_OK;

@@ -32,6 +32,7 @@ struct FaceRule {
 // nrules face rules (0 when the direction has nothing to apply).
 struct GhostPlan {
   int bound;              // bound_update knows the type (else wraps only)
+  int fused;              // the whole sequence is one pass (ghost_fused)
   FaceRule r[3][2];
   int nrules[3];
 };
@@ -50,7 +51,9 @@ struct CnRow {
 
 int plan_ghost(const FlowGrid& G, const char* vtype, const amg_flowbc& bc, GhostPlan* out,
                std::string* err);
-void launch_flow_ghost(double* a, int nx, int ny, int nz, const GhostPlan& P, hipStream_t s);
+// ghost() of nf (1 to 3) fields with a plan each.
+void launch_flow_ghost(double* const* a, const GhostPlan* P, int nf, int nx, int ny, int nz,
+                       hipStream_t s);
 
 int plan_cn(const FlowGrid& G, int var, double rkdt, double rRe, double rPr, double rSc,
             const amg_flowbc& bc, std::vector<CnRow>* rows, std::string* err);
