@@ -455,13 +455,14 @@ int amg_cn_advance_device(amg_handle h, const double* veltemp1, double* veltemp2
   if (plan_ghost(G, ghost_type[var], *bc, &P, &err) != 0)
     return fail(AMG_EINVAL, "amg_cn_advance_device: " + err);
   hipStream_t s = h->ctx.stream;
-  const size_t nb = sizeof(CnRow) * rows.size();
   if (!h->d_cn) {
-    AMG_HIP(hipMalloc((void**)&h->d_cn, nb));
-    AMG_HIP(hipHostMalloc((void**)&h->h_cn, nb, hipHostMallocDefault));
+    const size_t most = sizeof(double) * cn_table_doubles(G.nz);
+    AMG_HIP(hipMalloc((void**)&h->d_cn, most));
+    AMG_HIP(hipHostMalloc((void**)&h->h_cn, most, hipHostMallocDefault));
   }
-  std::memcpy(h->h_cn, rows.data(), nb);
-  AMG_HIP(hipMemcpyAsync(h->d_cn, h->h_cn, nb, hipMemcpyHostToDevice, s));
+  const std::vector<double> table = cn_table(rows, G.nx, G.ny, rkdt);
+  std::memcpy(h->h_cn, table.data(), sizeof(double) * table.size());
+  AMG_HIP(hipMemcpyAsync(h->d_cn, h->h_cn, sizeof(double) * table.size(), hipMemcpyHostToDevice, s));
   const double *rho, *rdxc, *rdyc, *rdzc, *rdxe, *rdye, *rdze;
   metric_ptrs(h->I, &rho, &rdxc, &rdyc, &rdzc, &rdxe, &rdye, &rdze);
   launch_cn_column(veltemp1, veltemp2, p, h->d_cn, rdxe, rdye, G.nx, G.ny, G.nz, f1, f2, f3, rkdt, var,

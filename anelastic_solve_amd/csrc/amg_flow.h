@@ -42,7 +42,6 @@ struct GhostPlan {
 // side (kind 1) or the physics row's viscous factors c1, m1, c2, m2, m3.
 struct CnRow {
   double ap, bp, c;
-  double rbp, cbp;  // 1/bp and -c/bp (the segmented solve's products)
   double cval;
   double c1, m1, c2, m2, m3;
   double pz;        // 1/dze(k): the predicted-pressure metric of w
@@ -57,7 +56,12 @@ void launch_flow_ghost(double* const* a, const GhostPlan* P, int nf, int nx, int
 
 int plan_cn(const FlowGrid& G, int var, double rkdt, double rRe, double rPr, double rSc,
             const amg_flowbc& bc, std::vector<CnRow>* rows, std::string* err);
-void launch_cn_column(const double* v1, double* v2, const double* p, const CnRow* T,
+// The table a launch reads, as doubles: the rows themselves for the serial
+// kernel, or the segmented kernel's (cn_segmented).
+bool cn_segmented(int nx, int ny, int nz);
+std::vector<double> cn_table(const std::vector<CnRow>& rows, int nx, int ny, double rkdt);
+size_t cn_table_doubles(int nz);   // at most
+void launch_cn_column(const double* v1, double* v2, const double* p, const double* T,
                       const double* rdxe, const double* rdye, int nx, int ny, int nz, double f1,
                       double f2, double f3, double rkdt, int var, hipStream_t s);
 

@@ -8,7 +8,7 @@
 // Floating-point contraction is off in this file: every product and sum is
 // rounded as written, in the order of the Fortran source, so the results
 // equal a plain IEEE evaluation of the reference's expressions (the
-// segmented line solve: to rounding).
+// segmented line solve, with explicit multiply-adds: to rounding).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -408,165 +408,150 @@ __global__ __launch_bounds__(kFlowBlock) void k_cn_column(const double* __restri
 
 // The same step with every column split into P segments of S interior rows
 // (at most kCnSeg rows and kCnSeg segments: nz <= 256), one wave per segment
-// and 64 columns per workgroup.  The recurrences' coefficients are
-// the same in every column, so their values are linear in the value carried
-// into a segment:
-//   forward   G_k = G'_k + (prod_{i=r0..k} ap_i) G_{r0-1},        G' from G_{r0-1} = 0,
-//   backward  x_k = x'_k + (prod_{i=k..r1-1} (-c_i/bp_i)) x_{r1},  x' from x_{r1} = 0.
-// Each wave solves its segment locally with the serial kernel's operations
-// (the division by the pivot as a product with its reciprocal, from the
-// table), the segments' end values are chained through LDS (a scan over at
-// most 16 segments), and each row adds its carry term: a few roundings more
-// per row than the serial solve, whose result this equals to rounding.
-// The column is read once and written once (24 B/cell against the serial
-// kernel's 40), and a 256^2 grid has 16 waves per column group instead of
-// one per SIMD.  Rows 0 and nz+1 (the wall rows) are taken by the first and
-// the last wave with the serial kernel's expressions.  Every load comes
-// before the first barrier and every store after the last, so the column is
-// rewritten in place.
+// and 64 columns per workgroup.  The recurrences' coefficients are the same
+// in every column, so their values are linear in the value carried into a
+// segment, with factors that the host's table holds:
+//   forward   G_k = G'_k + PF_k G_{r0-1},  PF_k = prod_{i=r0..k} ap_i,          G' from G_{r0-1} = 0,
+//   backward  x_k = x'_k + QB_k x_{r1},    QB_k = prod_{i=k..r1-1} (-c_i/bp_i), x' from x_{r1} = 0.
+// Each wave solves its segment, the segments' end values are chained through
+// LDS (a scan over at most 16 segments), and each row adds its carry term: the
+// serial kernel's result to rounding (its products of constants are made once,
+// and multiply-adds are fused).  The wall rows 0 and nz+1 are constant rows:
+// their right-hand sides are numbers.  Every load comes before the first
+// barrier and every store after the last, so the column is rewritten in place.
+//
+// It reads and writes each value once (24 B/cell, 32 with the pressure) and
+// is bound by memory as long as two 1024-lane workgroups share a CU, one's
+// loads under the other's chains: hence at most 64 registers, which is why the
+// table's backward part goes through LDS and rows are addressed as a scalar
+// row offset plus one lane offset (raw buffers).  256^3 u with the pressure
+// (549 MB): 135 us; 161 with 86 registers and one workgroup per CU.
 constexpr int kCnSeg = 16;     // rows per wave and waves per column group, at most
-constexpr int kCnChunk = 4;    // rows whose loads are in flight together
+constexpr int kCnFwd = 6;      // table words of a row: e1 e2 ap pz cval kind
+constexpr int kCnBack = 4;     // and of its backward part: PF 1/bp c QB
+struct CnEnds {
+  double g0, c0, rb0;          // row 0: right-hand side, -c/bp of its super-diagonal, 1/bp
+  double gt, at, rbt;          // row nz+1: right-hand side, eliminated sub-diagonal, 1/bp
+};
+typedef int int2v __attribute__((ext_vector_type(2)));
 template <int PV>
-__global__ __launch_bounds__(1024) void k_cn_seg(const double* __restrict__ v1,
-                                                 double* __restrict__ v2,
-                                                 const double* __restrict__ p,
-                                                 const CnRow* __restrict__ T,
-                                                 const double* __restrict__ rdxe,
-                                                 const double* __restrict__ rdye, int nx, int ny,
-                                                 int nz, int S, double f1, double f2, double f3,
-                                                 double rkdt, double h) {
-  __shared__ double gend[kCnSeg][64], xfirst[kCnSeg][64], g0[64], xtop[64];
-  __shared__ double pend[kCnSeg], qfirst[kCnSeg];
+__global__ __launch_bounds__(1024, 8) void k_cn_seg(const double* __restrict__ v1, double* v2,
+                                                    const double* __restrict__ p,
+                                                    const double* __restrict__ T,
+                                                    const double* __restrict__ rdxe,
+                                                    const double* __restrict__ rdye, int nx, int ny,
+                                                    int nz, int S, double f1, double f23, double rkdt) {
+  constexpr int N = kCnSeg;
+  __shared__ double gend[N][64], xfirst[N][64], xtop[64], back[N][N * kCnBack];
   const int lane = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.y), P = blockDim.y;
   const int t = blockIdx.x * 64 + lane;
   const bool live = t < nx * ny;
   const int tc = live ? t : nx * ny - 1;              // a spare lane repeats the last column
-  const int i = 1 + tc % nx, j = 1 + tc / nx;
+  const int jr = tc / nx, i = 1 + tc - jr * nx, j = 1 + jr;
+  const int r0 = 1 + w * S, len = min(S, nz + 1 - r0);
+  // the segment's backward table, one word per lane
+  const double* Bt = T + kCnFwd * (nz + 2) + sizeof(CnEnds) / 8;
+  const double bw = Bt[w * (N * kCnBack) + lane];
+  const CnEnds E = *reinterpret_cast<const CnEnds*>(T + kCnFwd * (nz + 2));
   const size_t st = (size_t)(nx + 2) * (ny + 2);
-  const size_t base = (size_t)j * (nx + 2) + i;
-  const int n = nz + 2;
-  constexpr bool pcv = PV != 0;
-  const size_t poff = PV == 1 ? 1 : (size_t)(nx + 2);
-  auto at = [&](int k) { return base + (size_t)k * st; };
-  auto pnb = [&](int k) -> size_t {
-    return PV == 3 ? at(min(k + 1, n - 1)) : at(k) + poff;
+  const unsigned plane = (unsigned)st * 8u;
+  // raw buffers from the row below the segment to the field's end
+  const size_t off = (size_t)(r0 - 1) * st;
+  const unsigned left = (unsigned)min((size_t)0x7fffffff, ((size_t)(nz + 2) * st - off) * 8);
+  auto buf = [&](const double* a) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(a + off), 0, (int)left, 0x00027000);
   };
-  const double dmc = PV == 1 ? rdxe[i] : (PV == 2 ? rdye[j] : 0.0);
-  // the serial kernel's right-hand side of row k
-  auto rhs = [&](int k, double vm, double vc, double vp, double a1, double pa, double pb) {
-    const CnRow R = T[k];
-    double r = f1 * vc + f2 * a1 * f3;
-    if constexpr (pcv) r = r - rkdt * (pb - pa) * (PV == 3 ? R.pz : dmc);
-    const double tv = R.c1 * (vp - vc) * R.m1 - R.c2 * (vc - vm) * R.m2;
-    r = r + h * tv * R.m3;
-    return R.kind ? R.cval : r;
+  const __amdgpu_buffer_rsrc_t b1 = buf(v1), b2 = buf(v2), bp = buf(PV ? p : v1);
+  auto ld = [](__amdgpu_buffer_rsrc_t b, unsigned l, unsigned row) {
+    return __builtin_bit_cast(double, (int2v)__builtin_amdgcn_raw_buffer_load_b64(b, (int)l, (int)row, 0));
   };
-  const int r0 = 1 + w * S, r1 = min(r0 + S, nz + 1);
-  // the wall rows' inputs, with the segment's (all before the first barrier)
-  double G0 = 0.0, rtop = 0.0;
-  if (w == 0)
-    G0 = rhs(0, 0.0, v2[at(0)], v2[at(1)], v1[at(0)], pcv ? p[at(0)] : 0.0,
-             pcv ? p[pnb(0)] : 0.0);
-  if (w == P - 1)
-    rtop = rhs(n - 1, v2[at(n - 2)], v2[at(n - 1)], v2[at(n - 1)], v1[at(n - 1)],
-               pcv ? p[at(n - 1)] : 0.0, pcv ? p[pnb(n - 1)] : 0.0);
-  // forward, locally: the loads of kCnChunk rows, then their steps
-  double G[kCnSeg];
-  double g = 0.0, pr = 1.0;
+  const unsigned bl = (unsigned)(j * (nx + 2) + i) * 8u;
+  const unsigned bn = bl + (PV == 1 ? 8u : (unsigned)(nx + 2) * 8u);   // the pressure's x or y neighbour
+  const double dm = PV == 1 ? rkdt * rdxe[i] : (PV == 2 ? rkdt * rdye[j] : 0.0);
+  // row q of the segment is q+1 rows past the buffers' start; rows past the
+  // segment repeat its last row's upper neighbour
+  auto row = [&](int q) { return (unsigned)min(q + 1, nz + 2 - r0) * plane; };
+  double G[N];
+  // right-hand sides of rows c0 .. c0+M-1
+  auto rhs = [&](int c0, auto M) {
+    constexpr int m = decltype(M)::value;
+    double v[m + 2], a1[m], pa[m + 1], pb[m];
 #pragma unroll
-  for (int c0 = 0; c0 < kCnSeg; c0 += kCnChunk) {
-    if (c0 < S) {
-      double wv[kCnChunk + 2], a1[kCnChunk], pa[kCnChunk], pb[kCnChunk];
+    for (int q = 0; q < m + 2; ++q) v[q] = ld(b2, bl, q == 0 && c0 == 0 ? 0u : row(c0 + q - 1));
 #pragma unroll
-      for (int q = 0; q < kCnChunk + 2; ++q) wv[q] = v2[at(min(r0 - 1 + c0 + q, n - 1))];
-#pragma unroll
-      for (int q = 0; q < kCnChunk; ++q) {
-        const int k = min(r0 + c0 + q, n - 1);
-        a1[q] = v1[at(k)];
-        pa[q] = pcv ? p[at(k)] : 0.0;
-        pb[q] = pcv ? p[pnb(k)] : 0.0;
-      }
-      // the right-hand sides (independent of the recurrence), then its steps
-      double rr[kCnChunk], apq[kCnChunk];
-#pragma unroll
-      for (int q = 0; q < kCnChunk; ++q) {
-        const int k = min(r0 + c0 + q, n - 1);
-        rr[q] = rhs(k, wv[q], wv[q + 1], wv[q + 2], a1[q], pa[q], pb[q]);
-        apq[q] = T[k].ap;
-      }
-#pragma unroll
-      for (int q = 0; q < kCnChunk; ++q) {
-        if (r0 + c0 + q < r1) {
-          g = rr[q] + apq[q] * g;
-          pr = apq[q] * pr;
-        }
-        G[c0 + q] = g;
-      }
+    for (int q = 0; q < m; ++q) {
+      a1[q] = ld(b1, bl, row(c0 + q));
+      if constexpr (PV != 0) pa[q] = ld(bp, bl, row(c0 + q));
+      if constexpr (PV == 1 || PV == 2) pb[q] = ld(bp, bn, row(c0 + q));
     }
+    if constexpr (PV == 3) pa[m] = ld(bp, bl, row(c0 + m));
+#pragma unroll
+    for (int q = 0; q < m; ++q) {
+      const double* R = T + kCnFwd * min(r0 + c0 + q, nz + 1);
+      // the increments first, so that the field's own value is rounded once
+      double r = f23 * a1[q];
+      if constexpr (PV == 1 || PV == 2) r = __builtin_fma(-dm, pb[q] - pa[q], r);
+      if constexpr (PV == 3) r = __builtin_fma(-R[3], pa[q + 1] - pa[q], r);
+      r = __builtin_fma(R[0], v[q + 2] - v[q + 1], r);
+      r = __builtin_fma(-R[1], v[q + 1] - v[q], r);
+      r = __builtin_fma(f1, v[q + 1], r);
+      G[c0 + q] = R[5] != 0.0 ? R[4] : r;
+    }
+  };
+  if (len == N) {
+    rhs(0, std::integral_constant<int, N>());
+  } else {
+#pragma unroll
+    for (int c0 = 0; c0 < N; c0 += 4)
+      if (c0 < S) rhs(c0, std::integral_constant<int, 4>());
   }
+  double g = 0.0;
+#pragma unroll
+  for (int q = 0; q < N; ++q)
+    if (q < len) {
+      g = __builtin_fma(T[kCnFwd * (r0 + q) + 2], g, G[q]);
+      G[q] = g;
+    }
   gend[w][lane] = g;
-  if (w == 0) g0[lane] = G0;
-  if (lane == 0) pend[w] = pr;
+  back[w][lane] = bw;
   __syncthreads();
-  // G_{r0-1}, the value carried into this segment, and the segment's G
-  double C = g0[lane];
-  for (int q = 0; q < w; ++q) C = gend[q][lane] + pend[q] * C;
-  pr = 1.0;
+  // G_{r0-1}, the value carried into this segment (a segment's PF is its last
+  // row's)
+  double C = E.g0;
+  for (int q = 0; q < w; ++q) C = __builtin_fma(back[q][(S - 1) * kCnBack], C, gend[q][lane]);
+  const double* B = back[w];
+  // the segment with its carry; then backward, locally
+  double gl = g;
+  double x = 0.0;
 #pragma unroll
-  for (int q = 0; q < kCnSeg; ++q) {
-    const int k = min(r0 + q, n - 1);
-    const double ap = T[k].ap;
-    if (r0 + q < r1) {
-      pr = ap * pr;
-      G[q] = G[q] + pr * C;
-    }
-  }
-  // the top wall row: G_{nz+1} from G_nz, x_{nz+1}
-  if (w == P - 1) {
-    double Gn = 0.0;
-#pragma unroll
-    for (int q = 0; q < kCnSeg; ++q)
-      if (r0 + q == r1 - 1) Gn = G[q];
-    xtop[lane] = (rtop + T[n - 1].ap * Gn) * T[n - 1].rbp;
-  }
-  // backward, locally (the rows' coefficients read before the chain)
-  double cq[kCnSeg], rq[kCnSeg], bq[kCnSeg];
-#pragma unroll
-  for (int q = 0; q < kCnSeg; ++q) {
-    const int k = min(r0 + q, n - 1);
-    cq[q] = T[k].c;
-    rq[q] = T[k].rbp;
-    bq[q] = T[k].cbp;
-  }
-  double x = 0.0, qr = 1.0;
-#pragma unroll
-  for (int q = kCnSeg - 1; q >= 0; --q) {
-    if (r0 + q < r1) {
-      x = (G[q] - cq[q] * x) * rq[q];
-      qr = bq[q] * qr;
+  for (int q = N - 1; q >= 0; --q)
+    if (q < len) {
+      const double Gq = __builtin_fma(B[q * kCnBack], C, G[q]);
+      if (q == len - 1) gl = Gq;
+      x = __builtin_fma(-B[q * kCnBack + 2], x, Gq) * B[q * kCnBack + 1];
       G[q] = x;
     }
-  }
+  // the top wall row: G_{nz+1} from G_nz, x_{nz+1}
+  if (w == P - 1) xtop[lane] = __builtin_fma(E.at, gl, E.gt) * E.rbt;
   xfirst[w][lane] = x;
-  if (lane == 0) qfirst[w] = qr;
   __syncthreads();
   // x_{r1}, the value carried into this segment from above, and the stores
   double X = xtop[lane];
-  for (int q = P - 1; q > w; --q) X = xfirst[q][lane] + qfirst[q] * X;
-  double qk = 1.0, x1 = 0.0;
+  for (int q = P - 1; q > w; --q) X = __builtin_fma(back[q][3], X, xfirst[q][lane]);
+  const unsigned bs = live ? bl : 0x80000000u;          // a spare lane's stores are dropped
+  auto store = [&](double v, unsigned r) {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(int2v, v), b2, (int)bs, (int)r, 0);
+  };
+  double x1 = 0.0;
 #pragma unroll
-  for (int q = kCnSeg - 1; q >= 0; --q) {
-    const int k = r0 + q;
-    if (k < r1) {
-      qk = bq[q] * qk;
-      const double xk = G[q] + qk * X;
-      if (live) v2[at(k)] = xk;
-      x1 = xk;
+  for (int q = N - 1; q >= 0; --q)
+    if (q < len) {
+      x1 = __builtin_fma(B[q * kCnBack + 3], X, G[q]);
+      store(x1, (unsigned)(q + 1) * plane);
     }
-  }
-  if (live && w == 0) v2[at(0)] = (G0 - T[0].c * x1) * T[0].rbp;
-  if (live && w == P - 1) v2[at(n - 1)] = xtop[lane];
+  if (w == 0) store(__builtin_fma(E.c0, x1, E.g0 * E.rb0), 0u);
+  if (w == P - 1) store(xtop[lane], (unsigned)(len + 1) * plane);
 }
 
 unsigned cdiv(long long a, int b) { return (unsigned)((a + b - 1) / b); }
@@ -815,23 +800,73 @@ int plan_cn(const FlowGrid& G, int var, double rkdt, double rRe, double rPr, dou
     R[k].ap = a[k];
     R[k].bp = b[k];
     R[k].c = sup[k];
-    R[k].rbp = 1.0 / b[k];
-    R[k].cbp = -(sup[k] / b[k]);
   }
   *rows = std::move(R);
   return 0;
 }
 
-void launch_cn_column(const double* v1, double* v2, const double* p, const CnRow* T,
+// The segmented kernel takes columns of at most 256 cells whose 18 rows of a
+// segment lie within 2 GiB.
+bool cn_segmented(int nx, int ny, int nz) {
+  return nz <= kCnSeg * kCnSeg && (long long)(nx + 2) * (ny + 2) * 8 * (kCnSeg + 2) < (1LL << 31);
+}
+
+size_t cn_table_doubles(int nz) {
+  return std::max(sizeof(CnRow) / 8 * (size_t)(nz + 2),
+                  kCnFwd * (size_t)(nz + 2) + sizeof(CnEnds) / 8 + kCnSeg * kCnSeg * kCnBack);
+}
+
+std::vector<double> cn_table(const std::vector<CnRow>& rows, int nx, int ny, double rkdt) {
+  const int nz = (int)rows.size() - 2;
+  std::vector<double> t;
+  if (!cn_segmented(nx, ny, nz)) {
+    t.resize(sizeof(CnRow) / 8 * rows.size());
+    std::memcpy(t.data(), rows.data(), sizeof(CnRow) * rows.size());
+    return t;
+  }
+  // products of constants in extended precision, rounded once
+  typedef long double ld;
+  const ld h = (ld)rkdt * 0.5;
+  for (const CnRow& R : rows) {
+    const double fwd[kCnFwd] = {(double)(h * R.c1 * R.m1 * R.m3), (double)(h * R.c2 * R.m2 * R.m3), R.ap,
+                                rkdt * R.pz, R.cval, R.kind ? 1.0 : 0.0};
+    t.insert(t.end(), fwd, fwd + kCnFwd);
+  }
+  const CnRow &B = rows.front(), &E = rows.back();
+  for (double v : {B.cval, -(B.c / B.bp), 1.0 / B.bp, E.cval, E.ap, 1.0 / E.bp}) t.push_back(v);
+  // segments of S <= 16 rows: PF downward from the segment's start, QB from
+  // its end
+  const int S = (nz + kCnSeg - 1) / kCnSeg;
+  std::vector<double> back((size_t)kCnSeg * kCnSeg * kCnBack, 0.0);
+  for (int r0 = 1, w = 0; r0 <= nz; r0 += S, ++w) {
+    const int len = std::min(S, nz + 1 - r0);
+    double* b = back.data() + (size_t)w * kCnSeg * kCnBack;
+    ld pf = 1.0, qb = 1.0;
+    for (int q = 0; q < len; ++q) {
+      const CnRow& R = rows[r0 + q];
+      pf = R.ap * pf;
+      b[q * kCnBack] = (double)pf;
+      b[q * kCnBack + 1] = 1.0 / R.bp;
+      b[q * kCnBack + 2] = R.c;
+    }
+    for (int q = len - 1; q >= 0; --q) {
+      qb = -((ld)rows[r0 + q].c / rows[r0 + q].bp) * qb;
+      b[q * kCnBack + 3] = (double)qb;
+    }
+  }
+  t.insert(t.end(), back.begin(), back.end());
+  return t;
+}
+
+void launch_cn_column(const double* v1, double* v2, const double* p, const double* T,
                       const double* rdxe, const double* rdye, int nx, int ny, int nz, double f1,
                       double f2, double f3, double rkdt, int var, hipStream_t s) {
   const int pv = (p != nullptr && var <= 3) ? var : 0;
-  const double h = rkdt * 0.5;
-  if (nz <= kCnSeg * kCnSeg) {
-    // segments of S <= 16 rows, at most 16 of them
+  if (cn_segmented(nx, ny, nz)) {
     const int S = (nz + kCnSeg - 1) / kCnSeg, P = (nz + S - 1) / S;
     const dim3 g(cdiv((long long)nx * ny, 64)), b(64, P);
-#define CS(V) hipLaunchKernelGGL(k_cn_seg<V>, g, b, 0, s, v1, v2, p, T, rdxe, rdye, nx, ny, nz, S, f1, f2, f3, rkdt, h)
+    const double f23 = f2 * f3;
+#define CS(V) hipLaunchKernelGGL(k_cn_seg<V>, g, b, 0, s, v1, v2, p, T, rdxe, rdye, nx, ny, nz, S, f1, f23, rkdt)
     if (pv == 1) CS(1);
     else if (pv == 2) CS(2);
     else if (pv == 3) CS(3);
@@ -839,11 +874,15 @@ void launch_cn_column(const double* v1, double* v2, const double* p, const CnRow
 #undef CS
     return;
   }
+  const double h = rkdt * 0.5;
+  const CnRow* R = reinterpret_cast<const CnRow*>(T);
   const dim3 g(cdiv((long long)nx * ny, kFlowBlock)), b(kFlowBlock);
-  if (pv == 1) hipLaunchKernelGGL(k_cn_column<1>, g, b, 0, s, v1, v2, p, T, rdxe, rdye, nx, ny, nz, f1, f2, f3, rkdt, h);
-  else if (pv == 2) hipLaunchKernelGGL(k_cn_column<2>, g, b, 0, s, v1, v2, p, T, rdxe, rdye, nx, ny, nz, f1, f2, f3, rkdt, h);
-  else if (pv == 3) hipLaunchKernelGGL(k_cn_column<3>, g, b, 0, s, v1, v2, p, T, rdxe, rdye, nx, ny, nz, f1, f2, f3, rkdt, h);
-  else hipLaunchKernelGGL(k_cn_column<0>, g, b, 0, s, v1, v2, p, T, rdxe, rdye, nx, ny, nz, f1, f2, f3, rkdt, h);
+#define CC(V) hipLaunchKernelGGL(k_cn_column<V>, g, b, 0, s, v1, v2, p, R, rdxe, rdye, nx, ny, nz, f1, f2, f3, rkdt, h)
+  if (pv == 1) CC(1);
+  else if (pv == 2) CC(2);
+  else if (pv == 3) CC(3);
+  else CC(0);
+#undef CC
 }
 
 }  // namespace amg

@@ -11,8 +11,8 @@ struct amg_solver_s {
   double* d_phi_stage = nullptr;   // staging for the host entry point
   double* d_rhs_stage = nullptr;
   double* d_div_partial = nullptr; // divergence partials (amg_divergence_device)
-  amg::CnRow* d_cn = nullptr;      // rows of the vertical CN system (nz+2)
-  amg::CnRow* h_cn = nullptr;      //   and their pinned host staging
+  double* d_cn = nullptr;          // table of the vertical CN system (cn_table)
+  double* h_cn = nullptr;          //   and its pinned host staging
 };
 
 namespace amg {

@@ -5,7 +5,8 @@
   one) and lines across block ends, every variable type, bit-exact against
   ``oracle.dns``;
 * ``Psource`` and ``divergence``: slabs of fewer than 8 planes, a last slab of
-  one, positions across block ends, to 1e-13 (a handful of roundings per cell).
+  one, positions across block ends, to 1e-13 (a handful of roundings per cell);
+* the viscous step's segments.
 """
 import numpy as np
 import pytest
@@ -22,11 +23,11 @@ def _box(n):
     return box_grid(*n, beta=1.2, rho=1.0 + 0.2 * np.cos(2.0 * z))
 
 
-def _handle(g):
-    """A handle of any small grid: pressure walls on every face, one level."""
+def _handle(g, lx=1):
+    """A handle of any small grid: pressure walls on every face, x alone coarsened."""
     from anelastic_solve_amd import PressureSolver, default_config
     return PressureSolver(g, default_config(precision="fp64", smoother="RBPGS", tbc=(2,) * 6,
-                                            vbc=(0.0,) * 6, nlevels=(1, 1, 1)))
+                                            vbc=(0.0,) * 6, nlevels=(lx, 1, 1)))
 
 
 @pytest.mark.parametrize("n", [(2, 1, 1), (2, 2, 2), (4, 3, 3), (6, 5, 4), (2, 3, 130)])
@@ -65,4 +66,32 @@ def test_source_and_divergence_edges(cuda, n):
     assert relerr(div.cpu().numpy()[1:-1, 1:-1, 1:-1], want) < 1e-13
     assert abs(avg - wavg) <= 1e-13 * wavg and abs(most - wmost) <= 1e-13 * wmost
     assert tuple(at) == wat
+    s.close()
+
+
+@pytest.mark.parametrize("var", [1, 2, 3, 5])
+@pytest.mark.parametrize("n,lx", [((2, 2, 2), 1), ((6, 10, 16), 1), ((10, 6, 17), 1), ((64, 3, 77), 6),
+                                  ((48, 5, 33), 4), ((2, 2, 255), 1)])
+def test_viscous_step_edges(cuda, var, n, lx):
+    """``var_advance_CN_PL`` on columns of one row per segment, of a full and a
+    partial last segment, and of column counts that are no multiple of 64,
+    against ``oracle.dns`` to 1e-13 (as in test_gpu_flow)."""
+    torch = cuda
+    from anelastic_solve_amd import FlowBC
+    from oracle import dns
+    g = _box(n)
+    s = _handle(g, lx)
+    t = {1: (1, 6), 2: (2, 1), 3: (1, 2), 5: (2, 2)}[var]
+    if var == 5 and n[2] == 2:
+        t = (1, 2)
+    bc = FlowBC.make((True, True, False), {(3, 1, var): (t[0], 0.3), (3, 2, var): (t[1], -0.2)})
+    rng = np.random.Generator(np.random.PCG64(33))
+    v1, v2, p = (rng.standard_normal(g.shape) for _ in range(3))
+    p = None if var == 5 else p
+    args = (0.9, 0.45, 0.7, 0.02, var)
+    want = dns.cn_advance(v1, v2.copy(), *args, g.rho_or_ones(), _axes(g), bc.TB, bc.VB, 1e-2, 1.4, 0.9,
+                          p=p)
+    d1, d2 = (torch.from_numpy(a).cuda() for a in (v1, v2))
+    s.var_advance_CN_PL(d1, d2, *args, bc, 1e-2, 1.4, 0.9, p=None if p is None else torch.from_numpy(p).cuda())
+    assert relerr(d2.cpu().numpy(), want) <= 1e-13
     s.close()
