@@ -31,6 +31,9 @@ FLAGS = [
     "-Wno-unused-function", "-Wno-unused-result",
     # packed-FP32 instructions stay off (see the design notes)
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # leading scalar kernel arguments arrive in registers (a kernel's start does not
+    # wait for its argument segment)
+    "-mllvm", "-amdgpu-kernarg-preload-count=14",
     "-I", os.path.join(ROOT, "include"), "-I", CSRC,
 ]
 

@@ -23,9 +23,9 @@ namespace amg {
 // Coefficient table of one level (precision T): 3*nx + 3*ny + 3*nz values,
 //   [wxm | wxp | dx] [wym | wyp | dy] [wzm | wzp | dz]
 // with (A u)_ijk = wxm_i u_{i-1} + wxp_i u_{i+1} + ... + (dx_i+dy_j+dz_k) u_ijk.
-// The first 128 bytes are what nearly every kernel needs of a level, read in
-// one go (level_head in amg_kernels.hip).
-struct DevLevel {
+// What nearly every kernel needs of a level: two cache lines that a kernel
+// reads in one go (level_head in amg_kernels.hip).
+struct LevelHead {
   int nx, ny, nz, hx;
   // the instance's solve state, written by the device (the gate at the end
   // of every cycle) on every level of the instance:
@@ -47,6 +47,9 @@ struct DevLevel {
                              // (k_zline_table), or null
   const double* vol;         // [dxc(nx) | dyc(ny) | dzc(nz)] interior widths
   const double* rho;         // rho(z) interior, nz values
+};
+static_assert(sizeof(LevelHead) == 128, "two cache lines");
+struct DevLevel : LevelHead {
   int inst;                  // instance id (batched/served runs)
   int link;                  // FP64 finest entry: index of the FP32 finest level (mixed)
   int nullsp;                // the operator is singular (periodic/Neumann): constants in the null space
@@ -65,7 +68,8 @@ struct DevLevel {
   const double* bcfold;      // [x(nx) | y(ny) | z(nz)] boundary-value RHS shifts (finest only)
   const double* minvT;       // coarsest level: transposed dense (pseudo-)inverse, ncell^2
   const double* minv;        // the same, row-major, when the coarse solve is its own kernel
-  void* scr;                 // z-line scratch: nz * hx * ny values
+  const float* e32;          // mixed FP64 finest: u and f of the FP32 finest level (link)
+  float* r32;
   // separable direct solve of a coarse level (amg_direct.cpp, k_direct_*)
   // the direct level's tables, in its compute type (FP64 for an FP64
   // V-cycle, FP32 -- stored behind these pointers -- for a mixed solve's):
@@ -268,7 +272,7 @@ void launch_restrict(bool fp64, const DevLevel* L, const DevXfer* X, const Launc
 #endif
 constexpr long long kRestrictMinCells = AMG_RESTRICT_MIN_CELLS;
 constexpr long long kRestrictThreads = 1 << 18;
-__host__ __device__ inline int restrict222_k(const DevLevel& C) {
+__host__ __device__ inline int restrict222_k(const LevelHead& C) {
   const long long cells = (long long)C.nx * C.ny * C.nz;
   int k = 8;
   while (k > 1 && cells / k < kRestrictThreads) k >>= 1;
@@ -372,6 +376,7 @@ struct GateArgs {
   DevLevel* Lt;
   int nL;
   ItemGate* ig;
+  int slot, inst;              // of the item, when the launch has one
 };
 // Clears the state words of the instances of the items of ll.
 // only_stopped: just the instances whose solve has stopped (a reset that may

@@ -61,30 +61,47 @@ template <class A, class... V> __device__ __forceinline__ void pin_s(A& a, V&...
   }
 }
 
+// A kernel's list: the counts and the first item as scalar arguments, then the
+// list itself.  Scalar arguments are preloaded into registers by the dispatch
+// (kernarg preload), so a launch of one item (a single solve) starts with its
+// level's address at hand: it used to read the list, the item, the stop word
+// and then field after field, each from memory in turn, which small launches
+// mostly consist of.  Back to back: 64^3 FP64 point half-sweep 3.24 -> 2.69
+// us, 128^3 FP32 z-line 5.1 -> 4.8, 64^3 direct solve (three launches) 22.1
+// -> 18.8; also the 256^3 sweep 19.5 -> 18.5.
+#define LIST_PARAMS int ln, int lnb, int li0
+#define LIST_ARGS(ll) (ll).nitems, (ll).nblocks, (ll).items[0]
+
 __device__ __forceinline__ int xcd_swizzle(int b, int n);
 // The item of this block and the block's number within it (blocks swizzled
-// over the XCDs).  A launch of one item (a single solve) reads no list.
+// over the XCDs); b is the block's number in the launch.
 struct Work {
-  int t, idx, lb;
+  int t, idx, lb, b;
 };
-__device__ __forceinline__ Work work_item(const LaunchList& ll) {
-  int n = ll.nitems, nb = ll.nblocks, i0 = ll.items[0];
-  pin_s(n, nb, i0);
-  const int b = xcd_swizzle(blockIdx.x, nb);
-  if (n == 1) return {0, i0, b};
-  const int t = find_item(ll.prefix, n, b);
-  return {t, ll.items[t], b - ll.prefix[t]};
+__device__ __forceinline__ Work work_item(LIST_PARAMS, const LaunchList& ll) {
+  const int b = xcd_swizzle(blockIdx.x, lnb);
+  if (ln == 1) return {0, li0, b, b};
+  const int t = find_item(ll.prefix, ln, b);
+  return {t, ll.items[t], b - ll.prefix[t], b};
+}
+
+// The head of a level's descriptor, read in one go.
+__device__ __forceinline__ LevelHead level_head(const DevLevel& L) {
+  LevelHead h = L;
+  pin_s(h.nx, h.ny, h.nz, h.hx, h.stop, h.warm, h.skipc, h.pcur, h.gmhx, h.gmny, h.gshx, h.gsny, h.px,
+        h.py, h.pz, h.ncell, h.u, h.f, h.u2, h.co64, h.co32, h.zt, h.vol, h.rho);
+  return h;
 }
 
 // A gated cycle has stopped (DevLevel::stop): the kernel returns at once.
-__device__ __forceinline__ bool level_off(const DevLevel& L) { return L.stop != 0; }
+__device__ __forceinline__ bool level_off(const LevelHead& L) { return L.stop != 0; }
 
 // Zero-guess flags of a smoothing launch (bit 0: the other colour is zero;
 // bit 1: the own colour's old values are zero).  With kZgDyn, the finest
 // level's first sweep of a mixed cycle, they hold only when the cycle does
 // not continue the previous one's iterate (DevLevel::warm); kZgWarm marks
 // the launch that does that sweep when the cycle continues it.
-__device__ __forceinline__ int zero_flags(const DevLevel& L, int zero_guess) {
+__device__ __forceinline__ int zero_flags(const LevelHead& L, int zero_guess) {
   if (zero_guess & kZgWarm) return 0;
   if (!(zero_guess & kZgDyn)) return zero_guess;
   return L.warm ? 0 : (zero_guess & 3);
@@ -113,11 +130,11 @@ __device__ __forceinline__ double fm(double a, double b, double c) { return __bu
 __device__ __forceinline__ float over(float a, float d) { return a * __builtin_amdgcn_rcpf(d); }
 __device__ __forceinline__ double over(double a, double d) { return a / d; }
 
-template <class T> __device__ __forceinline__ sp<kG, const T> coefs(const DevLevel& L);
-template <> __device__ __forceinline__ sp<kG, const double> coefs<double>(const DevLevel& L) {
+template <class T> __device__ __forceinline__ sp<kG, const T> coefs(const LevelHead& L);
+template <> __device__ __forceinline__ sp<kG, const double> coefs<double>(const LevelHead& L) {
   return gp(L.co64);
 }
-template <> __device__ __forceinline__ sp<kG, const float> coefs<float>(const DevLevel& L) {
+template <> __device__ __forceinline__ sp<kG, const float> coefs<float>(const LevelHead& L) {
   return gp(L.co32);
 }
 
@@ -177,7 +194,7 @@ struct Nb {
   int c, xm, xp, ym, yp, zm, zp;
 };
 
-__device__ __forceinline__ Nb neighbours(const DevLevel& L, int i, int j, int k) {
+__device__ __forceinline__ Nb neighbours(const LevelHead& L, int i, int j, int k) {
   const int hx = L.hx, ny = L.ny, nz = L.nz;
   const int col = (i + j) & 1, oth = col ^ 1, m = i >> 1, r = i & 1;
   int ml = m - 1 + r; if (ml < 0) ml = hx - 1;
@@ -205,7 +222,7 @@ __device__ __forceinline__ int gm_div(int n, unsigned m, int sh) {
   return (int)((t + ((un - t) >> (sh & 0xff))) >> (sh >> 8));
 }
 
-__device__ __forceinline__ void decode(const DevLevel& L, int e, int& i, int& j, int& k) {
+__device__ __forceinline__ void decode(const LevelHead& L, int e, int& i, int& j, int& k) {
   const int t = gm_div(e, L.gmhx, L.gshx);
   const int m = e - t * L.hx;
   const int c = t & 1;
@@ -217,7 +234,7 @@ __device__ __forceinline__ void decode(const DevLevel& L, int e, int& i, int& j,
 
 // Off-diagonal stencil sum, in a fixed order: x-, x+, y-, y+, z-, z+.
 template <class T, class CP>
-__device__ __forceinline__ T offsum(CP co, const DevLevel& L, int i, int j, int k, T uxm, T uxp,
+__device__ __forceinline__ T offsum(CP co, const LevelHead& L, int i, int j, int k, T uxm, T uxp,
                                     T uym, T uyp, T uzm, T uzp) {
   const int nx = L.nx, ny = L.ny;
   const auto cy = co + 3 * nx;
@@ -231,7 +248,7 @@ __device__ __forceinline__ T offsum(CP co, const DevLevel& L, int i, int j, int 
 }
 
 template <class T, class CP>
-__device__ __forceinline__ T diag_at(CP co, const DevLevel& L, int i, int j, int k) {
+__device__ __forceinline__ T diag_at(CP co, const LevelHead& L, int i, int j, int k) {
   const int nx = L.nx, ny = L.ny;
   const auto cy = co + 3 * nx;
   const auto cz = cy + 3 * ny;
@@ -244,7 +261,7 @@ __device__ __forceinline__ T diag_at(CP co, const DevLevel& L, int i, int j, int
 // e enumerates the cells of the colour; in plane k the colour is column
 // colour (parity+k)&1, so consecutive e are one contiguous half-row.
 template <class T, class UP, class FP, class CP>
-__device__ __forceinline__ void rb_point_mjk(const DevLevel& L, UP u, FP f, CP co, int m, int j,
+__device__ __forceinline__ void rb_point_mjk(const LevelHead& L, UP u, FP f, CP co, int m, int j,
                                              int k, int parity, int zero_guess) {
   const int c = (k + parity) & 1;
   const int i = 2 * m + ((c + j) & 1);
@@ -261,7 +278,7 @@ __device__ __forceinline__ void rb_point_mjk(const DevLevel& L, UP u, FP f, CP c
 }
 
 template <class T, class UP, class FP, class CP>
-__device__ __forceinline__ void rb_point_elem(const DevLevel& L, UP u, FP f, CP co, int e,
+__device__ __forceinline__ void rb_point_elem(const LevelHead& L, UP u, FP f, CP co, int e,
                                               int parity, int zero_guess) {
   const int row = gm_div(e, L.gmhx, L.gshx), m = e - row * L.hx;
   const int k = gm_div(row, L.gmny, L.gsny), j = row - k * L.ny;
@@ -282,13 +299,12 @@ __device__ __forceinline__ void rb_point_small(const DevLevel& L, UP u, FP f, CP
 }
 
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_rb_point(const DevLevel* __restrict__ Lt, LaunchList ll,
-                                                     int parity, int zero_guess) {
-  const int b = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int t = find_item(ll.prefix, ll.nitems, b);
-  const DevLevel& L = Lt[ll.items[t]];
+__global__ __launch_bounds__(kBlock) void k_rb_point(const DevLevel* __restrict__ Lt, LIST_PARAMS,
+                                                     int parity, int zero_guess, LaunchList ll) {
+  const Work wk = work_item(ln, lnb, li0, ll);
+  const LevelHead L = level_head(Lt[wk.idx]);
   if (level_off(L)) return;
-  const int e = (b - ll.prefix[t]) * kBlock + threadIdx.x;
+  const int e = wk.lb * kBlock + threadIdx.x;
   if (e < L.hx * L.ny * L.nz)
     rb_point_elem<T>(L, gfield<T>(L.u), gfield<const T>((const void*)L.f), coefs<T>(L), e, parity,
                      zero_flags(L, zero_guess));
@@ -305,16 +321,15 @@ __global__ __launch_bounds__(kBlock) void k_rb_point(const DevLevel* __restrict_
 // per thread, those of z (wave-uniform) from the scalar cache.  The update is
 // rb_point_mjk's, in its order.
 template <class T, int K>
-__global__ __launch_bounds__(kBlock) void k_rb_march(const DevLevel* __restrict__ Lt, LaunchList ll,
-                                                     int parity, int zero_guess) {
-  const int b = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int t = find_item(ll.prefix, ll.nitems, b);
-  const DevLevel& L = Lt[ll.items[t]];
+__global__ __launch_bounds__(kBlock) void k_rb_march(const DevLevel* __restrict__ Lt, LIST_PARAMS,
+                                                     int parity, int zero_guess, LaunchList ll) {
+  const Work wk = work_item(ln, lnb, li0, ll);
+  const LevelHead L = level_head(Lt[wk.idx]);
   if (level_off(L)) return;
   const int zg = zero_flags(L, zero_guess);
   const int hx = L.hx, ny = L.ny, nz = L.nz, nx = L.nx;
   const int npos = hx * ny, ncb = (npos + kBlock - 1) / kBlock;
-  const int lb = b - ll.prefix[t];
+  const int lb = wk.lb;
   const int bk = lb / ncb, pos = (lb - bk * ncb) * kBlock + threadIdx.x;
   if (pos >= npos) return;
   const int j = gm_div(pos, L.gmhx, L.gshx), m = pos - j * hx;
@@ -433,7 +448,7 @@ __device__ __forceinline__ T zline_nbr(T wxl, T wxr, T wys, T wyn, T xl, T xr, T
 // within the workgroup's 32) are then per lane, and the z rows are staged
 // in LDS.  Every lane does the same operations in either shape.
 template <class T, int S, int C, bool NBR, bool LEAN, bool H>
-__device__ __forceinline__ void zline_group(const DevLevel& L, int parity, int zero_guess, int col0,
+__device__ __forceinline__ void zline_group(const LevelHead& L, int parity, int zero_guess, int col0,
                                             int p, int lane, int P, T* __restrict__ lds, bool act) {
   const int hx = L.hx, ny = L.ny, nz = L.nz, nx = L.nx;
   const int ncol = hx * ny;
@@ -686,11 +701,10 @@ __device__ __forceinline__ void zline_group(const DevLevel& L, int parity, int z
 // registers.
 template <class T, int S, int C, bool NBR, bool LEAN, bool H>
 __global__ __launch_bounds__(H ? 512 : 1024, H ? 2 : ((LEAN && sizeof(T) == 4) ? 8 : 4)) void k_zline(
-    const DevLevel* __restrict__ Lt, LaunchList ll, int parity, int zero_guess) {
+    const DevLevel* __restrict__ Lt, LIST_PARAMS, int parity, int zero_guess, LaunchList ll) {
   extern __shared__ unsigned char lds_raw[];
-  const int b = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int t = find_item(ll.prefix, ll.nitems, b);
-  const DevLevel& L = Lt[ll.items[t]];
+  const Work wk = work_item(ln, lnb, li0, ll);
+  const LevelHead L = level_head(Lt[wk.idx]);
   if (level_off(L)) return;
   // the first sweep of a mixed cycle's finest level runs as two launches,
   // from zero (NBR false) and continuing the iterate (kZgWarm): one returns
@@ -701,11 +715,11 @@ __global__ __launch_bounds__(H ? 512 : 1024, H ? 2 : ((LEAN && sizeof(T) == 4) ?
   if constexpr (H) {
     const int cl = threadIdx.x & 31;
     zline_group<T, S, C, NBR, LEAN, true>(L, parity, zero_flags(L, zero_guess),
-                                          (b - ll.prefix[t]) * 32 + cl, 2 * seg + (threadIdx.x >> 5),
+                                          wk.lb * 32 + cl, 2 * seg + (threadIdx.x >> 5),
                                           cl, 2 * blockDim.y, reinterpret_cast<T*>(lds_raw), true);
   } else {
     zline_group<T, S, C, NBR, LEAN, false>(L, parity, zero_flags(L, zero_guess),
-                                           (b - ll.prefix[t]) * 64 + threadIdx.x, seg, threadIdx.x,
+                                           wk.lb * 64 + threadIdx.x, seg, threadIdx.x,
                                            blockDim.y, reinterpret_cast<T*>(lds_raw), true);
   }
 }
@@ -828,23 +842,18 @@ __device__ __forceinline__ void buf_st(Buf b, unsigned lane, unsigned row, float
 // memory phase and by the start of its 8192 waves, not by arithmetic.
 template <bool H>
 __global__ __launch_bounds__(H ? 512 : 1024, H ? 2 : 8) void k_zline_shared(
-    const DevLevel* __restrict__ Lt, int parity, int zero_guess, LaunchList ll) {
+    const DevLevel* __restrict__ Lt, LIST_PARAMS, int parity, int zero_guess, LaunchList ll) {
   extern __shared__ float zlds[];
   constexpr int S = kZSeg, CW = H ? 32 : 64;
-  const Work wk = work_item(ll);
-  const DevLevel& L = Lt[wk.idx];
-  int nx = L.nx, ny = L.ny, nz = L.nz, hx = L.hx, stop = L.stop, warm = L.warm, pz = L.pz;
-  unsigned gmhx = L.gmhx;
-  int gshx = L.gshx, ncell = L.ncell;
-  const void *up = L.u, *fp = L.f;
-  const float *cp = L.co32, *zp = L.zt;
-  pin_s(nx, ny, nz, hx, stop, warm, pz, gmhx, gshx, ncell, up, fp, cp, zp);
-  if (stop) return;
+  const Work wk = work_item(ln, lnb, li0, ll);
+  const LevelHead L = level_head(Lt[wk.idx]);
+  if (level_off(L)) return;
+  const int nx = L.nx, ny = L.ny, nz = L.nz, hx = L.hx;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y), tx = threadIdx.x;
   const int half = H ? tx >> 5 : 0, lane = tx & (CW - 1);
   const int P = (nz + S - 1) / S, PA = H ? (P + 1) & ~1 : P;
   const int p = H ? 2 * wave + half : wave;
-  const sp<kG, const float> zr = gp(zp) + (H ? 2 * wave : wave) * kZRec;
+  const sp<kG, const float> zr = gp(L.zt) + (H ? 2 * wave : wave) * kZRec;
   float* const zl = zlds + 4 * PA * CW + 2 * wave * kZRec;   // H: the wave's two records
   float ra[S], rd[S], tback = 0.0f, tstep = 0.0f, tr[6];
   if constexpr (H) {
@@ -866,18 +875,18 @@ __global__ __launch_bounds__(H ? 512 : 1024, H ? 2 : 8) void k_zline_shared(
   auto stepw = [&](int q) { return H ? rec(kZRecStep + q) : word(tstep, q); };
   const int col0 = wk.lb * CW + lane, ncol = hx * ny;
   const int col = min(col0, ncol - 1);
-  const int j = gm_div(col, gmhx, gshx), m = col - j * hx;
+  const int j = gm_div(col, L.gmhx, L.gshx), m = col - j * hx;
   const int c = parity, oth = parity ^ 1;
   const int r = (c + j) & 1, i = 2 * m + r;
   int ml = m - 1 + r; if (ml < 0) ml = hx - 1;
   int mr = m + r;     if (mr >= hx) mr = 0;
   const int jm = (j == 0) ? ny - 1 : j - 1, jp = (j == ny - 1) ? 0 : j + 1;
-  const sp<kG, const float> co = gp(cp);
+  const sp<kG, const float> co = gp(L.co32);
   const sp<kG, const float> cy = co + 3 * nx;
   const sp<kG, const float> cz = cy + 3 * ny;
   const float wxl = co[i], wxr = co[nx + i], wys = cy[j], wyn = cy[ny + j];
   constexpr unsigned W = sizeof(float);
-  const Buf u = field_buf(up, (unsigned)ncell * W), f = field_buf(fp, (unsigned)ncell * W);
+  const Buf u = field_buf(L.u, (unsigned)L.ncell * W), f = field_buf(L.f, (unsigned)L.ncell * W);
   const unsigned plane = (unsigned)(ny * 2 * hx) * W;
   const int ks = p * S, len = max(0, min(S, nz - ks));
   const unsigned bown = (unsigned)cidx(m, j, 0, c, hx, ny) * W;
@@ -887,9 +896,9 @@ __global__ __launch_bounds__(H ? 512 : 1024, H ? 2 : 8) void k_zline_shared(
   const unsigned bno = (unsigned)cidx(m, jp, 0, oth, hx, ny) * W;
   // the sweep from zero reads b alone; a mixed cycle's first sweep is one
   // unless the cycle continues the previous one's iterate (kZgDyn)
-  const int zg = (zero_guess & kZgDyn) && warm ? 0 : zero_guess & 3;
+  const int zg = (zero_guess & kZgDyn) && L.warm ? 0 : zero_guess & 3;
   // periodic z: the lagged wrap values, as in zline_group
-  const bool lag = pz != 0 && !(zg & 2);
+  const bool lag = L.pz != 0 && !(zg & 2);
   float lagb = 0.0f, lagt = 0.0f;
   if (lag) {
     const float ubot = buf_ld(u, bown, (unsigned)(nz - 1) * plane), utop = buf_ld(u, bown, 0);
@@ -1013,7 +1022,7 @@ template <> struct TailNz<double> { static constexpr int value = kTailNz64; };
 // right-hand-side data and the z coefficients) is issued before the
 // elimination; with EXACT (nz == NZ) the chains carry no predicates.
 template <class T, int NZ, bool EXACT, class UP, class FP, class CP>
-__device__ __forceinline__ void zline_column(const DevLevel& L, UP u, FP f, CP co, int parity,
+__device__ __forceinline__ void zline_column(const LevelHead& L, UP u, FP f, CP co, int parity,
                                              int zero_guess, int col) {
   const int hx = L.hx, ny = L.ny, nx = L.nx;
   const int nz = EXACT ? NZ : L.nz;
@@ -1093,7 +1102,7 @@ __device__ __forceinline__ void zline_column(const DevLevel& L, UP u, FP f, CP c
 // Dispatch on the column length: an exact instantiation for full columns
 // of NZ, NZ/2 and NZ/4 cells, the predicated one otherwise.
 template <class T, int NZ, class UP, class FP, class CP>
-__device__ __forceinline__ void zline_column_n(const DevLevel& L, UP u, FP f, CP co, int parity,
+__device__ __forceinline__ void zline_column_n(const LevelHead& L, UP u, FP f, CP co, int parity,
                                                int zero_guess, int col) {
   const int nz = L.nz;
   if (nz == NZ) zline_column<T, NZ, true>(L, u, f, co, parity, zero_guess, col);
@@ -1104,20 +1113,19 @@ __device__ __forceinline__ void zline_column_n(const DevLevel& L, UP u, FP f, CP
 
 // The standalone short-column sweep (tests of the tail's line solve).
 template <class T, class UP, class FP, class CP>
-__device__ __forceinline__ void zline_column_any(const DevLevel& L, UP u, FP f, CP co, int parity,
+__device__ __forceinline__ void zline_column_any(const LevelHead& L, UP u, FP f, CP co, int parity,
                                                  int zero_guess, int col) {
   if (L.nz <= 16 || TailNz<T>::value <= 16) zline_column_n<T, 16>(L, u, f, co, parity, zero_guess, col);
   else zline_column_n<T, TailNz<T>::value>(L, u, f, co, parity, zero_guess, col);
 }
 
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_zline_col(const DevLevel* __restrict__ Lt, LaunchList ll,
-                                                      int parity, int zero_guess) {
-  const int b = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int t = find_item(ll.prefix, ll.nitems, b);
-  const DevLevel& L = Lt[ll.items[t]];
+__global__ __launch_bounds__(kBlock) void k_zline_col(const DevLevel* __restrict__ Lt, LIST_PARAMS,
+                                                      int parity, int zero_guess, LaunchList ll) {
+  const Work wk = work_item(ln, lnb, li0, ll);
+  const LevelHead L = level_head(Lt[wk.idx]);
   if (level_off(L)) return;
-  const int e = (b - ll.prefix[t]) * kBlock + threadIdx.x;
+  const int e = wk.lb * kBlock + threadIdx.x;
   if (e < L.hx * L.ny)
     zline_column_any<T>(L, gfield<T>(L.u), gfield<const T>((const void*)L.f), coefs<T>(L), parity,
                         zero_flags(L, zero_guess), e);
@@ -1130,8 +1138,8 @@ __global__ __launch_bounds__(kBlock) void k_zline_col(const DevLevel* __restrict
 // FX, FY, FZ: the coarsening factors (1 or 2), compile-time so that the
 // children loop unrolls and its loads are issued together.
 template <class T, int FX, int FY, int FZ, class UP, class FP, class CP, class VP, class CFP>
-__device__ __forceinline__ void restrict_elem(const DevLevel& F, UP u, FP f, CP co, VP vol,
-                                              const DevLevel& C, CFP fc, int e) {
+__device__ __forceinline__ void restrict_elem(const LevelHead& F, UP u, FP f, CP co, VP vol,
+                                              const LevelHead& C, CFP fc, int e) {
   // nx = 2 hx: e / nx = (e >> 1) / hx
   const int JK = gm_div(e >> 1, C.gmhx, C.gshx), I = e - JK * C.nx;
   const int K = gm_div(JK, C.gmny, C.gsny), J = JK - K * C.ny;
@@ -1161,8 +1169,8 @@ __device__ __forceinline__ void restrict_elem(const DevLevel& F, UP u, FP f, CP 
 }
 
 template <class T, class UP, class FP, class CP, class VP, class CFP>
-__device__ __forceinline__ void restrict_any(const DevLevel& F, UP u, FP f, CP co, VP vol,
-                                             const DevLevel& C, CFP fc, const DevXfer& x, int e) {
+__device__ __forceinline__ void restrict_any(const LevelHead& F, UP u, FP f, CP co, VP vol,
+                                             const LevelHead& C, CFP fc, const DevXfer& x, int e) {
   const int code = (x.fx - 1) * 4 + (x.fy - 1) * 2 + (x.fz - 1);
   switch (code) {
     case 7: restrict_elem<T, 2, 2, 2>(F, u, f, co, vol, C, fc, e); break;
@@ -1176,16 +1184,31 @@ __device__ __forceinline__ void restrict_any(const DevLevel& F, UP u, FP f, CP c
   }
 }
 
+// A transfer's descriptor and its two levels' heads: two reads, not one per
+// field used.
+__device__ __forceinline__ DevXfer xfer_of(const DevXfer& X) {
+  DevXfer x = X;
+  pin_s(x.fine, x.coarse, x.fx, x.fy, x.fz, x.skip, x.rskip, x.pmx, x.pmy, x.psx, x.psy);
+  return x;
+}
+__device__ __forceinline__ void level_heads(const DevLevel& A, const DevLevel& B, LevelHead& a,
+                                            LevelHead& b) {
+  a = A;
+  b = B;
+  pin_s(a.nx, a.ny, a.nz, a.hx, a.stop, a.gmhx, a.gmny, a.gshx, a.gsny, a.px, a.py, a.pz, a.u, a.f);
+  pin_s(a.co64, a.co32, a.vol, b.nx, b.ny, b.nz, b.hx, b.gmhx, b.gmny, b.gshx, b.gsny, b.ncell, b.u, b.f);
+}
+
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_restrict(const DevLevel* __restrict__ Lt,
-                                                     const DevXfer* __restrict__ X, LaunchList ll) {
-  const int b = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int t = find_item(ll.prefix, ll.nitems, b);
-  const DevXfer x = X[ll.items[t]];
-  const DevLevel& C = Lt[x.coarse];
-  const DevLevel& F = Lt[x.fine];
+                                                     const DevXfer* __restrict__ X, LIST_PARAMS,
+                                                     LaunchList ll) {
+  const Work wk = work_item(ln, lnb, li0, ll);
+  const DevXfer x = xfer_of(X[wk.idx]);
+  LevelHead F, C;
+  level_heads(Lt[x.fine], Lt[x.coarse], F, C);
   if (level_off(F)) return;
-  const int e = (b - ll.prefix[t]) * kBlock + threadIdx.x;
+  const int e = wk.lb * kBlock + threadIdx.x;
   if (e < C.ncell)
     restrict_any<T>(F, gfield<const T>((const void*)F.u), gfield<const T>((const void*)F.f),
                     coefs<T>(F), gp(F.vol), C, gfield<T>(C.f), x, e);
@@ -1218,7 +1241,7 @@ __device__ __forceinline__ constexpr bool restrict_keeps(int cx, int cy, int h) 
 }
 
 template <class T, int SK>
-__device__ __forceinline__ void restrict222_cols(const DevLevel& F, const DevLevel& C, int I, int J,
+__device__ __forceinline__ void restrict222_cols(const LevelHead& F, const LevelHead& C, int I, int J,
                                                  int K0, int K1) {
   const auto u = gfield<const T>((const void*)F.u);
   const auto f = gfield<const T>((const void*)F.f);
@@ -1326,17 +1349,16 @@ __device__ __forceinline__ void restrict222_cols(const DevLevel& F, const DevLev
 // pre-smoothing); 0 forms every residual.
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_restrict222(const DevLevel* __restrict__ Lt,
-                                                        const DevXfer* __restrict__ X,
-                                                        LaunchList ll, int use_skip) {
-  const int b = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int t = find_item(ll.prefix, ll.nitems, b);
-  const DevXfer x = X[ll.items[t]];
-  const DevLevel& C = Lt[x.coarse];
-  const DevLevel& F = Lt[x.fine];
+                                                        const DevXfer* __restrict__ X, LIST_PARAMS,
+                                                        int use_skip, LaunchList ll) {
+  const Work wk = work_item(ln, lnb, li0, ll);
+  const DevXfer x = xfer_of(X[wk.idx]);
+  LevelHead F, C;
+  level_heads(Lt[x.fine], Lt[x.coarse], F, C);
   if (level_off(F)) return;
   const int cols = C.nx * C.ny;
   const int ncb = (cols + kBlock - 1) / kBlock;
-  const int lb = b - ll.prefix[t];
+  const int lb = wk.lb;
   const int bk = lb / ncb, col = (lb - bk * ncb) * kBlock + threadIdx.x;
   if (col >= cols) return;
   const int J = gm_div(col >> 1, C.gmhx, C.gshx), I = col - J * C.nx;   // col / nx, nx = 2 hx
@@ -1425,7 +1447,7 @@ __device__ __forceinline__ constexpr bool prolong_keeps(int h, int q, int a) {
 }
 
 template <class T, int FX, int FY, int FZ, int SK = kXferSkipNone, class UP, class CUP>
-__device__ __forceinline__ void prolong_dual(const DevLevel& F, UP u, const DevLevel& C, CUP uc,
+__device__ __forceinline__ void prolong_dual(const DevLevel& F, UP u, const LevelHead& C, CUP uc,
                                              const DevXfer& x, int e) {
   static_assert(SK == kXferSkipNone || (FX == 2 && FY == 2 && FZ == 2), "skip: 2:2:2 duals only");
   constexpr int NX = FX == 2 ? 2 : 1, NY = FY == 2 ? 2 : 1, NZ = FZ == 2 ? 2 : 1;
@@ -1501,7 +1523,7 @@ __device__ __forceinline__ void prolong_dual(const DevLevel& F, UP u, const DevL
 }
 
 template <class T, class UP, class CUP>
-__device__ __forceinline__ void prolong_any(const DevLevel& F, UP u, const DevLevel& C, CUP uc,
+__device__ __forceinline__ void prolong_any(const DevLevel& F, UP u, const LevelHead& C, CUP uc,
                                             const DevXfer& x, int e, int skip = kXferSkipNone) {
   const int code = (x.fx - 1) * 4 + (x.fy - 1) * 2 + (x.fz - 1);
   switch (code) {
@@ -1527,16 +1549,19 @@ __device__ __forceinline__ void prolong_any(const DevLevel& F, UP u, const DevLe
 // every cell.
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_prolong(const DevLevel* __restrict__ Lt,
-                                                    const DevXfer* __restrict__ X, LaunchList ll,
-                                                    int use_skip) {
-  const int b = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int t = find_item(ll.prefix, ll.nitems, b);
-  const DevXfer x = X[ll.items[t]];
-  const DevLevel& F = Lt[x.fine];
-  const DevLevel& C = Lt[x.coarse];
+                                                    const DevXfer* __restrict__ X, LIST_PARAMS,
+                                                    int use_skip, LaunchList ll) {
+  const Work wk = work_item(ln, lnb, li0, ll);
+  const DevXfer x = xfer_of(X[wk.idx]);
+  DevLevel F = Lt[x.fine];
+  LevelHead C;
+  pin_s(F.bcx0, F.bcx1, F.bcy0, F.bcy1, F.bcz0, F.bcz1);
+  level_heads(F, Lt[x.coarse], F, C);
   if (level_off(F)) return;
-  const int e = (b - ll.prefix[t]) * kBlock + threadIdx.x;
-  if (e < prolong_duals(F, C, x))
+  const int e = wk.lb * kBlock + threadIdx.x;
+  const int nd = prolong_duals_dir(C.nx, x.fx, F.px) * prolong_duals_dir(C.ny, x.fy, F.py) *
+                 prolong_duals_dir(C.nz, x.fz, F.pz);
+  if (e < nd)
     prolong_any<T>(F, gfield<T>(F.u), C, gfield<const T>((const void*)C.u), x, e,
                    use_skip ? x.skip : kXferSkipNone);
 }
@@ -1939,25 +1964,30 @@ __device__ __forceinline__ void fine_march(sp<kG, const double> __restrict__ u,
 // shifted b back, mixed keeps b and records the shift in the instance's
 // bshift word, which its outer steps subtract as they load b.
 template <int MODE, bool SHIFT>
-__global__ __launch_bounds__(kBlock) void k_fine(DevLevel* __restrict__ Lt, LaunchList ll,
+__global__ __launch_bounds__(kBlock) void k_fine(DevLevel* __restrict__ Lt, LIST_PARAMS,
                                                  const double* __restrict__ csum,
-                                                 double* __restrict__ partial) {
+                                                 double* __restrict__ partial, LaunchList ll) {
   constexpr int NV = MODE == kCorrDefect32 ? 3 : 2;
-  const int b = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int t = find_item(ll.prefix, ll.nitems, b);
-  const DevLevel& L = Lt[ll.items[t]];
+  const Work wk = work_item(ln, lnb, li0, ll);
+  const int b = wk.b, t = wk.t;
+  const DevLevel& D = Lt[wk.idx];
+  // the FP32 finest level's fields (mixed; an FP64 solve has none)
+  const float* e32 = D.e32;
+  float* r32 = D.r32;
+  double bshift = D.bshift, vsum = D.vsum;
+  int nullsp = D.nullsp;
+  pin_s(e32, r32, bshift, vsum, nullsp);
+  const LevelHead L = level_head(D);
   if (level_off(L)) return;
   // the first cycle of a pair: no correction (its gate reads no norms)
   if (MODE == kCorrDefect32 && L.skipc) return;
-  // the FP32 finest level (mixed); an FP64 solve has none and reads no correction
-  const DevLevel& S = Lt[L.link >= 0 ? L.link : ll.items[t]];
   const int hx = L.hx, nx = L.nx, ny = L.ny, nz = L.nz;
   // the current FP64 pressure and its ping-pong partner
   const void* pin = L.pcur ? L.u2 : L.u;
   void* pout = L.pcur ? L.u : L.u2;
   const int plane = 2 * hx * ny;
   const int ncb = (plane + kBlock - 1) / kBlock;
-  const int lb = b - ll.prefix[t];
+  const int lb = wk.lb;
   const int bk = lb / ncb, bc = lb - bk * ncb;
   const int col = bc * kBlock + threadIdx.x;
   const int k0 = bk * kMarchK, k1 = min(k0 + kMarchK, nz);
@@ -1973,12 +2003,12 @@ __global__ __launch_bounds__(kBlock) void k_fine(DevLevel* __restrict__ Lt, Laun
     const auto co = gp(L.co64);
     const auto cy = co + 3 * nx;
     const auto cz = cy + 3 * ny;
-    const double cs = MODE == kCorrDefect32 ? L.bshift : (SHIFT && L.nullsp) ? csum[t] / L.vsum : 0.0;
-    if (SHIFT && MODE == kDefect32 && lb == 0 && threadIdx.x == 0) Lt[ll.items[t]].bshift = cs;
+    const double cs = MODE == kCorrDefect32 ? bshift : (SHIFT && nullsp) ? csum[t] / vsum : 0.0;
+    if (SHIFT && MODE == kDefect32 && lb == 0 && threadIdx.x == 0) Lt[wk.idx].bshift = cs;
     fine_march<MODE, NV, SHIFT>(gfield<const double>(pin),
-                         gfield<const float>((const void*)S.u), gfield<double>(L.f), cs,
+                         gp(e32), gfield<double>(L.f), cs,
                          gfield<double>(pout),
-                         gfield<float>(S.f), cz, nz, plane, col, (j * 2 + oth) * hx + ml,
+                         gp(r32), cz, nz, plane, col, (j * 2 + oth) * hx + ml,
                          (j * 2 + oth) * hx + mr, (jm * 2 + oth) * hx + m, (jp * 2 + oth) * hx + m,
                          co[i], co[nx + i], cy[j], cy[ny + j], cy[2 * ny + j], co[2 * nx + i], k0, k1, v);
   }
@@ -2023,7 +2053,7 @@ struct GatePre {
   int gslot, inst;
 };
 __device__ __forceinline__ GatePre gate_pre(const ItemGate* g, const double* out, const double* outc,
-                                            const DevLevel& L) {
+                                            const DevLevel& L, int slot, int inst) {
   GatePre P;
   for (int q = 0; q < 4; ++q) P.o[q] = out[q];
   P.oc[0] = outc[0];
@@ -2041,8 +2071,8 @@ __device__ __forceinline__ GatePre gate_pre(const ItemGate* g, const double* out
   P.rprev = g->rprev;
   P.skipc = L.skipc;
   P.warm = L.warm;
-  P.gslot = L.gslot;
-  P.inst = L.inst;
+  P.gslot = slot;
+  P.inst = inst;
   return P;
 }
 
@@ -2125,22 +2155,26 @@ __global__ void k_gate_init(LaunchList ll, const double* __restrict__ out, ItemG
 // per-instance gates, thread 0 of every item's block then ends its cycle and
 // the block's threads write the resulting state words, one table entry each.
 constexpr int kFinBlock = 1024;
-__global__ __launch_bounds__(kFinBlock) void k_finalize(LaunchList ll, const double* __restrict__ partial,
-                                                        int nvals, int op_sum, double* __restrict__ out,
-                                                        int ostride, GateArgs ga) {
+__global__ __launch_bounds__(kFinBlock) void k_finalize(LIST_PARAMS, int nvals, int op_sum,
+                                                        const double* __restrict__ partial,
+                                                        double* __restrict__ out, int ostride,
+                                                        GateArgs ga, LaunchList ll) {
   __shared__ double sm[kFinBlock / 64];
   const int t = blockIdx.x;
-  const int b0 = ll.prefix[t], b1 = ll.prefix[t + 1];
+  const bool one = ln == 1;
+  const int b0 = one ? 0 : ll.prefix[t], b1 = one ? lnb : ll.prefix[t + 1];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   // the gate's inputs, loaded before the fold (thread 0), and the instance
-  // number of every thread's first table entry (never written on the device)
+  // number of every thread's first table entry (never written on the device);
+  // a launch of one item knows its gate's place
   GatePre gpre;
   int inst0 = -1;
   if (ga.ig) {
     if (threadIdx.x < ga.nL) inst0 = ga.Lt[threadIdx.x].inst;
     if (threadIdx.x == 0) {
-      const DevLevel& L = ga.Lt[ll.items[t]];
-      gpre = gate_pre(ga.ig + L.gslot, ga.out + (size_t)t * 4, ga.outc + (size_t)t * 2, L);
+      const DevLevel& L = ga.Lt[one ? li0 : ll.items[t]];
+      const int slot = one ? ga.slot : L.gslot, inst = one ? ga.inst : L.inst;
+      gpre = gate_pre(ga.ig + slot, ga.out + (size_t)t * 4, ga.outc + (size_t)t * 2, L, slot, inst);
     }
   }
   // one pass over the partials for every value (nvals <= 4), kFinU
@@ -2781,20 +2815,24 @@ __device__ __forceinline__ void stage3(int na, LA&& la, SA&& sa, int nb, LB&& lb
 // dscr + n.  Either is My (X Mx[:, slab]) with the whole plane X staged.
 // The tables (dmat, dinv, dscr) hold CT values.
 template <class T, class CT, bool FWD>
-__global__ __launch_bounds__(kBlock) void k_direct_xy(const DevLevel* __restrict__ Lt, LaunchList ll) {
+__global__ __launch_bounds__(kBlock) void k_direct_xy(const DevLevel* __restrict__ Lt, LIST_PARAMS,
+                                                      LaunchList ll) {
   extern __shared__ double dl[];
-  const int b = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int t = find_item(ll.prefix, ll.nitems, b);
-  const DevLevel& L = Lt[ll.items[t]];
+  const Work wk = work_item(ln, lnb, li0, ll);
+  const DevLevel& D = Lt[wk.idx];
+  const double* dmat = D.dmat;
+  double* dscr = D.dscr;
+  pin_s(dmat, dscr);
+  const LevelHead L = level_head(D);
   if (level_off(L)) return;
   const int nx = L.nx, ny = L.ny, hx = L.hx, sx = nx + 1, sy = ny + 1;
   constexpr int sc = kDirectCols + 1;
-  const int ns = nx / kDirectCols, q = b - ll.prefix[t], k = q / ns, c0 = (q - k * ns) * kDirectCols;
+  const int ns = nx / kDirectCols, q = wk.lb, k = q / ns, c0 = (q - k * ns) * kDirectCols;
   const sp<kS, CT> X = (sp<kS, CT>)(sp<kS, double>)dl;   // the plane, ny x nx (stride sx)
   const sp<kS, CT> My = X + ny * sx;         // FWD: Vy^-1, else Vy (ny x ny, stride sy)
   const sp<kS, CT> Mx = My + ny * sy;        // columns c0.. of Vx^-T / Vx^T (nx x 16)
   const sp<kS, CT> Y = Mx + nx * sc;         // X Mx (ny x 16)
-  const auto m = gp(reinterpret_cast<const CT*>(L.dmat));
+  const auto m = gp(reinterpret_cast<const CT*>(dmat));
   const size_t ox = FWD ? 0 : (size_t)nx * nx;
   const size_t oy = (size_t)2 * nx * nx + (FWD ? 0 : (size_t)ny * ny);
   auto lmx = [&](int e) { return m[ox + (size_t)(e / kDirectCols) * nx + c0 + e % kDirectCols]; };
@@ -2810,7 +2848,7 @@ __global__ __launch_bounds__(kBlock) void k_direct_xy(const DevLevel* __restrict
     const int r = gm_div(e >> 1, L.gmhx, L.gshx);
     X[r * sx + e - r * nx] = v;
   };
-  const auto scr = gp(reinterpret_cast<CT*>(L.dscr));
+  const auto scr = gp(reinterpret_cast<CT*>(dscr));
   if constexpr (FWD) {
     const auto f = gfield<const T>((const void*)L.f);
     auto lf = [&](int e) {
@@ -2841,24 +2879,30 @@ __global__ __launch_bounds__(kBlock) void k_direct_xy(const DevLevel* __restrict
 // The z pass, one workgroup per slab of kDirectCols modes m0.. (all k):
 // x^ = Vz (inv .* (Vz^-1 f^)).
 template <class CT>
-__global__ __launch_bounds__(kBlock) void k_direct_z(const DevLevel* __restrict__ Lt, LaunchList ll) {
+__global__ __launch_bounds__(kBlock) void k_direct_z(const DevLevel* __restrict__ Lt, LIST_PARAMS,
+                                                      LaunchList ll) {
   extern __shared__ double dl[];
-  const int b = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int t = find_item(ll.prefix, ll.nitems, b);
-  const DevLevel& L = Lt[ll.items[t]];
+  const Work wk = work_item(ln, lnb, li0, ll);
+  const DevLevel& D = Lt[wk.idx];
+  const double *dmat = D.dmat, *dinv = D.dinv;
+  double* dscr = D.dscr;
+  unsigned gmzp = D.gmzp;
+  int gszp = D.gszp;
+  pin_s(dmat, dinv, dscr, gmzp, gszp);
+  const LevelHead L = level_head(D);
   if (level_off(L)) return;
   const int nx = L.nx, ny = L.ny, nz = L.nz, nzp = direct_nzp(nz);
-  const int plane = nx * ny, m0 = (b - ll.prefix[t]) * kDirectCols, sz = nzp + 1;
+  const int plane = nx * ny, m0 = wk.lb * kDirectCols, sz = nzp + 1;
   constexpr int sc = kDirectCols + 1;
   const sp<kS, CT> S = (sp<kS, CT>)(sp<kS, double>)dl;   // nzp x 16 (stride 17)
   const sp<kS, CT> Tm = S + nzp * sc;        // nzp x 16
   const sp<kS, CT> Wi = Tm + nzp * sc;       // Vz^-1 (nzp x nzp, stride sz)
   const sp<kS, CT> W = Wi + nzp * sz;        // Vz
-  const auto m = gp(reinterpret_cast<const CT*>(L.dmat));
+  const auto m = gp(reinterpret_cast<const CT*>(dmat));
   const size_t oz = (size_t)2 * nx * nx + (size_t)2 * ny * ny;
-  const auto fh = gp(reinterpret_cast<const CT*>(L.dscr));
-  const auto inv = gp(reinterpret_cast<const CT*>(L.dinv));
-  auto zrow = [&](int e) { return gm_div(e, L.gmzp, L.gszp); };   // e / nzp
+  const auto fh = gp(reinterpret_cast<const CT*>(dscr));
+  const auto inv = gp(reinterpret_cast<const CT*>(dinv));
+  auto zrow = [&](int e) { return gm_div(e, gmzp, gszp); };   // e / nzp
   stage3<16, CT>(
       nzp * nzp, [&](int e) { return m[oz + e]; }, [&](int e, CT v) { Wi[zrow(e) * sz + e - zrow(e) * nzp] = v; },
       nzp * nzp, [&](int e) { return m[oz + (size_t)nzp * nzp + e]; },
@@ -2873,7 +2917,7 @@ __global__ __launch_bounds__(kBlock) void k_direct_z(const DevLevel* __restrict_
     Tm[r * sc + c] = r < nz ? v * inv[(size_t)r * plane + m0 + c] : CT(0);
   });
   __syncthreads();
-  const auto xo = gp(reinterpret_cast<CT*>(L.dscr)) + (size_t)L.ncell;
+  const auto xo = gp(reinterpret_cast<CT*>(dscr)) + (size_t)L.ncell;
   mfma_products<CT>(W, sz, Tm, sc, nzp, kDirectCols, nzp, [&](int r, int c, CT v) {
     if (r < nz) xo[(size_t)r * plane + m0 + c] = v;
   });
@@ -2917,7 +2961,7 @@ static int device_cus() {
 
 void launch_rb_march(bool fp64, const DevLevel* L, const LaunchList& ll, int parity, int zero_guess,
                      int planes, hipStream_t s) {
-#define RM(T, K) LAUNCH((k_rb_march<T, K>), ll.nblocks, kBlock, L, ll, parity, zero_guess)
+#define RM(T, K) LAUNCH((k_rb_march<T, K>), ll.nblocks, kBlock, L, LIST_ARGS(ll), parity, zero_guess, ll)
   if (fp64) {
     if (planes == 8) RM(double, 8); else if (planes == 4) RM(double, 4); else RM(double, 2);
   } else {
@@ -2927,8 +2971,8 @@ void launch_rb_march(bool fp64, const DevLevel* L, const LaunchList& ll, int par
 }
 void launch_rb_point(bool fp64, const DevLevel* L, const LaunchList& ll, int parity, int zero_guess,
                      hipStream_t s) {
-  if (fp64) LAUNCH(k_rb_point<double>, ll.nblocks, kBlock, L, ll, parity, zero_guess);
-  else LAUNCH(k_rb_point<float>, ll.nblocks, kBlock, L, ll, parity, zero_guess);
+  if (fp64) LAUNCH(k_rb_point<double>, ll.nblocks, kBlock, L, LIST_ARGS(ll), parity, zero_guess, ll);
+  else LAUNCH(k_rb_point<float>, ll.nblocks, kBlock, L, LIST_ARGS(ll), parity, zero_guess, ll);
 }
 static void zline_variant(bool fp64, const DevLevel* L, const LaunchList& ll, int parity,
                           int zero_guess, int segs, hipStream_t s, int form, bool nbr, bool half) {
@@ -2938,8 +2982,8 @@ static void zline_variant(bool fp64, const DevLevel* L, const LaunchList& ll, in
   // reduced-system state (two buffers in FP32, one in FP64) + staged rows
   const size_t lds = (size_t)((fp64 ? 6 : 12) * cw + 3 * kZSeg) * ps * (fp64 ? 8 : 4);
 #define ZL(T, CH, NBR, LEAN, H)                                                                   \
-  hipLaunchKernelGGL((k_zline<T, kZSeg, CH, NBR, LEAN, H>), dim3(ll.nblocks), blk, lds, s, L, ll, \
-                     parity, zero_guess)
+  hipLaunchKernelGGL((k_zline<T, kZSeg, CH, NBR, LEAN, H>), dim3(ll.nblocks), blk, lds, s, L, \
+                     LIST_ARGS(ll), parity, zero_guess, ll)
   // FP64 always takes the lean form (the short one does not fit its
   // registers).  FP32 takes it when there are more blocks than CUs, so that
   // blocks can pair up; a smaller launch is latency-bound and takes the
@@ -3008,33 +3052,33 @@ void launch_zline_shared(const DevLevel* L, const LaunchList& ll, int parity, in
     hl.nblocks = 2 * ll.nblocks;
     const int wy = (segs + 1) / 2;
     const size_t lds = (size_t)2 * wy * (4 * 32 + kZRec) * sizeof(float);
-    hipLaunchKernelGGL(k_zline_shared<true>, dim3(hl.nblocks), dim3(64, wy), lds, s, L, parity,
-                       zero_guess, hl);
+    hipLaunchKernelGGL(k_zline_shared<true>, dim3(hl.nblocks), dim3(64, wy), lds, s, L, LIST_ARGS(hl),
+                       parity, zero_guess, hl);
     return;
   }
   const size_t lds = (size_t)4 * segs * 64 * sizeof(float);
-  hipLaunchKernelGGL(k_zline_shared<false>, dim3(ll.nblocks), dim3(64, segs), lds, s, L, parity,
-                     zero_guess, ll);
+  hipLaunchKernelGGL(k_zline_shared<false>, dim3(ll.nblocks), dim3(64, segs), lds, s, L, LIST_ARGS(ll),
+                     parity, zero_guess, ll);
 }
 void launch_zline_col(bool fp64, const DevLevel* L, const LaunchList& ll, int parity,
                       int zero_guess, hipStream_t s) {
-  if (fp64) LAUNCH(k_zline_col<double>, ll.nblocks, kBlock, L, ll, parity, zero_guess);
-  else LAUNCH(k_zline_col<float>, ll.nblocks, kBlock, L, ll, parity, zero_guess);
+  if (fp64) LAUNCH(k_zline_col<double>, ll.nblocks, kBlock, L, LIST_ARGS(ll), parity, zero_guess, ll);
+  else LAUNCH(k_zline_col<float>, ll.nblocks, kBlock, L, LIST_ARGS(ll), parity, zero_guess, ll);
 }
 void launch_restrict(bool fp64, const DevLevel* L, const DevXfer* X, const LaunchList& ll,
                      hipStream_t s) {
-  if (fp64) LAUNCH(k_restrict<double>, ll.nblocks, kBlock, L, X, ll);
-  else LAUNCH(k_restrict<float>, ll.nblocks, kBlock, L, X, ll);
+  if (fp64) LAUNCH(k_restrict<double>, ll.nblocks, kBlock, L, X, LIST_ARGS(ll), ll);
+  else LAUNCH(k_restrict<float>, ll.nblocks, kBlock, L, X, LIST_ARGS(ll), ll);
 }
 void launch_restrict222(bool fp64, const DevLevel* L, const DevXfer* X, const LaunchList& ll,
                         hipStream_t s, bool use_skip) {
-  if (fp64) LAUNCH(k_restrict222<double>, ll.nblocks, kBlock, L, X, ll, use_skip ? 1 : 0);
-  else LAUNCH(k_restrict222<float>, ll.nblocks, kBlock, L, X, ll, use_skip ? 1 : 0);
+  if (fp64) LAUNCH(k_restrict222<double>, ll.nblocks, kBlock, L, X, LIST_ARGS(ll), use_skip ? 1 : 0, ll);
+  else LAUNCH(k_restrict222<float>, ll.nblocks, kBlock, L, X, LIST_ARGS(ll), use_skip ? 1 : 0, ll);
 }
 void launch_prolong(bool fp64, const DevLevel* L, const DevXfer* X, const LaunchList& ll,
                     hipStream_t s, bool use_skip) {
-  if (fp64) LAUNCH(k_prolong<double>, ll.nblocks, kBlock, L, X, ll, use_skip ? 1 : 0);
-  else LAUNCH(k_prolong<float>, ll.nblocks, kBlock, L, X, ll, use_skip ? 1 : 0);
+  if (fp64) LAUNCH(k_prolong<double>, ll.nblocks, kBlock, L, X, LIST_ARGS(ll), use_skip ? 1 : 0, ll);
+  else LAUNCH(k_prolong<float>, ll.nblocks, kBlock, L, X, LIST_ARGS(ll), use_skip ? 1 : 0, ll);
 }
 size_t direct_lds_limit() {
   static size_t limit = 0;
@@ -3069,13 +3113,13 @@ void launch_direct(bool fp64, const DevLevel* L, const LaunchList& planes, const
                    size_t lds, hipStream_t s) {
   const dim3 blk(kBlock);
   if (fp64) {
-    hipLaunchKernelGGL((k_direct_xy<double, double, true>), dim3(planes.nblocks), blk, lds, s, L, planes);
-    hipLaunchKernelGGL(k_direct_z<double>, dim3(slabs.nblocks), blk, lds, s, L, slabs);
-    hipLaunchKernelGGL((k_direct_xy<double, double, false>), dim3(planes.nblocks), blk, lds, s, L, planes);
+    hipLaunchKernelGGL((k_direct_xy<double, double, true>), dim3(planes.nblocks), blk, lds, s, L, LIST_ARGS(planes), planes);
+    hipLaunchKernelGGL(k_direct_z<double>, dim3(slabs.nblocks), blk, lds, s, L, LIST_ARGS(slabs), slabs);
+    hipLaunchKernelGGL((k_direct_xy<double, double, false>), dim3(planes.nblocks), blk, lds, s, L, LIST_ARGS(planes), planes);
   } else {
-    hipLaunchKernelGGL((k_direct_xy<float, float, true>), dim3(planes.nblocks), blk, lds, s, L, planes);
-    hipLaunchKernelGGL(k_direct_z<float>, dim3(slabs.nblocks), blk, lds, s, L, slabs);
-    hipLaunchKernelGGL((k_direct_xy<float, float, false>), dim3(planes.nblocks), blk, lds, s, L, planes);
+    hipLaunchKernelGGL((k_direct_xy<float, float, true>), dim3(planes.nblocks), blk, lds, s, L, LIST_ARGS(planes), planes);
+    hipLaunchKernelGGL(k_direct_z<float>, dim3(slabs.nblocks), blk, lds, s, L, LIST_ARGS(slabs), slabs);
+    hipLaunchKernelGGL((k_direct_xy<float, float, false>), dim3(planes.nblocks), blk, lds, s, L, LIST_ARGS(planes), planes);
   }
 }
 void launch_coarse(bool fp64, const DevLevel* L, const LaunchList& ll, hipStream_t s) {
@@ -3153,13 +3197,14 @@ size_t tail_lds_limit() {
 }
 // (k_fine takes the table writable: the mixed first defect records bshift)
 void launch_residual_max(const DevLevel* L, const LaunchList& ll, double* partial, hipStream_t s) {
-  LAUNCH((k_fine<kResMax, false>), ll.nblocks, kBlock, const_cast<DevLevel*>(L), ll, nullptr, partial);
+  LAUNCH((k_fine<kResMax, false>), ll.nblocks, kBlock, const_cast<DevLevel*>(L), LIST_ARGS(ll), nullptr,
+         partial, ll);
 }
 void launch_first_defect(bool fp64, const DevLevel* L, const LaunchList& ll, const double* c,
                          double* partial, hipStream_t s) {
   DevLevel* W = const_cast<DevLevel*>(L);
-  if (fp64) LAUNCH((k_fine<kResMax, true>), ll.nblocks, kBlock, W, ll, c, partial);
-  else LAUNCH((k_fine<kDefect32, true>), ll.nblocks, kBlock, W, ll, c, partial);
+  if (fp64) LAUNCH((k_fine<kResMax, true>), ll.nblocks, kBlock, W, LIST_ARGS(ll), c, partial, ll);
+  else LAUNCH((k_fine<kDefect32, true>), ll.nblocks, kBlock, W, LIST_ARGS(ll), c, partial, ll);
 }
 void launch_ingest(const DevLevel* L, const LaunchList& ll, const PtrList& rhs, const PtrList& phi,
                    double* partial, hipStream_t s) {
@@ -3170,8 +3215,8 @@ void launch_change_max(const DevLevel* L, const LaunchList& ll, double* partial,
 }
 void launch_correct_defect32(const DevLevel* L, const LaunchList& ll, double* partial,
                              hipStream_t s) {
-  LAUNCH((k_fine<kCorrDefect32, false>), ll.nblocks, kBlock, const_cast<DevLevel*>(L), ll, nullptr,
-         partial);
+  LAUNCH((k_fine<kCorrDefect32, false>), ll.nblocks, kBlock, const_cast<DevLevel*>(L), LIST_ARGS(ll), nullptr,
+         partial, ll);
 }
 void launch_zero(double* a, int n, hipStream_t s) {
   LAUNCH(k_zero, nb((size_t)n), kBlock, a, n);
@@ -3188,7 +3233,7 @@ void launch_finalize(const LaunchList& ll, const double* partial, int nvals, int
                      int ostride, hipStream_t s, const GateArgs* gate) {
   GateArgs ga{};
   if (gate) ga = *gate;
-  LAUNCH(k_finalize, ll.nitems, kFinBlock, ll, partial, nvals, op_sum, out, ostride, ga);
+  LAUNCH(k_finalize, ll.nitems, kFinBlock, LIST_ARGS(ll), nvals, op_sum, partial, out, ostride, ga, ll);
 }
 void launch_from_fortran(const DevLevel* L, const LaunchList& ll, const PtrList& ptr, int which,
                          int add_fold, hipStream_t s) {

@@ -373,7 +373,6 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
     // fields of the V-cycle precision
     d.u = I->mem.alloc((size_t)d.ncell * w);
     d.f = I->mem.alloc((size_t)d.ncell * w);
-    d.scr = nullptr;
     if (!d.u || !d.f) return fail();
   }
   // FP64 finest entries
@@ -387,8 +386,8 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
     void* pB = I->mem.alloc((size_t)fA.ncell * 8);
     void* b = I->mem.alloc((size_t)fA.ncell * 8);
     if (!pA || !pB || !b) return fail();
-    fA.u = pA; fA.u2 = pB; fA.f = b; fA.scr = nullptr;
-    fB.u = pB; fB.u2 = pA; fB.f = b; fB.scr = nullptr;
+    fA.u = pA; fA.u2 = pB; fA.f = b;
+    fB.u = pB; fB.u2 = pA; fB.f = b;
   }
   // descriptor indices: this instance's entries follow the context's
   const int base = (int)hL.size(), xbase = (int)hX.size();
@@ -402,6 +401,8 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
     I->fine[0] = I->fine[1] = I->lev[0];
   } else {
     fA.link = fB.link = I->lev[0];
+    fA.e32 = fB.e32 = (const float*)ents[0].u;
+    fA.r32 = fB.r32 = (float*)ents[0].f;
     I->fine[0] = base + (int)newL.size();
     newL.push_back(fA);
     I->fine[1] = base + (int)newL.size();
@@ -872,7 +873,7 @@ int Context::cycle_and_norms(const std::vector<Instance*>& S) {
   // per-instance gates: item t of a list at offset ioff
   auto each_args = [&](int ioff) {
     return GateArgs{d_out + (size_t)ioff * nv, d_out + kOutRegion * 2 + (size_t)ioff * 2, dL,
-                    (int)hL.size(), d_igate};
+                    (int)hL.size(), d_igate, S[ioff]->gslot, S[ioff]->id};
   };
   for_lists(items, [&](const LaunchList& ll, int ioff, int boff) {
     double* part = d_partial + (size_t)boff * nv;
