@@ -198,6 +198,20 @@ constexpr size_t kTailMinvLds = 16384;   // largest coarsest inverse staged in L
 // phases around it (one workgroup reading the whole inverse is bound by its
 // memory latency, about 65 GB/s).
 constexpr int kSplitCells = 256;
+// A level of the line tail: word offsets of its u and f and of its LDS
+// tables, and that of its eliminated column matrix in the tail's tables.
+struct LineLevel {
+  int nx, ny, nz, hx, st;         // st: words between columns (tail_stride)
+  int px, py;
+  unsigned gmhx;                  // division by hx (gm_magic)
+  int gshx, u, f, xy, z, col;
+  int bc[6];                      // boundary codes of x, y, z (prolongation ghosts)
+};
+// Steps of the line tail: a whole smoothing phase (sweeps from zero or from
+// the iterate), a transfer, or the coarse solve.
+constexpr int line_step(int type, int level, int sweeps, bool from_zero) {
+  return type | (level << 3) | ((from_zero ? 1 : 0) << 7) | (sweeps << 8);
+}
 struct DevTail {
   int nlev;                       // tail levels, the last is the coarsest
   int copy_u_in;                  // the first tail level's u is read (not zero)
@@ -214,7 +228,28 @@ struct DevTail {
   int lds_minv;                   // the coarsest inverse staged in LDS (level precision), or -1
   int lev[kTailMaxLevels];        // DevLevel index per tail level
   int xf[kTailMaxLevels];         // DevXfer index of tail level d -> d+1
+  // the line tail (k_tail_line), when the instance's tail can take it: its
+  // tables in global memory (tab; the first tab_words words are copied to the
+  // start of the LDS), its levels and its steps
+  const float* tab;
+  int tab_words;
+  int lin_m, lin_c;               // word offsets of the coarse solve's tables and workspace (doubles)
+  int lin_nsteps;
+  int lin_steps[4 * kTailMaxLevels];   // line_step
+  LineLevel lin[kTailMaxLevels];
 };
+// Line-tail layout: a level's fields are stored column by column, its nz rows
+// padded to a multiple of 4 (tail_rows) and the columns tail_stride words
+// apart, an odd multiple of 4: a lane reads four rows of a column at once and
+// eight neighbouring lanes' reads fall into different LDS banks.
+__host__ __device__ inline int tail_rows(int nz) { return (nz + 3) & ~3; }
+__host__ __device__ inline int tail_stride(int nz) {
+  const int r = tail_rows(nz);
+  return (r & 4) ? r : r + 4;
+}
+constexpr int kLineWaves = 16;    // waves of the line tail's workgroup
+void launch_tail_line(const DevLevel* L, const DevTail* T, const LaunchList& ll, size_t lds_bytes,
+                      hipStream_t s);
 
 void launch_fill_zero(bool fp64, const DevLevel* L, const LaunchList& ll, hipStream_t s);
 

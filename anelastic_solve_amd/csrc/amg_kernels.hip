@@ -1747,6 +1747,317 @@ __global__ __launch_bounds__(NZ == 0 ? 64 * kTailWavesPoint : 64 * kTailWaves) v
   for (int e = tid; e < G0.ncell; e += nthr) gu[e] = lu[e];
 }
 
+// ---------------------------------------------------------------------------
+// The coarse tail of an FP32 z-line V-cycle whose levels' columns share one
+// matrix (DevLevel::zt), with walls in z, 2:2:2 transfers and smoothing on
+// both ways on every level: the same sub-V-cycle as k_tail's, in one
+// workgroup, but with the fields in LDS column by column (tail_stride), so
+// that every step reads and writes four rows at a time:
+//  - a half-sweep is one column per lane with the column's eliminated matrix
+//    in scalar registers: no reciprocal, two dependent operations per row down
+//    and one up (k_tail: a reciprocal per row and 130 four-byte LDS reads);
+//  - the restriction forms the residuals of the colour-0 cells only, the
+//    others being solved by the pre-smoothing (as k_restrict222), a task being
+//    two coarse cells of a column;
+//  - the prolongation corrects the colour-1 cells only, the others being
+//    rewritten by the post-smoothing (as k_prolong), a task being eight rows
+//    of a column;
+//  - the coarsest level is solved by eigenvector transforms held in LDS.
+// Bound by the steps' LDS and dependent latencies (one CU).  32x24x16 and
+// below: 27 us against k_tail's 53; 24x24x24 and below: 32 against 45;
+// 20x14x10 and 10x7x5: 17 against 44 (k_tail split around the dense product).
+template <class T> using cst = const __attribute__((address_space(4))) T*;
+template <class T> __device__ __forceinline__ cst<T> cp4(const T* p) { return (cst<T>)p; }
+
+__device__ __forceinline__ float4& lds4(float* p) { return *reinterpret_cast<float4*>(p); }
+
+// A smoothing phase, columns of 4*NC rows (rows past nz have zero table rows).
+template <int NC>
+__device__ __forceinline__ void line_smooth(float* __restrict__ lds, const LineLevel& L, cst<float> tabs,
+                                            int sweeps, bool zero_first, int tid) {
+  const int ncol = L.hx * L.ny, st = L.st, hx = L.hx;
+  const cst<float> tab = tabs + L.col;
+  for (int half = 0; half < 2 * sweeps; ++half) {
+    const int parity = half & 1;
+    const bool from_zero = zero_first && half == 0;
+    if (half > 0) __syncthreads();
+    for (int col = tid; col < ncol; col += 64 * kLineWaves) {
+      const int j = gm_div(col, L.gmhx, L.gshx), m = col - j * hx;
+      const int oth = parity ^ 1, r = (parity + j) & 1, i = 2 * m + r;
+      float* const own = lds + L.u + ((j * 2 + parity) * hx + m) * st;
+      const float* const fo = lds + L.f + ((j * 2 + parity) * hx + m) * st;
+      float g[4 * NC];
+#pragma unroll
+      for (int q = 0; q < NC; ++q) {
+        const float4 v = *reinterpret_cast<const float4*>(fo + 4 * q);
+        g[4 * q] = v.x; g[4 * q + 1] = v.y; g[4 * q + 2] = v.z; g[4 * q + 3] = v.w;
+      }
+      if (!from_zero) {
+        int ml = m - 1 + r; if (ml < 0) ml = hx - 1;
+        int mr = m + r;     if (mr >= hx) mr = 0;
+        const int jm = (j == 0) ? L.ny - 1 : j - 1, jp = (j == L.ny - 1) ? 0 : j + 1;
+        const float* const t = lds + L.xy;
+        const float wxl = t[i], wxr = t[L.nx + i], wys = t[2 * L.nx + j], wyn = t[2 * L.nx + L.ny + j];
+        const float* const ub = lds + L.u;
+        const float* const xl = ub + ((j * 2 + oth) * hx + ml) * st;
+        const float* const xr = ub + ((j * 2 + oth) * hx + mr) * st;
+        const float* const ys = ub + ((jm * 2 + oth) * hx + m) * st;
+        const float* const yn = ub + ((jp * 2 + oth) * hx + m) * st;
+#pragma unroll
+        for (int q = 0; q < NC; ++q) {
+          const float4 a = *reinterpret_cast<const float4*>(xl + 4 * q);
+          const float4 b = *reinterpret_cast<const float4*>(xr + 4 * q);
+          const float4 c = *reinterpret_cast<const float4*>(ys + 4 * q);
+          const float4 d = *reinterpret_cast<const float4*>(yn + 4 * q);
+          g[4 * q] -= zline_nbr(wxl, wxr, wys, wyn, a.x, b.x, c.x, d.x);
+          g[4 * q + 1] -= zline_nbr(wxl, wxr, wys, wyn, a.y, b.y, c.y, d.y);
+          g[4 * q + 2] -= zline_nbr(wxl, wxr, wys, wyn, a.z, b.z, c.z, d.z);
+          g[4 * q + 3] -= zline_nbr(wxl, wxr, wys, wyn, a.w, b.w, c.w, d.w);
+        }
+      }
+      float y = 0.0f;
+#pragma unroll
+      for (int q = 0; q < 4 * NC; ++q) {
+        y = fm(-tab[q], y, g[q]) * tab[kTailNz + q];
+        g[q] = y;
+      }
+      float x = 0.0f;
+#pragma unroll
+      for (int q = 4 * NC - 1; q >= 0; --q) {
+        x = fm(-tab[2 * kTailNz + q], x, g[q]);
+        g[q] = x;
+      }
+#pragma unroll
+      for (int q = 0; q < NC; ++q)
+        lds4(own + 4 * q) = make_float4(g[4 * q], g[4 * q + 1], g[4 * q + 2], g[4 * q + 3]);
+    }
+  }
+}
+
+// Residuals of the colour-0 cells, weighted into the coarse right-hand side.
+// Each 1-D weight is a cell's share of its coarse cell's width.
+__device__ __forceinline__ void line_restrict(float* __restrict__ lds, const LineLevel& F,
+                                              const LineLevel& C, int tid) {
+  const int ncc = C.nx * C.ny, kp = (C.nz + 1) >> 1, st = F.st, hx = F.hx;
+  const float* const t = lds + F.xy;
+  const float* const wnx = t + 2 * F.nx + 2 * F.ny;
+  const float* const wny = wnx + F.nx;
+  const float* const zt = lds + F.z;
+  const int nzp = tail_rows(F.nz);
+  for (int e = tid; e < ncc * kp; e += 64 * kLineWaves) {
+    const int q0 = e / ncc, cc = e - q0 * ncc, J = gm_div(cc >> 1, C.gmhx, C.gshx), I = cc - J * C.nx;
+    const int k0 = 4 * q0;
+    const float4 za = *reinterpret_cast<const float4*>(zt + k0);
+    const float4 ze = *reinterpret_cast<const float4*>(zt + nzp + k0);
+    const float4 zd = *reinterpret_cast<const float4*>(zt + 2 * nzp + k0);
+    const float4 zw = *reinterpret_cast<const float4*>(zt + 3 * nzp + k0);
+    float lo = 0.0f, hi = 0.0f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {                 // fine columns (2I, 2J) and (2I+1, 2J+1)
+      const int i = 2 * I + h, j = 2 * J + h;
+      const int jm = (j == 0) ? F.ny - 1 : j - 1, jp = (j == F.ny - 1) ? 0 : j + 1;
+      const int ml = h ? I : (I == 0 ? hx - 1 : I - 1), mr = h ? (I + 1 == hx ? 0 : I + 1) : I;
+      const float* const ub = lds + F.u;
+      const int own = (j * 2 * hx + I) * st + k0;
+      const float4 c4 = *reinterpret_cast<const float4*>(ub + own);
+      const float um = ub[own - (k0 > 0 ? 1 : 0)], up = ub[own + (k0 + 4 < nzp ? 4 : 3)];
+      const float4 f4 = *reinterpret_cast<const float4*>(lds + F.f + own);
+      const float4 a = *reinterpret_cast<const float4*>(ub + ((j * 2 + 1) * hx + ml) * st + k0);
+      const float4 b = *reinterpret_cast<const float4*>(ub + ((j * 2 + 1) * hx + mr) * st + k0);
+      const float4 c = *reinterpret_cast<const float4*>(ub + ((jm * 2 + 1) * hx + I) * st + k0);
+      const float4 d = *reinterpret_cast<const float4*>(ub + ((jp * 2 + 1) * hx + I) * st + k0);
+      const float wxl = t[i], wxr = t[F.nx + i], wys = t[2 * F.nx + j], wyn = t[2 * F.nx + F.ny + j];
+      auto res = [&](float fv, float xl, float xr, float ys, float yn, float dn, float upv, float cc0,
+                     float A, float E, float D) {
+        return fv - fm(D, cc0, fm(E, upv, fm(A, dn, zline_nbr(wxl, wxr, wys, wyn, xl, xr, ys, yn))));
+      };
+      const float r0 = res(f4.x, a.x, b.x, c.x, d.x, um, c4.y, c4.x, za.x, ze.x, zd.x);
+      const float r1 = res(f4.y, a.y, b.y, c.y, d.y, c4.x, c4.z, c4.y, za.y, ze.y, zd.y);
+      const float r2 = res(f4.z, a.z, b.z, c.z, d.z, c4.y, c4.w, c4.z, za.z, ze.z, zd.z);
+      const float r3 = res(f4.w, a.w, b.w, c.w, d.w, c4.z, up, c4.w, za.w, ze.w, zd.w);
+      const float wxy = wnx[i] * wny[j];
+      lo = fm(wxy, fm(zw.y, r1, zw.x * r0), lo);
+      hi = fm(wxy, fm(zw.w, r3, zw.z * r2), hi);
+    }
+    float* const fc = lds + C.f + ((J * 2 + ((I + J) & 1)) * C.hx + (I >> 1)) * C.st + 2 * q0;
+    *reinterpret_cast<float2*>(fc) = make_float2(lo, hi);
+  }
+}
+
+// Trilinear prolongation-add to the colour-1 cells (at a Dirichlet wall the
+// correction vanishes at the ghost, at a Neumann wall it is copied).
+__device__ __forceinline__ void line_prolong(float* __restrict__ lds, const LineLevel& F,
+                                             const LineLevel& C, int tid) {
+  const int bx0 = F.bc[0], bx1 = F.bc[1], by0 = F.bc[2], by1 = F.bc[3], bz0 = F.bc[4], bz1 = F.bc[5];
+  const int ncol = F.hx * F.ny, nch = (C.nz + 3) >> 2, hx = F.hx, nzc = C.nz;
+  for (int e = tid; e < ncol * nch; e += 64 * kLineWaves) {
+    const int ch = e / ncol, col = e - ch * ncol;
+    const int j = gm_div(col, F.gmhx, F.gshx), m = col - j * hx;
+    const int r = (1 + j) & 1, I = m, J = j >> 1, K0 = 4 * ch;
+    int I2 = r ? I + 1 : I - 1, J2 = (j & 1) ? J + 1 : J - 1;
+    float fx = 1.0f, fy = 1.0f;
+    if (I2 < 0) { if (F.px) I2 = C.nx - 1; else { I2 = 0; if (bx0 == 2) fx = 0.0f; } }
+    if (I2 >= C.nx) { if (F.px) I2 = 0; else { I2 = C.nx - 1; if (bx1 == 2) fx = 0.0f; } }
+    if (J2 < 0) { if (F.py) J2 = C.ny - 1; else { J2 = 0; if (by0 == 2) fy = 0.0f; } }
+    if (J2 >= C.ny) { if (F.py) J2 = 0; else { J2 = C.ny - 1; if (by1 == 2) fy = 0.0f; } }
+    const float* const ub = lds + C.u;
+    auto at = [&](int a, int b) { return ub + ((b * 2 + ((a + b) & 1)) * C.hx + (a >> 1)) * C.st; };
+    const float* const c0 = at(I, J);
+    const float* const c1 = at(I2, J);
+    const float* const c2 = at(I, J2);
+    const float* const c3 = at(I2, J2);
+    const float w0 = 0.5625f, w1 = 0.1875f * fx, w2 = 0.1875f * fy, w3 = 0.0625f * fx * fy;
+    auto mix = [&](float a, float b, float c, float d) { return fm(w3, d, fm(w2, c, fm(w1, b, w0 * a))); };
+    // coarse rows K0-1 .. K0+4
+    float t[6];
+    const int kb = max(K0 - 1, 0), ka = min(K0 + 4, nzc - 1);
+    const float4 a4 = *reinterpret_cast<const float4*>(c0 + K0), b4 = *reinterpret_cast<const float4*>(c1 + K0);
+    const float4 d4 = *reinterpret_cast<const float4*>(c2 + K0), e4 = *reinterpret_cast<const float4*>(c3 + K0);
+    t[0] = mix(c0[kb], c1[kb], c2[kb], c3[kb]);
+    t[1] = mix(a4.x, b4.x, d4.x, e4.x);
+    t[2] = mix(a4.y, b4.y, d4.y, e4.y);
+    t[3] = mix(a4.z, b4.z, d4.z, e4.z);
+    t[4] = mix(a4.w, b4.w, d4.w, e4.w);
+    t[5] = mix(c0[ka], c1[ka], c2[ka], c3[ka]);
+    if (K0 == 0) t[0] = bz0 == 2 ? 0.0f : t[1];
+#pragma unroll
+    for (int q = 2; q < 6; ++q)
+      if (K0 - 1 + q >= nzc) t[q] = bz1 == 2 ? 0.0f : t[q - 1];
+    float* const uo = lds + F.u + ((j * 2 + 1) * hx + m) * F.st + 8 * ch;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {                  // fine rows 8ch + 4h ..: coarse rows K0+2h, +1
+      if (K0 + 2 * h >= nzc) break;
+      float4 v = lds4(uo + 4 * h);
+      v.x += fm(0.75f, t[1 + 2 * h], 0.25f * t[2 * h]);
+      v.y += fm(0.75f, t[1 + 2 * h], 0.25f * t[2 + 2 * h]);
+      v.z += fm(0.75f, t[2 + 2 * h], 0.25f * t[1 + 2 * h]);
+      v.w += fm(0.75f, t[2 + 2 * h], 0.25f * t[3 + 2 * h]);
+      lds4(uo + 4 * h) = v;
+    }
+  }
+}
+
+// Separable solve of the coarsest level (direct_setup's tables in LDS, FP64):
+// transforms in x, y and z, the inverse eigenvalue sums, and back, one value
+// per lane and stage.  (Multiplying by the dense inverse took 5 us at 192
+// cells and 14 at 350: one CU reads it at its L2 rate.)
+__device__ __forceinline__ void line_coarse(float* __restrict__ lds, const LineLevel& L, int m0, int w0,
+                                            int tid) {
+  const int nx = L.nx, ny = L.ny, nz = L.nz, nxy = nx * ny, n = nxy * nz;
+  const double* const xi = reinterpret_cast<const double*>(lds + m0);
+  const double *const xv = xi + nx * nx, *const yi = xv + nx * nx, *const yv = yi + ny * ny;
+  const double *const zi = yv + ny * ny, *const zv = zi + nz * nz, *const inv = zv + nz * nz;
+  double* const A = reinterpret_cast<double*>(lds + w0);
+  double* const B = A + n;
+  const bool on = tid < n;
+  const int k = tid / nxy, q = tid - k * nxy, j = q / nx, i = q - j * nx;
+  const int col = ((j * 2 + ((i + j) & 1)) * L.hx + (i >> 1)) * L.st + k;
+  // sum over c < len of a[c * sa] * b[c * sb]
+  auto dot = [](const double* a, int sa, const double* b, int sb, int len) {
+    double s = 0.0;
+#pragma unroll 4
+    for (int c = 0; c < len; ++c) s = fm(a[c * sa], b[c * sb], s);
+    return s;
+  };
+  if (on) A[tid] = (double)lds[L.f + col];
+  __syncthreads();
+  if (on) B[tid] = dot(A + tid - i, 1, xi + i, nx, nx);
+  __syncthreads();
+  if (on) A[tid] = dot(yi + j * ny, 1, B + k * nxy + i, nx, ny);
+  __syncthreads();
+  if (on) B[tid] = dot(zi + k * nz, 1, A + q, nxy, nz) * inv[tid];
+  __syncthreads();
+  if (on) A[tid] = dot(zv + k * nz, 1, B + q, nxy, nz);
+  __syncthreads();
+  if (on) B[tid] = dot(yv + j * ny, 1, A + k * nxy + i, nx, ny);
+  __syncthreads();
+  if (on) lds[L.u + col] = (float)dot(B + tid - i, 1, xv + i, nx, nx);
+}
+
+__global__ __launch_bounds__(64 * kLineWaves) void k_tail_line(const DevLevel* __restrict__ Lt,
+                                                                const DevTail* __restrict__ Tt, LIST_PARAMS,
+                                                                LaunchList ll) {
+  extern __shared__ float lds[];
+  const int tid = threadIdx.x;
+  constexpr int nthr = 64 * kLineWaves;
+  const cst<DevTail> tl = cp4(Tt + (ln == 1 ? li0 : ll.items[blockIdx.x]));
+  const int nst = tl->lin_nsteps, words = tl->tab_words;
+  const float* tabg = tl->tab;
+  const LevelHead H0 = level_head(Lt[tl->lev[0]]);
+  if (H0.stop) return;
+  auto level = [&](int d) {
+    const auto* l = &tl->lin[d];
+    return LineLevel{l->nx, l->ny, l->nz, l->hx, l->st, l->px, l->py, l->gmhx, l->gshx, l->u, l->f, l->xy,
+                     l->z, l->col, {l->bc[0], l->bc[1], l->bc[2], l->bc[3], l->bc[4], l->bc[5]}};
+  };
+  // the first level's right-hand side on its way while the LDS is cleared (the
+  // rows past nz have to be finite) and the tables are copied
+  constexpr int U = 16;
+  const int plane = H0.nx * H0.ny, n0 = H0.ncell;
+  const sp<kG, const float> f0 = gfield<const float>((const void*)H0.f);
+  float fv[U];
+#pragma unroll
+  for (int q = 0; q < U; ++q) fv[q] = f0[min(tid + q * nthr, n0 - 1)];
+  const int end = tl->lin_c;
+  for (int e = words + 4 * tid; e < end; e += 4 * nthr) lds4(lds + e) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (int e = tid; e < words; e += nthr) lds[e] = gp(tabg)[e];
+  __syncthreads();
+  const LineLevel L0 = level(0);
+  {
+    const int dk = nthr / plane, dc = nthr - dk * plane;
+    int k = tid / plane, c = tid - k * plane;
+    for (int e0 = tid; e0 < n0; e0 += U * nthr) {
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        if (e0 + q * nthr < n0) lds[L0.f + c * L0.st + k] = fv[q];
+        c += dc;
+        k += dk;
+        if (c >= plane) { c -= plane; ++k; }
+      }
+      if (e0 + U * nthr < n0) {
+#pragma unroll
+        for (int q = 0; q < U; ++q) fv[q] = f0[min(e0 + (U + q) * nthr, n0 - 1)];
+      }
+    }
+  }
+  __syncthreads();
+  int code = tl->lin_steps[0];
+  for (int st = 0; st < nst; ++st) {
+    const int type = code & 7, d = (code >> 3) & 15, zf = (code >> 7) & 1, sweeps = code >> 8;
+    code = tl->lin_steps[st + 1];                 // (one past the last is allocated)
+    const LineLevel L = level(d);
+    if (type == kStepHalf) {
+      const cst<float> tabs = cp4(tabg);
+      switch (tail_rows(L.nz) >> 2) {
+        case 1: line_smooth<1>(lds, L, tabs, sweeps, zf, tid); break;
+        case 2: line_smooth<2>(lds, L, tabs, sweeps, zf, tid); break;
+        case 3: line_smooth<3>(lds, L, tabs, sweeps, zf, tid); break;
+        case 4: line_smooth<4>(lds, L, tabs, sweeps, zf, tid); break;
+        case 5: line_smooth<5>(lds, L, tabs, sweeps, zf, tid); break;
+        case 6: line_smooth<6>(lds, L, tabs, sweeps, zf, tid); break;
+        case 7: line_smooth<7>(lds, L, tabs, sweeps, zf, tid); break;
+        default: line_smooth<8>(lds, L, tabs, sweeps, zf, tid); break;
+      }
+    } else if (type == kStepRestrict) {
+      line_restrict(lds, L, level(d + 1), tid);
+    } else if (type == kStepProlong) {
+      line_prolong(lds, L, level(d + 1), tid);
+    } else {
+      line_coarse(lds, L, tl->lin_m, end, tid);
+    }
+    __syncthreads();
+  }
+  const sp<kG, float> u0 = gfield<float>(H0.u);
+  const int dk = nthr / plane, dc = nthr - dk * plane;
+  int k = tid / plane, c = tid - k * plane;
+  for (int e = tid; e < n0; e += nthr) {
+    u0[e] = lds[L0.u + c * L0.st + k];
+    c += dc;
+    k += dk;
+    if (c >= plane) { c -= plane; ++k; }
+  }
+}
+
 // Coarsest level of a split tail: u = M f with the row-major (pseudo-)inverse,
 // one wave per row (FP64 partial sums over the lane's columns in a fixed
 // order, then a fixed butterfly), so a large inverse is read by the whole
@@ -3154,6 +3465,12 @@ void launch_tail(bool fp64, int nz_class, bool all222, const DevLevel* L, const 
 #undef GO
 }
 
+void launch_tail_line(const DevLevel* L, const DevTail* T, const LaunchList& ll, size_t lds_bytes,
+                      hipStream_t s) {
+  hipLaunchKernelGGL(k_tail_line, dim3(ll.nitems), dim3(64 * kLineWaves), lds_bytes, s, L, T,
+                     LIST_ARGS(ll), ll);
+}
+
 void launch_coarse_wide(bool fp64, const DevLevel* L, const LaunchList& ll, hipStream_t s) {
   if (fp64) LAUNCH(k_coarse_wide<double>, ll.nblocks, kBlock, L, ll);
   else LAUNCH(k_coarse_wide<float>, ll.nblocks, kBlock, L, ll);
@@ -3171,6 +3488,7 @@ size_t tail_lds_limit() {
   // room for the static descriptor array of the kernel
   lim -= sizeof(DevLevel) * kTailMaxLevels + 256;
   const void* kernels[] = {
+      reinterpret_cast<const void*>(&k_tail_line),
       reinterpret_cast<const void*>(&k_tail<double, 0, true>),
       reinterpret_cast<const void*>(&k_tail<double, 0, false>),
       reinterpret_cast<const void*>(&k_tail<float, 0, true>),

@@ -526,6 +526,8 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
     I->tail_split = tl.lds_minv < 0 && (int)nco >= kSplitCells;
     I->tail = (int)hT.size();
     I->tail_lds = off;
+    const int rc = plan_line_tail(I, ents, newX, tl);
+    if (rc != AMG_OK) return rc;
   }
   // separable direct solve of the first level below the finest, above the
   // coarse tail (the tail solves small levels in one launch), that the
@@ -603,6 +605,120 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
     return rc2;
   }
   *out = I;
+  return AMG_OK;
+}
+
+int Context::plan_line_tail(Instance* I, const std::vector<DevLevel>& ents,
+                            const std::vector<DevXfer>& xf, DevTail& tl) {
+  tl.tab = nullptr;
+  const int nl = tl.nlev, l0 = I->l0;
+  if (I->fp64 || cfg.smoother != AMG_SMOOTHER_LJ || nl < 2 || I->H.bc[2][0] == AMG_BC_PERIODIC ||
+      I->H.lv.back().ncell() > 64 * kLineWaves)
+    return AMG_OK;
+  for (int d = 0; d + 1 < nl; ++d) {
+    const DevXfer& x = xf[l0 + d];
+    if (!ents[l0 + d].zt || x.fx != 2 || x.fy != 2 || x.fz != 2 || I->pre[l0 + d] < 1 ||
+        I->post[l0 + d] < 1)
+      return AMG_OK;
+  }
+  const HostLevel& HC = I->H.lv.back();
+  DirectTables D;
+  std::string derr;
+  if (!direct_setup(HC, I->H.bc, I->H.singular, &D, &derr)) return AMG_OK;
+  // the LDS tables of every level and of the coarse solve, then the eliminated
+  // column matrices
+  std::vector<float> tab;
+  auto pad4 = [&] { tab.resize((tab.size() + 3) & ~(size_t)3, 0.0f); };
+  for (int d = 0; d + 1 < nl; ++d) {
+    const HostLevel& H = I->H.lv[l0 + d];
+    const int nx = H.nx, ny = H.ny, nz = H.nz, nzp = tail_rows(nz);
+    const double *cx = H.co.data(), *cy = cx + 3 * nx, *cz = cy + 3 * ny;
+    const double *vx = H.vol.data(), *vy = vx + nx, *vz = vy + ny;
+    auto share = [](const double* v, int i) { return (float)(v[i] / (v[i & ~1] + v[i | 1])); };
+    tl.lin[d].xy = (int)tab.size();
+    tab.insert(tab.end(), cx, cx + 2 * nx);
+    tab.insert(tab.end(), cy, cy + 2 * ny);
+    for (int i = 0; i < nx; ++i) tab.push_back(share(vx, i));
+    for (int j = 0; j < ny; ++j) tab.push_back(share(vy, j));
+    pad4();
+    tl.lin[d].z = (int)tab.size();
+    for (int t = 0; t < 4; ++t)
+      for (int k = 0; k < nzp; ++k)
+        tab.push_back(k >= nz ? 0.0f : t == 3 ? share(vz, k)
+                      : (float)(cz[t * nz + k] + (t == 2 ? cx[2 * nx] + cy[2 * ny] : 0.0)));
+  }
+  {
+    // direct_setup's tables with the z matrices unpadded, as doubles
+    pad4();
+    tl.lin_m = (int)tab.size();
+    const size_t nxy2 = 2 * ((size_t)HC.nx * HC.nx + (size_t)HC.ny * HC.ny), nzp = (size_t)D.nzp;
+    std::vector<double> m(D.mats.begin(), D.mats.begin() + nxy2);
+    for (size_t t = 0; t < 2; ++t)
+      for (int r = 0; r < HC.nz; ++r) {
+        const auto row = D.mats.begin() + nxy2 + t * nzp * nzp + r * nzp;
+        m.insert(m.end(), row, row + HC.nz);
+      }
+    m.insert(m.end(), D.inv.begin(), D.inv.end());
+    tab.resize(tab.size() + 2 * m.size());
+    std::memcpy(tab.data() + tl.lin_m, m.data(), 8 * m.size());
+  }
+  pad4();
+  tl.tab_words = (int)tab.size();
+  for (int d = 0; d + 1 < nl; ++d) {
+    const HostLevel& H = I->H.lv[l0 + d];
+    const int nz = H.nz;
+    const double *cx = H.co.data(), *cy = cx + 3 * H.nx, *cz = cy + 3 * H.ny;
+    const double dxy = cx[2 * H.nx] + cy[2 * H.ny];
+    tl.lin[d].col = (int)tab.size();
+    tab.resize(tab.size() + 3 * kTailNz, 0.0f);
+    float* t = tab.data() + tl.lin[d].col;
+    double cp = 0.0;
+    for (int k = 0; k < nz; ++k) {
+      const double a = k == 0 ? 0.0 : cz[k], rd = 1.0 / (cz[2 * nz + k] + dxy - a * cp);
+      cp = k == nz - 1 ? 0.0 : cz[nz + k] * rd;
+      t[k] = (float)a;
+      t[kTailNz + k] = (float)rd;
+      t[2 * kTailNz + k] = (float)cp;
+    }
+  }
+  size_t off = (size_t)tl.tab_words;
+  for (int d = 0; d < nl; ++d) {
+    const HostLevel& H = I->H.lv[l0 + d];
+    const size_t n = (size_t)H.nx * H.ny * tail_stride(H.nz);
+    const DevLevel& e = ents[l0 + d];
+    LineLevel& l = tl.lin[d];
+    l.nx = e.nx; l.ny = e.ny; l.nz = e.nz; l.hx = e.hx;
+    l.st = tail_stride(e.nz);
+    l.px = e.px; l.py = e.py;
+    l.gmhx = e.gmhx; l.gshx = e.gshx;
+    l.u = (int)off;
+    l.f = (int)(off + n);
+    for (int q = 0; q < 6; ++q) l.bc[q] = I->H.bc[q >> 1][q & 1];
+    off += 2 * n;
+  }
+  // the sub-V-cycle, in the order of mgMK/mg_cycle.F90
+  int ns = 0;
+  for (int d = 0; d + 1 < nl; ++d) {
+    tl.lin_steps[ns++] = line_step(kStepHalf, d, I->pre[l0 + d], true);
+    tl.lin_steps[ns++] = line_step(kStepRestrict, d, 0, false);
+  }
+  tl.lin_steps[ns++] = line_step(kStepCoarse, nl - 1, 0, false);
+  for (int d = nl - 2; d >= 0; --d) {
+    tl.lin_steps[ns++] = line_step(kStepProlong, d, 0, false);
+    tl.lin_steps[ns++] = line_step(kStepHalf, d, I->post[l0 + d], false);
+  }
+  tl.lin_nsteps = ns;
+  tl.lin_c = (int)off;
+  const size_t bytes = off * 4 + 16 * (size_t)HC.ncell();
+  if (bytes > tail_lds_limit()) return AMG_OK;
+  float* dt = (float*)I->mem.alloc(tab.size() * 4);
+  if (!dt) {
+    set_error("device allocation failed");
+    return AMG_ENOMEM;
+  }
+  AMG_HIP(hipMemcpy(dt, tab.data(), tab.size() * 4, hipMemcpyHostToDevice));
+  tl.tab = dt;
+  I->tail_line = bytes;
   return AMG_OK;
 }
 
@@ -782,13 +898,23 @@ void Context::vcycle(const std::vector<Instance*>& S, bool fp64) {
   }
   // the coarse tails, one launch per kernel variant; a split tail runs down,
   // then the coarse solve across the device, then up
+  {
+    std::vector<Item> items;
+    size_t lds = 0;
+    for (Instance* I : S) {
+      if (I->ld >= 0 || I->tail_line == 0) continue;
+      items.push_back({I->tail, 1});
+      lds = std::max(lds, I->tail_line);
+    }
+    for_lists(items, [&](const LaunchList& ll, int, int) { launch_tail_line(L, dT, ll, lds, stream); });
+  }
   for (int nzc : {0, 8, 16, 32}) {
     for (int a222 = 0; a222 < 2; ++a222) {
       for (int split = 0; split < 2; ++split) {
         std::vector<Item> items, coarse;
         size_t lds = 0;
         for (Instance* I : S) {
-          if (I->ld >= 0) continue;
+          if (I->ld >= 0 || I->tail_line > 0) continue;
           if (I->tail_nzc != nzc || (int)I->tail_222 != a222 || (int)I->tail_split != split) continue;
           items.push_back({I->tail, 1});
           lds = std::max(lds, I->tail_lds);

@@ -61,6 +61,7 @@ struct Instance {
   int tail_nzc = 16;             // tail kernel variant: column length class
   bool tail_222 = true;          //   and uniform 2:1 transfers
   bool tail_split = false;       // the coarse solve is its own kernel (large coarsest level)
+  size_t tail_line = 0;          // dynamic LDS bytes of the line tail (0: k_tail runs it)
   int fine[2] = {-1, -1};        // FP64 finest entries (u = p_cur for cur = 0/1)
   bool pairok = false;           // may pair cycles (DevLevel::pairok)
   int cur = 0;                   // which fine entry holds the current pressure
@@ -112,6 +113,10 @@ struct Context {
 
   int init(const amg_config& c);
   ~Context();
+  // lays out the line tail of a new instance, whose levels are ents, if it can
+  // take it (tl.tab, I->tail_line)
+  int plan_line_tail(Instance* I, const std::vector<DevLevel>& ents, const std::vector<DevXfer>& xf,
+                     DevTail& tl);
   // builds the hierarchy (or takes `built`, from check_grid) and allocates
   int add_instance(const amg_grid& g, Instance** out, Hierarchy* built = nullptr);
   int upload_tables();
