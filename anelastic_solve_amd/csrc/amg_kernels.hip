@@ -118,7 +118,15 @@ __device__ __forceinline__ int xcd_swizzle(int b, int n) {
 // Reciprocal for the line solves: the hardware rcp (1 ulp) in FP32, a
 // correctly rounded division in FP64.
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ double rcp(double x) { return 1.0 / x; }
+// FP64: the hardware's 24-bit estimate and two Newton steps, within 1 ulp
+// wherever x and its reciprocal are normal.  A z-line sweep has a chain of
+// kZSeg dependent reciprocals per segment: with the division in its place a
+// 64^3 half-sweep took 7.4 us instead of 6.8, a 128^3 one 10.1 instead of 9.5.
+__device__ __forceinline__ double rcp(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+  return __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+}
 
 // Fused multiply-add a*b + c, written out where several kernels have to
 // round alike.
@@ -443,10 +451,10 @@ __device__ __forceinline__ T zline_nbr(T wxl, T wxr, T wys, T wyn, T xl, T xr, T
 // NBR false: the other colour is zero (zero_guess bit 0, the first
 // half-sweep from u = 0) and is not read.  LEAN: the register-lean form of
 // the segment elimination (below).  H: a wave holds two segments of 32
-// columns (lanes 0-31 segment 2w, lanes 32-63 segment 2w+1), so a launch of
-// few column groups spreads over twice the CUs; p and lane (the column
-// within the workgroup's 32) are then per lane, and the z rows are staged
-// in LDS.  Every lane does the same operations in either shape.
+// columns (lanes 0-31 segment 2w, lanes 32-63 segment 2w+1), so a workgroup
+// has half the waves; p and lane (the column within the workgroup's 32) are
+// then per lane, and the z rows are staged in LDS.  Every lane does the same
+// operations in either shape.
 template <class T, int S, int C, bool NBR, bool LEAN, bool H>
 __device__ __forceinline__ void zline_group(const LevelHead& L, int parity, int zero_guess, int col0,
                                             int p, int lane, int P, T* __restrict__ lds, bool act) {
@@ -696,11 +704,12 @@ __device__ __forceinline__ void zline_group(const LevelHead& L, int parity, int 
 }
 
 // The LEAN FP32 form is built for 8 waves per SIMD (64 registers), so two
-// 1024-lane blocks share a CU and one's loads overlap the other's solve.
-// With H a workgroup has at most 8 waves and a CU holds one: up to 256
-// registers.
+// 1024-lane blocks share a CU and one's loads overlap the other's solve; the
+// LEAN FP64 form needs 128 registers and gets the same overlap from H, whose
+// workgroups have 8 waves.  H without LEAN is for launches of few column
+// groups: a CU holds one workgroup, which may use up to 256 registers.
 template <class T, int S, int C, bool NBR, bool LEAN, bool H>
-__global__ __launch_bounds__(H ? 512 : 1024, H ? 2 : ((LEAN && sizeof(T) == 4) ? 8 : 4)) void k_zline(
+__global__ __launch_bounds__(H ? 512 : 1024, LEAN ? 32 / (int)sizeof(T) : (H ? 2 : 4)) void k_zline(
     const DevLevel* __restrict__ Lt, LIST_PARAMS, int parity, int zero_guess, LaunchList ll) {
   extern __shared__ unsigned char lds_raw[];
   const Work wk = work_item(ln, lnb, li0, ll);
@@ -3286,7 +3295,7 @@ void launch_rb_point(bool fp64, const DevLevel* L, const LaunchList& ll, int par
   else LAUNCH(k_rb_point<float>, ll.nblocks, kBlock, L, LIST_ARGS(ll), parity, zero_guess, ll);
 }
 static void zline_variant(bool fp64, const DevLevel* L, const LaunchList& ll, int parity,
-                          int zero_guess, int segs, hipStream_t s, int form, bool nbr, bool half) {
+                          int zero_guess, int segs, hipStream_t s, bool lean, bool nbr, bool half) {
   // half: two segments of 32 columns per wave, segs rounded up to even
   const int wy = half ? (segs + 1) / 2 : segs, ps = half ? 2 * wy : segs, cw = half ? 32 : 64;
   const dim3 blk(64, wy);
@@ -3295,15 +3304,13 @@ static void zline_variant(bool fp64, const DevLevel* L, const LaunchList& ll, in
 #define ZL(T, CH, NBR, LEAN, H)                                                                   \
   hipLaunchKernelGGL((k_zline<T, kZSeg, CH, NBR, LEAN, H>), dim3(ll.nblocks), blk, lds, s, L, \
                      LIST_ARGS(ll), parity, zero_guess, ll)
-  // FP64 always takes the lean form (the short one does not fit its
-  // registers).  FP32 takes it when there are more blocks than CUs, so that
-  // blocks can pair up; a smaller launch is latency-bound and takes the
-  // shorter dependent chains of the short form (and, with half, twice the
-  // workgroups).
   if (fp64) {
-    if (half) {
+    if (!lean) {
       if (nbr) ZL(double, kZChunk64, true, false, true);
       else ZL(double, kZChunk64, false, false, true);
+    } else if (half) {
+      if (nbr) ZL(double, kZChunk64, true, true, true);
+      else ZL(double, kZChunk64, false, true, true);
     } else {
       if (nbr) ZL(double, kZChunk64, true, true, false);
       else ZL(double, kZChunk64, false, true, false);
@@ -3311,7 +3318,7 @@ static void zline_variant(bool fp64, const DevLevel* L, const LaunchList& ll, in
   } else if (half) {
     if (nbr) ZL(float, kZChunk32, true, false, true);
     else ZL(float, kZChunk32, false, false, true);
-  } else if (form == 2 || (form == 0 && ll.nblocks > device_cus())) {
+  } else if (lean) {
     if (nbr) ZL(float, kZChunk32, true, true, false);
     else ZL(float, kZChunk32, false, true, false);
   } else {
@@ -3322,10 +3329,23 @@ static void zline_variant(bool fp64, const DevLevel* L, const LaunchList& ll, in
 }
 void launch_zline(bool fp64, const DevLevel* L, const LaunchList& ll, int parity, int zero_guess,
                   int segs, hipStream_t s, int form) {
-  // A launch of at most half as many column groups as the device has CUs
-  // (and columns of two segments or more) runs 32 columns per workgroup:
-  // every item's block range doubles.  Forced forms keep 64.
-  const bool half = form == 0 && segs >= 2 && 2 * ll.nblocks <= device_cus();
+  // The shape, from the count of 64-column groups (forced forms keep 64
+  // columns):
+  // - at most half as many as the device has CUs, and columns of two segments
+  //   or more: 32 columns per workgroup, over twice the CUs, with the shorter
+  //   dependent chains of the short form;
+  // - up to the count of CUs: one group per CU is latency-bound too.  FP32
+  //   takes the short form, FP64 (which the short form leaves no registers)
+  //   the lean one;
+  // - more: blocks pair up on the CUs, the lean form's registers allowing.
+  //   FP64 needs the 32-column shape for that (256^3 48.1 -> 42.9 us, 4.18 ->
+  //   4.69 TB/s, where the lone 16-wave group of a CU loaded and solved in
+  //   turn; 512x256x128 41.4 -> 40.2; of 140 groups 11.2 -> 12.0).
+  const int cus = device_cus();
+  const bool few = form == 0 && segs >= 2 && 2 * ll.nblocks <= cus;
+  const bool many = form == 0 && ll.nblocks > cus;
+  const bool half = few || (many && fp64 && segs >= 2);
+  const bool lean = !few && (fp64 || many || form == 2);
   LaunchList hl;
   if (half) {
     hl = ll;
@@ -3337,11 +3357,11 @@ void launch_zline(bool fp64, const DevLevel* L, const LaunchList& ll, int parity
   // sweep for the instances whose cycle continues the iterate; each kernel
   // returns at once for the instances of the other
   if ((zero_guess & kZgDyn) && (zero_guess & 1)) {
-    zline_variant(fp64, L, l2, parity, zero_guess, segs, s, form, false, half);
-    zline_variant(fp64, L, l2, parity, kZgWarm, segs, s, form, true, half);
+    zline_variant(fp64, L, l2, parity, zero_guess, segs, s, lean, false, half);
+    zline_variant(fp64, L, l2, parity, kZgWarm, segs, s, lean, true, half);
     return;
   }
-  zline_variant(fp64, L, l2, parity, zero_guess, segs, s, form, !(zero_guess & 1), half);
+  zline_variant(fp64, L, l2, parity, zero_guess, segs, s, lean, !(zero_guess & 1), half);
 }
 size_t zline_table_bytes(int nz) { return sizeof(float) * kZRec * (((nz + kZSeg - 1) / kZSeg + 1) & ~1); }
 void launch_zline_table(const float* co32, int nx, int ny, int nz, float* zt, hipStream_t s) {
