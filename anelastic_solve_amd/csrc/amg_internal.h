@@ -57,8 +57,6 @@ struct DevLevel : LevelHead {
   int gslot;                 // the instance's slot in the per-instance gate array
   unsigned mhx, mny;         // ceil(2^32/hx), ceil(2^32/ny) (0 for a divisor of 1): e/hx = umulhi(e, mhx)
                              // exactly while e*hx < 2^32 (the coarse tail's small levels)
-  unsigned gmzp;             // gm_magic of nz rounded up to a multiple of 16 (the direct
-  int gszp;                  // solve's padded z extent)
   int bcx0, bcx1, bcy0, bcy1, bcz0, bcz1;   // boundary codes (prolongation ghosts)
   double vsum;               // finest: sum of cell volumes
   double vrsum;              // finest: sum of V*rho
@@ -331,16 +329,18 @@ void launch_coarse(bool fp64, const DevLevel* L, const LaunchList& ll, hipStream
 // at most kDirectCells cells with nx, ny multiples of 16 and nz <= 64,
 // computed in FP64 for an FP64 V-cycle and in FP32 for the FP32 V-cycle of
 // a mixed solve.  Every pass splits its output into slabs of kDirectCols
-// columns, one workgroup each (a level of 64^3 fills the device with 256):
-// 'planes' has nz*nx/kDirectCols blocks per item, 'slabs' nx*ny/kDirectCols;
-// lds = the largest direct_lds() of the items, at most direct_lds_limit().
-// (A larger FP32 level fits the LDS -- 128^3 does -- but its passes take
-// longer than the levels they would replace.)
+// rows or modes, one workgroup each (a level of 64^3 fills the device with
+// 256): 'planes' has nz*ny/kDirectCols blocks per item, 'slabs'
+// nx*ny/kDirectCols; lds = the largest direct_lds() of the items.
+// direct_fits: a plane's operands (the plane, the y matrix, 16 columns of the
+// x matrix) and the z pass's are at most one CU's LDS.  (A larger FP32 level
+// fits -- 128^3 does -- but its passes take longer than the levels they would
+// replace.)
 constexpr long long kDirectCells = 1 << 18;
 constexpr int kDirectCols = 16;
 constexpr int kDirectMaxNz = 64;
-size_t direct_lds(int nx, int ny, int nz, bool fp64);
-size_t direct_lds_limit();
+bool direct_fits(int nx, int ny, int nz, bool fp64);
+size_t direct_lds(int nx, int nz, bool fp64);
 void launch_direct(bool fp64, const DevLevel* L, const LaunchList& planes, const LaunchList& slabs,
                    size_t lds, hipStream_t s);
 // the coarse tail's short-column z-line sweep as a standalone launch (tests)

@@ -3039,8 +3039,18 @@ __global__ __launch_bounds__(kDivFin) void k_divergence_finalize(const double* _
 //   k_direct_z        per 16 modes:     x^ = Vz (inv .* (Vz^-1 f^))    (-> dscr + n)
 //   k_direct_xy<inv>  per plane k:      u_k = Vy x^_k Vx^T
 // with inv = 1/(lx + ly + lz) per eigenmode (0 for a singular operator's
-// null mode: the solution then has sum V u = 0).  Operands are staged in
-// LDS; rows are padded by one word against bank conflicts.
+// null mode: the solution then has sum V u = 0).
+//
+// Each pass is a few hundred short workgroups, so its time is its chain of
+// waits, not its products (a wave's two products at 64^3 are 32 matrix
+// instructions).  Every operand that comes from memory is therefore loaded
+// straight into the lanes that feed it to the matrix core, all of them before
+// the first product, and only the first product's result goes through LDS.
+// The plane passes take 16 rows of the plane per workgroup, (My[rows] X) Mx,
+// so that the elements of X and Mx lie across the lanes; the order of the sum
+// over k is free, and a lane takes four consecutive k of a row of My.  With
+// all operands staged through LDS in passes of 48 loads per thread the three
+// launches took 20.6 us at 64^3 in FP32 and 16.3 at 32^3 in FP64.
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 typedef float flt4 __attribute__((ext_vector_type(4)));
 
@@ -3063,77 +3073,54 @@ template <> struct Mfma16<float> {
   static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
 };
 
-// LDS of the plane passes and of the z pass (es: bytes per element)
-__host__ __device__ inline size_t direct_lds_xy(int nx, int ny, size_t es) {
-  return ((size_t)ny * (nx + 1) + (size_t)ny * (ny + 1) + (size_t)(nx + ny) * (kDirectCols + 1)) * es;
-}
-__host__ __device__ inline size_t direct_lds_z(int nzp, size_t es) {
-  return ((size_t)2 * nzp * (kDirectCols + 1) + (size_t)2 * nzp * (nzp + 1)) * es;
-}
+constexpr int kDirectZs = 20;   // row stride of the z pass's LDS (kDirectCols modes)
 __host__ __device__ inline int direct_nzp(int nz) { return (nz + 15) & ~15; }
 
-// C = A B for an nr x nc output, A (nr x nq, row stride as) and B (nq x nc,
-// row stride bs) in LDS; nr, nc, nq multiples of 16.  A wave takes one
-// 16x16 tile at a time (Mfma16 lane layout).  The operands of four products
-// are read before them.
-template <class CT, class AP, class BP, class F>
-__device__ __forceinline__ void mfma_products(AP A, int as, BP B, int bs, int nr, int nc, int nq,
-                                              F&& store) {
-  typedef Mfma16<CT> M;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const int li = lane & 15, lk = lane >> 4;
-  const int tr = nr >> 4, tc = nc >> 4;
-  for (int tile = wave; tile < tr * tc; tile += nw) {
-    const int r0 = (tile / tc) << 4, c0 = (tile % tc) << 4;
-    typename M::V acc = {CT(0), CT(0), CT(0), CT(0)};
-    for (int q0 = 0; q0 < nq; q0 += 16) {
-      CT av[4], bv[4];
+// A lane's operands of up to 64 consecutive k (n groups of 16): value [g][q]
+// belongs to k = k0 + 16 g + 4 (l / 16) + q of the lane's row or column.
+template <class CT> struct DirectOps {
+  typedef CT V4 __attribute__((ext_vector_type(4)));
+  CT v[4][4];
+  // f(k): the operand at k
+  template <class F> __device__ __forceinline__ void load(int n, int k0, F&& f) {
+    const int lk = (threadIdx.x & 63) >> 4;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        av[q] = A[(r0 + li) * as + q0 + 4 * q + lk];
-        bv[q] = B[(q0 + 4 * q + lk) * bs + c0 + li];
+    for (int g = 0; g < 4; ++g)
+      if (g < n) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[g][q] = f(k0 + 16 * g + 4 * lk + q);
       }
-#pragma unroll
-      for (int q = 0; q < 4; ++q) acc = M::op(av[q], bv[q], acc);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) store(r0 + M::row(lk, r), c0 + li, acc[r]);
   }
+  // row: the lane's row of operands, 4-element aligned
+  template <int AS, class E> __device__ __forceinline__ void load_row(int n, int k0, sp<AS, E> row) {
+    const int lk = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      if (g < n) {
+        const V4 t = *(sp<AS, const V4>)(row + k0 + 16 * g + 4 * lk);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[g][q] = t[q];
+      }
+  }
+};
+template <class CT>
+__device__ __forceinline__ typename Mfma16<CT>::V direct_mac(int n, const DirectOps<CT>& a,
+                                                             const DirectOps<CT>& b,
+                                                             typename Mfma16<CT>::V acc) {
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+    if (g < n) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc = Mfma16<CT>::op(a.v[g][q], b.v[g][q], acc);
+    }
+  return acc;
 }
 
-// Global -> LDS staging of three arrays at once, N loads of each in flight
-// per thread before any store (a loop of load-store pairs would wait out a
-// memory round trip per element): store_a(e, load_a(e)) for e < na, and
-// the same for b and c.
-template <int N, class CT, class LA, class SA, class LB, class SB, class LC, class SC>
-__device__ __forceinline__ void stage3(int na, LA&& la, SA&& sa, int nb, LB&& lb, SB&& sb, int nc,
-                                       LC&& lc, SC&& sc) {
-  const int bd = blockDim.x, step = N * bd;
-  const int n = max(na, max(nb, nc));
-  for (int e0 = threadIdx.x; e0 < n; e0 += step) {
-    CT va[N], vb[N], vc[N];
-#pragma unroll
-    for (int q = 0; q < N; ++q) {
-      const int e = e0 + q * bd;
-      va[q] = la(min(e, na - 1));
-      vb[q] = lb(min(e, nb - 1));
-      vc[q] = lc(min(e, nc - 1));
-    }
-#pragma unroll
-    for (int q = 0; q < N; ++q) {
-      const int e = e0 + q * bd;
-      if (e < na) sa(e, va[q]);
-      if (e < nb) sb(e, vb[q]);
-      if (e < nc) sc(e, vc[q]);
-    }
-  }
-}
-
-// The plane passes, one workgroup per (plane k, slab of kDirectCols columns
-// c0..): FWD: the slab of f^_k = Vy^-1 f_k Vx^-T into dscr, from plane k of
-// f (level precision T); otherwise the slab of u_k = Vy x^_k Vx^T from
-// dscr + n.  Either is My (X Mx[:, slab]) with the whole plane X staged.
-// The tables (dmat, dinv, dscr) hold CT values.
+// The plane passes, one workgroup per (plane k, 16 rows r0.. of it), a wave
+// per 16 columns: FWD: rows of f^_k = Vy^-1 f_k Vx^-T into dscr, from plane k
+// of f (level precision T); otherwise rows of u_k = Vy x^_k Vx^T from
+// dscr + n.  Either is (My[rows] X) Mx.  The tables (dmat, dinv, dscr) hold
+// CT values.
 template <class T, class CT, bool FWD>
 __global__ __launch_bounds__(kBlock) void k_direct_xy(const DevLevel* __restrict__ Lt, LIST_PARAMS,
                                                       LaunchList ll) {
@@ -3145,102 +3132,118 @@ __global__ __launch_bounds__(kBlock) void k_direct_xy(const DevLevel* __restrict
   pin_s(dmat, dscr);
   const LevelHead L = level_head(D);
   if (level_off(L)) return;
-  const int nx = L.nx, ny = L.ny, hx = L.hx, sx = nx + 1, sy = ny + 1;
-  constexpr int sc = kDirectCols + 1;
-  const int ns = nx / kDirectCols, q = wk.lb, k = q / ns, c0 = (q - k * ns) * kDirectCols;
-  const sp<kS, CT> X = (sp<kS, CT>)(sp<kS, double>)dl;   // the plane, ny x nx (stride sx)
-  const sp<kS, CT> My = X + ny * sx;         // FWD: Vy^-1, else Vy (ny x ny, stride sy)
-  const sp<kS, CT> Mx = My + ny * sy;        // columns c0.. of Vx^-T / Vx^T (nx x 16)
-  const sp<kS, CT> Y = Mx + nx * sc;         // X Mx (ny x 16)
+  const int nx = L.nx, ny = L.ny, hx = L.hx, sz = nx + 4;
+  const int rs = ny / kDirectCols, k = wk.lb / rs, r0 = (wk.lb - k * rs) * kDirectCols;
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), cstep = kBlock / 64 * 16;
+  const sp<kS, CT> Z = (sp<kS, CT>)(sp<kS, double>)dl;   // My[rows] X (16 x nx, stride sz)
   const auto m = gp(reinterpret_cast<const CT*>(dmat));
-  const size_t ox = FWD ? 0 : (size_t)nx * nx;
-  const size_t oy = (size_t)2 * nx * nx + (FWD ? 0 : (size_t)ny * ny);
-  auto lmx = [&](int e) { return m[ox + (size_t)(e / kDirectCols) * nx + c0 + e % kDirectCols]; };
-  auto smx = [&](int e, CT v) { Mx[(e / kDirectCols) * sc + e % kDirectCols] = v; };
-  auto lmy = [&](int e) { return m[oy + e]; };
-  // row and column of a staged element by the level's invariant divisors
-  // (e / nx = (e / 2) / hx)
-  auto smy = [&](int e, CT v) {
-    const int r = gm_div(e, L.gmny, L.gsny);
-    My[r * sy + e - r * ny] = v;
-  };
-  auto sxp = [&](int e, CT v) {
-    const int r = gm_div(e >> 1, L.gmhx, L.gshx);
-    X[r * sx + e - r * nx] = v;
-  };
+  const auto Mx = m + (FWD ? 0 : nx * nx);               // Vx^-T or Vx^T
+  const auto My = m + 2 * nx * nx + (FWD ? 0 : ny * ny) + (r0 + li) * ny;   // Vy^-1 or Vy
   const auto scr = gp(reinterpret_cast<CT*>(dscr));
-  if constexpr (FWD) {
-    const auto f = gfield<const T>((const void*)L.f);
-    auto lf = [&](int e) {
-      const int j = gm_div(e >> 1, L.gmhx, L.gshx), i = e - j * nx;
-      return (CT)f[cidx(i >> 1, j, k, (i + j) & 1, hx, ny)];
-    };
-    stage3<16, CT>(nx * ny, lf, sxp, ny * ny, lmy, smy, nx * kDirectCols, lmx, smx);
-  } else {
-    const auto in = scr + (size_t)L.ncell + (size_t)k * ny * nx;
-    stage3<16, CT>(nx * ny, [&](int e) { return in[e]; }, sxp, ny * ny, lmy, smy, nx * kDirectCols, lmx,
-                   smx);
+  const auto f = gfield<const T>((const void*)L.f);
+  const auto in = scr + (size_t)L.ncell + (size_t)k * ny * nx;
+  auto x_at = [&](int j, int i) {
+    if constexpr (FWD) return (CT)f[cidx(i >> 1, j, k, (i + j) & 1, hx, ny)];
+    else return (CT)in[j * nx + i];
+  };
+  auto groups = [](int left) { return min(4, left >> 4); };
+  DirectOps<CT> a, b, c;
+  auto load1 = [&](int c0, int q0) {
+    a.load_row(groups(ny - q0), q0, My);
+    b.load(groups(ny - q0), q0, [&](int j) { return x_at(j, c0 + li); });
+  };
+  auto load2 = [&](int c0, int q0) {
+    c.load(groups(nx - q0), q0, [&](int i) { return Mx[i * nx + c0 + li]; });
+  };
+  const int cw = 16 * wave;
+  if (cw < nx) {
+    load1(cw, 0);
+    load2(cw, 0);
+  }
+  typedef typename Mfma16<CT>::V V;
+  for (int c0 = cw; c0 < nx; c0 += cstep) {
+    V acc = {CT(0), CT(0), CT(0), CT(0)};
+    for (int q0 = 0; q0 < ny; q0 += 64) {
+      if (c0 != cw || q0) load1(c0, q0);
+      acc = direct_mac<CT>(groups(ny - q0), a, b, acc);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) Z[Mfma16<CT>::row(lk, r) * sz + c0 + li] = acc[r];
   }
   __syncthreads();
-  mfma_products<CT>(X, sx, Mx, sc, ny, kDirectCols, nx, [&](int r, int c, CT v) { Y[r * sc + c] = v; });
-  __syncthreads();
-  if constexpr (FWD) {
-    const auto out = scr + (size_t)k * ny * nx + c0;
-    mfma_products<CT>(My, sy, Y, sc, ny, kDirectCols, ny, [&](int r, int c, CT v) { out[r * nx + c] = v; });
-  } else {
-    const auto u = gfield<T>(L.u);
-    mfma_products<CT>(My, sy, Y, sc, ny, kDirectCols, ny, [&](int r, int c, CT v) {
-      const int i = c0 + c;
-      u[cidx(i >> 1, r, k, (i + r) & 1, hx, ny)] = (T)v;
-    });
+  for (int c0 = cw; c0 < nx; c0 += cstep) {
+    V acc = {CT(0), CT(0), CT(0), CT(0)};
+    for (int q0 = 0; q0 < nx; q0 += 64) {
+      if (c0 != cw || q0) load2(c0, q0);
+      a.load_row(groups(nx - q0), q0, Z + li * sz);
+      acc = direct_mac<CT>(groups(nx - q0), a, c, acc);
+    }
+    const int i = c0 + li;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int j = r0 + Mfma16<CT>::row(lk, r);
+      if constexpr (FWD) scr[(size_t)k * ny * nx + j * nx + i] = acc[r];
+      else gfield<T>(L.u)[cidx(i >> 1, j, k, (i + j) & 1, hx, ny)] = (T)acc[r];
+    }
   }
 }
 
-// The z pass, one workgroup per slab of kDirectCols modes m0.. (all k):
-// x^ = Vz (inv .* (Vz^-1 f^)).
+// The z pass, one workgroup per slab of kDirectCols modes m0.. (all k), a
+// wave per 16 of the nzp rows: x^ = Vz (inv .* (Vz^-1 f^)).
 template <class CT>
 __global__ __launch_bounds__(kBlock) void k_direct_z(const DevLevel* __restrict__ Lt, LIST_PARAMS,
                                                       LaunchList ll) {
+  static_assert(kDirectMaxNz <= 16 * (kBlock / 64) && kDirectMaxNz <= 64, "one chunk of rows per wave");
   extern __shared__ double dl[];
   const Work wk = work_item(ln, lnb, li0, ll);
   const DevLevel& D = Lt[wk.idx];
   const double *dmat = D.dmat, *dinv = D.dinv;
   double* dscr = D.dscr;
-  unsigned gmzp = D.gmzp;
-  int gszp = D.gszp;
-  pin_s(dmat, dinv, dscr, gmzp, gszp);
+  pin_s(dmat, dinv, dscr);
   const LevelHead L = level_head(D);
   if (level_off(L)) return;
-  const int nx = L.nx, ny = L.ny, nz = L.nz, nzp = direct_nzp(nz);
-  const int plane = nx * ny, m0 = wk.lb * kDirectCols, sz = nzp + 1;
-  constexpr int sc = kDirectCols + 1;
-  const sp<kS, CT> S = (sp<kS, CT>)(sp<kS, double>)dl;   // nzp x 16 (stride 17)
-  const sp<kS, CT> Tm = S + nzp * sc;        // nzp x 16
-  const sp<kS, CT> Wi = Tm + nzp * sc;       // Vz^-1 (nzp x nzp, stride sz)
-  const sp<kS, CT> W = Wi + nzp * sz;        // Vz
-  const auto m = gp(reinterpret_cast<const CT*>(dmat));
-  const size_t oz = (size_t)2 * nx * nx + (size_t)2 * ny * ny;
-  const auto fh = gp(reinterpret_cast<const CT*>(dscr));
-  const auto inv = gp(reinterpret_cast<const CT*>(dinv));
-  auto zrow = [&](int e) { return gm_div(e, gmzp, gszp); };   // e / nzp
-  stage3<16, CT>(
-      nzp * nzp, [&](int e) { return m[oz + e]; }, [&](int e, CT v) { Wi[zrow(e) * sz + e - zrow(e) * nzp] = v; },
-      nzp * nzp, [&](int e) { return m[oz + (size_t)nzp * nzp + e]; },
-      [&](int e, CT v) { W[zrow(e) * sz + e - zrow(e) * nzp] = v; }, nzp * kDirectCols,
-      [&](int e) {
-        const int k = min(e / kDirectCols, nz - 1);
-        return fh[(size_t)k * plane + m0 + e % kDirectCols];
-      },
-      [&](int e, CT v) { S[(e / kDirectCols) * sc + e % kDirectCols] = e / kDirectCols < nz ? v : CT(0); });
+  const int nx = L.nx, ny = L.ny, nz = L.nz, nzp = direct_nzp(nz), n = nzp >> 4;
+  const int plane = nx * ny, m0 = wk.lb * kDirectCols;
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int r0 = 16 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const sp<kS, CT> Tm = (sp<kS, CT>)(sp<kS, double>)dl;   // inv .* (Vz^-1 f^) (nzp x 16)
+  const auto Wi = gp(reinterpret_cast<const CT*>(dmat)) + 2 * nx * nx + 2 * ny * ny + (r0 + li) * nzp;
+  const auto W = Wi + nzp * nzp;                          // Vz, after Vz^-1
+  const auto fh = gp(reinterpret_cast<const CT*>(dscr)) + m0 + li;
+  const auto inv = gp(reinterpret_cast<const CT*>(dinv)) + m0 + li;
+  typedef typename Mfma16<CT>::V V;
+  DirectOps<CT> a, b, c;
+  const V zero = {CT(0), CT(0), CT(0), CT(0)};
+  const bool on = r0 < nzp;
+  if (on) {
+    CT iv[4];
+    a.load_row(n, 0, Wi);
+    b.load(n, 0, [&](int k) { return fh[min(k, nz - 1) * plane]; });
+#pragma unroll
+    for (int r = 0; r < 4; ++r) iv[r] = inv[min(r0 + Mfma16<CT>::row(lk, r), nz - 1) * plane];
+    c.load_row(n, 0, W);
+    // rows past nz are zero in the tables; the clamped data there may not be finite
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      if (16 * (e >> 2) + 4 * lk + (e & 3) >= nz) b.v[e >> 2][e & 3] = CT(0);
+    const V acc = direct_mac<CT>(n, a, b, zero);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = r0 + Mfma16<CT>::row(lk, r);
+      Tm[row * kDirectZs + li] = row < nz ? acc[r] * iv[r] : CT(0);
+    }
+  }
   __syncthreads();
-  mfma_products<CT>(Wi, sz, S, sc, nzp, kDirectCols, nzp, [&](int r, int c, CT v) {
-    Tm[r * sc + c] = r < nz ? v * inv[(size_t)r * plane + m0 + c] : CT(0);
-  });
-  __syncthreads();
-  const auto xo = gp(reinterpret_cast<CT*>(dscr)) + (size_t)L.ncell;
-  mfma_products<CT>(W, sz, Tm, sc, nzp, kDirectCols, nzp, [&](int r, int c, CT v) {
-    if (r < nz) xo[(size_t)r * plane + m0 + c] = v;
-  });
+  if (!on) return;
+  b.load(n, 0, [&](int k) { return Tm[k * kDirectZs + li]; });
+  const V acc = direct_mac<CT>(n, c, b, zero);
+  const auto xo = gp(reinterpret_cast<CT*>(dscr)) + (size_t)L.ncell + m0 + li;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = r0 + Mfma16<CT>::row(lk, r);
+    if (row < nz) xo[(size_t)row * plane] = acc[r];
+  }
 }
 
 inline unsigned nb(size_t n, int bs = kBlock) { return (unsigned)((n + bs - 1) / bs); }
@@ -3411,7 +3414,7 @@ void launch_prolong(bool fp64, const DevLevel* L, const DevXfer* X, const Launch
   if (fp64) LAUNCH(k_prolong<double>, ll.nblocks, kBlock, L, X, LIST_ARGS(ll), use_skip ? 1 : 0, ll);
   else LAUNCH(k_prolong<float>, ll.nblocks, kBlock, L, X, LIST_ARGS(ll), use_skip ? 1 : 0, ll);
 }
-size_t direct_lds_limit() {
+static size_t direct_lds_limit() {
   static size_t limit = 0;
   if (limit) return limit;
   int dev = 0, v = 0;
@@ -3436,9 +3439,15 @@ size_t direct_lds_limit() {
   limit = lim;
   return limit;
 }
-size_t direct_lds(int nx, int ny, int nz, bool fp64) {
+size_t direct_lds(int nx, int nz, bool fp64) {
   const size_t es = fp64 ? sizeof(double) : sizeof(float);
-  return std::max(direct_lds_xy(nx, ny, es), direct_lds_z(direct_nzp(nz), es));
+  return es * std::max((size_t)kDirectCols * (nx + 4), (size_t)direct_nzp(nz) * kDirectZs);
+}
+bool direct_fits(int nx, int ny, int nz, bool fp64) {
+  const size_t nzp = direct_nzp(nz), pad = kDirectCols + 1;
+  const size_t xy = (size_t)ny * (nx + 1) + (size_t)ny * (ny + 1) + (size_t)(nx + ny) * pad;
+  const size_t z = 2 * nzp * pad + 2 * nzp * (nzp + 1);
+  return std::max(xy, z) * (fp64 ? sizeof(double) : sizeof(float)) <= direct_lds_limit();
 }
 void launch_direct(bool fp64, const DevLevel* L, const LaunchList& planes, const LaunchList& slabs,
                    size_t lds, hipStream_t s) {

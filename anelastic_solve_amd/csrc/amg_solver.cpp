@@ -303,7 +303,6 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
     d.mny = magic((unsigned)d.ny);
     d.gmhx = gm_magic((unsigned)d.hx, &d.gshx);
     d.gmny = gm_magic((unsigned)d.ny, &d.gsny);
-    d.gmzp = gm_magic((unsigned)((d.nz + 15) & ~15), &d.gszp);
     d.px = I->H.bc[0][0] == AMG_BC_PERIODIC;
     d.py = I->H.bc[1][0] == AMG_BC_PERIODIC;
     d.pz = I->H.bc[2][0] == AMG_BC_PERIODIC;
@@ -532,7 +531,7 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
   // separable direct solve of the first level below the finest, above the
   // coarse tail (the tail solves small levels in one launch), that the
   // direct solve takes: at most kDirectCells cells, nx and ny multiples of
-  // 16, nz <= kDirectMaxNz, the operands within the LDS; the levels below it
+  // 16, nz <= kDirectMaxNz, direct_fits; the levels below it
   // are not cycled.  A mixed solve computes it in FP32 (its tables are
   // FP32), an FP64 one in FP64.
   if (cfg.coarse_direct != 0) {
@@ -541,10 +540,9 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
     for (int cand = 1; cand < I->l0; ++cand) {
       const HostLevel& H = I->H.lv[cand];
       if (H.ncell() > kDirectCells) continue;
-      const size_t lds = direct_lds(H.nx, H.ny, H.nz, f64);
       DirectTables D;
       std::string derr;
-      if (!(H.nx % 16 == 0 && H.ny % 16 == 0 && H.nz <= kDirectMaxNz && lds <= direct_lds_limit() &&
+      if (!(H.nx % 16 == 0 && H.ny % 16 == 0 && H.nz <= kDirectMaxNz && direct_fits(H.nx, H.ny, H.nz, f64) &&
             direct_setup(H, I->H.bc, I->H.singular, &D, &derr)))
         continue;
       void* dm = I->mem.alloc(D.mats.size() * es);
@@ -564,7 +562,7 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
       d.dinv = (double*)di;
       d.dscr = (double*)ds;
       I->ld = cand;
-      I->dlds = lds;
+      I->dlds = direct_lds(H.nx, H.nz, f64);
       break;
     }
   }
@@ -890,7 +888,7 @@ void Context::vcycle(const std::vector<Instance*>& S, bool fp64) {
     for (Instance* I : S) {
       if (I->ld < 0) continue;
       const int li = I->lev[I->ld];
-      planes.push_back({li, hL[li].nz * (hL[li].nx / kDirectCols)});
+      planes.push_back({li, hL[li].nz * (hL[li].ny / kDirectCols)});
       modes.push_back({li, hL[li].ny * (hL[li].nx / kDirectCols)});
       lds = std::max(lds, I->dlds);
     }
@@ -1437,7 +1435,7 @@ int Context::run_kernel(Instance* I, int which, int level, int reps, double* byt
     }
     b = 2.0 * w * d.ncell;
     for (int r = 0; r < reps; ++r)
-      direct_launches({{I->lev[level], d.nz * (d.nx / kDirectCols)}},
+      direct_launches({{I->lev[level], d.nz * (d.ny / kDirectCols)}},
                       {{I->lev[level], d.ny * (d.nx / kDirectCols)}}, I->dlds, fp64);
     AMG_HIP(hipGetLastError());
     if (bytes) *bytes = b;
