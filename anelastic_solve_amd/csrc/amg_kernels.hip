@@ -3048,9 +3048,10 @@ __global__ __launch_bounds__(kDivFin) void k_divergence_finalize(const double* _
 // the first product, and only the first product's result goes through LDS.
 // The plane passes take 16 rows of the plane per workgroup, (My[rows] X) Mx,
 // so that the elements of X and Mx lie across the lanes; the order of the sum
-// over k is free, and a lane takes four consecutive k of a row of My.  With
-// all operands staged through LDS in passes of 48 loads per thread the three
-// launches took 20.6 us at 64^3 in FP32 and 16.3 at 32^3 in FP64.
+// over k is free, and a lane takes four consecutive k of a row of My.  The three
+// launches take 11.4 us at 64^3 in FP32 and 9.4 at 32^3 in FP64 (22.0 and
+// 20.2 with every operand staged through LDS, in passes of 48 loads per
+// thread whatever the size); FP32 64x16x64 17.2 -> 9.4, FP64 64^3 28.2 -> 17.
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 typedef float flt4 __attribute__((ext_vector_type(4)));
 
