@@ -2396,16 +2396,17 @@ __device__ __forceinline__ GatePre gate_pre(const ItemGate* g, const double* out
   return P;
 }
 
-// End of a gated cycle of one instance (one thread; L its item's level,
-// the FP64 finest): the first cycle of a pair only hands over to the
+// End of a gated cycle of one instance (its item's level is the FP64
+// finest): the first cycle of a pair only hands over to the
 // second; otherwise the correction's norms are recorded and the stop rule
 // of the host's norm step (Context::post_norms) applied to them with the
 // same double operations, so the host's replay reaches the same decision;
 // then the next cycle is planned (paired or not).  Returns the state words
 // the instance's levels take.
 // P holds what it reads (gate_pre, with the norms of the calling fold put
-// in); only stores remain here.
-__device__ GateWords item_gate_check(ItemGate* g, const GatePre& P) {
+// in); only stores remain here, and only the thread with `keep` makes them:
+// the others take the same words from the same values.
+__device__ __forceinline__ GateWords item_gate_check(ItemGate* g, const GatePre& P, bool keep) {
   const double* o = P.o;
   const double* oc = P.oc;
   const int gstop = P.gstop, cycles = P.cycles + 1, n = P.n, maxcy = P.maxcy;
@@ -2413,20 +2414,22 @@ __device__ GateWords item_gate_check(ItemGate* g, const GatePre& P) {
   const double bnorm = P.bnorm, tol = P.tol, rprev = P.rprev;
   const int skipc = P.skipc, warm = P.warm;
   if (gstop) return {-1, -1, -1, 0};
-  g->cycles = cycles;
+  if (keep) g->cycles = cycles;
   if (skipc) return {-1, 1, 0, 0};
   const int m = warm ? 2 : 1;
-  double* h = g->hist[n % kItemRing];
-  for (int q = 0; q < 4; ++q) h[q] = o[q];
-  h[4] = report ? oc[0] : 0.0;
-  h[5] = report ? oc[1] : 0.0;
-  g->hcyc[n % kItemRing] = m;
+  if (keep) {
+    double* h = g->hist[n % kItemRing];
+    for (int q = 0; q < 4; ++q) h[q] = o[q];
+    h[4] = report ? oc[0] : 0.0;
+    h[5] = report ? oc[1] : 0.0;
+    g->hcyc[n % kItemRing] = m;
+    g->count = n + 1;
+  }
   const double rmax = o[0];
   double relmax;
   if (fp64) relmax = report ? (oc[1] > 0.0 ? oc[0] / oc[1] : 0.0) : __longlong_as_double(0x7ff8000000000000ll);
   else relmax = o[2] > 0.0 ? o[1] / o[2] : 0.0;
   const double relres = bnorm > 0.0 ? rmax / bnorm : rmax;
-  g->count = n + 1;
   int stop = 0;
   if (!isfinite(rmax)) {
     stop = 1;
@@ -2435,8 +2438,10 @@ __device__ GateWords item_gate_check(ItemGate* g, const GatePre& P) {
     if (crit <= tol || cycles >= maxcy) stop = 1;
   }
   const bool pair = !stop && gpair && cycles + 2 <= maxcy && pair_next(relres, rprev, m, tol);
-  g->rprev = relres;
-  g->stop = stop;
+  if (keep) {
+    g->rprev = relres;
+    g->stop = stop;
+  }
   return {stop, 0, pair ? 1 : 0, fp64 ? 0 : 1};
 }
 
@@ -2472,30 +2477,45 @@ __global__ void k_gate_init(LaunchList ll, const double* __restrict__ out, ItemG
 
 // One block per item: thread t folds partials b0+t, b0+t+kFinBlock, ... in
 // order, then a fixed-shape tree combines the threads (deterministic).  With
-// per-instance gates, thread 0 of every item's block then ends its cycle and
-// the block's threads write the resulting state words, one table entry each.
+// per-instance gates, the block then ends its item's cycle and writes the
+// resulting state words, one table entry per thread.
+//
+// The kernel is one chain of waits: a store before a barrier is one (the
+// barrier waits until it has arrived), a load after it another.  So the gate
+// and the entries' own words are loaded before the fold, all values meet at
+// one barrier, the waves' values are read from LDS together (a loop of
+// read-and-fold costs 0.8 us per value), every thread with a table entry then
+// takes the decision for itself, and all stores come last.  4096 partials of
+// three values: 6.3 us (9.7 with two barriers per value, the decision passed
+// on by another and pcur read to toggle it); 1024: 5.7 (8.9); 64: 4.6 (6.3).
+// SUM: the values are summed; otherwise they are magnitudes (or NaN) and the
+// largest is taken.
 constexpr int kFinBlock = 1024;
-__global__ __launch_bounds__(kFinBlock) void k_finalize(LIST_PARAMS, int nvals, int op_sum,
+template <bool SUM>
+__global__ __launch_bounds__(kFinBlock) void k_finalize(LIST_PARAMS, int nvals,
                                                         const double* __restrict__ partial,
                                                         double* __restrict__ out, int ostride,
                                                         GateArgs ga, LaunchList ll) {
-  __shared__ double sm[kFinBlock / 64];
+  constexpr int kWaves = kFinBlock / 64;
+  __shared__ double sm[4][kWaves];
   const int t = blockIdx.x;
   const bool one = ln == 1;
   const int b0 = one ? 0 : ll.prefix[t], b1 = one ? lnb : ll.prefix[t + 1];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  // the gate's inputs, loaded before the fold (thread 0), and the instance
-  // number of every thread's first table entry (never written on the device);
-  // a launch of one item knows its gate's place
+  // the threads that see the folded values: one per table entry with gates
+  const int nsee = ga.ig ? max(64, ga.nL) : 64;
+  // a launch of one item knows its gate's place; a thread's first entry (its
+  // instance never changes on the device, its pcur only here)
   GatePre gpre;
-  int inst0 = -1;
-  if (ga.ig) {
-    if (threadIdx.x < ga.nL) inst0 = ga.Lt[threadIdx.x].inst;
-    if (threadIdx.x == 0) {
-      const DevLevel& L = ga.Lt[one ? li0 : ll.items[t]];
-      const int slot = one ? ga.slot : L.gslot, inst = one ? ga.inst : L.inst;
-      gpre = gate_pre(ga.ig + slot, ga.out + (size_t)t * 4, ga.outc + (size_t)t * 2, L, slot, inst);
+  int inst0 = -1, pcur0 = 0;
+  if (ga.ig && (int)threadIdx.x < nsee) {
+    if ((int)threadIdx.x < ga.nL) {
+      inst0 = ga.Lt[threadIdx.x].inst;
+      pcur0 = ga.Lt[threadIdx.x].pcur;
     }
+    const DevLevel& L = ga.Lt[one ? li0 : ll.items[t]];
+    const int slot = one ? ga.slot : L.gslot, inst = one ? ga.inst : L.inst;
+    gpre = gate_pre(ga.ig + slot, ga.out + (size_t)t * 4, ga.outc + (size_t)t * 2, L, slot, inst);
   }
   // one pass over the partials for every value (nvals <= 4), kFinU
   // partials per thread and round: their loads (clamped into the item, so
@@ -2515,59 +2535,57 @@ __global__ __launch_bounds__(kFinBlock) void k_finalize(LIST_PARAMS, int nvals, 
       if (b + r * kFinBlock < b1) {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          if (q < nvals) acc[q] = op_sum ? acc[q] + x[r][q] : nmax(acc[q], x[r][q]);
+          if (q < nvals) acc[q] = SUM ? acc[q] + x[r][q] : amax(acc[q], x[r][q]);
       }
     }
   }
-  double fr[4] = {0.0, 0.0, 0.0, 0.0};   // thread 0: the folded values
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     if (q >= nvals) break;
-    double a = acc[q];
-    a = op_sum ? wave_sum(a) : wave_max(a);
-    if (lane == 0) sm[w] = a;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      double r = sm[0];
-      for (int i = 1; i < kFinBlock / 64; ++i) r = op_sum ? r + sm[i] : nmax(r, sm[i]);
-      out[(size_t)t * ostride + q] = r;
-      fr[q] = r;
-    }
-    __syncthreads();
-  }
-  if (ga.ig) {
-    __shared__ GateWords gw;
-    __shared__ int ginst;
-    if (threadIdx.x == 0) {
-      // the gate's norms that this fold wrote: its values, not the loads
-      // made before it
-      const double* mine = out + (size_t)t * ostride;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (q >= nvals) break;
-        for (int r = 0; r < 4; ++r)
-          if (ga.out + (size_t)t * 4 + r == mine + q) gpre.o[r] = fr[q];
-        for (int r = 0; r < 2; ++r)
-          if (ga.outc + (size_t)t * 2 + r == mine + q) gpre.oc[r] = fr[q];
-      }
-      // (the descriptor's words as loaded before the fold: the stores to
-      // out may alias the table as far as the compiler knows)
-      gw = item_gate_check(ga.ig + gpre.gslot, gpre);
-      ginst = gpre.inst;
+    for (int off = 32; off > 0; off >>= 1) {
+      const double o = __shfl_xor(acc[q], off, 64);
+      acc[q] = SUM ? acc[q] + o : amax(acc[q], o);
     }
-    __syncthreads();
-    // the first entry of each thread from its prefetched instance number
-    const GateWords wv = gw;
-    const int gi = ginst;
-    if (threadIdx.x < ga.nL && inst0 == gi) {
-      DevLevel& d = ga.Lt[threadIdx.x];
-      if (wv.stop >= 0) d.stop = wv.stop;
-      if (wv.warm >= 0) d.warm = wv.warm;
-      if (wv.skipc >= 0) d.skipc = wv.skipc;
-      if (wv.pflip) d.pcur ^= 1;
-    }
-    set_words(ga.Lt, ga.nL, gi, wv, threadIdx.x + kFinBlock, kFinBlock);
+    if (lane == 0) sm[q][w] = acc[q];
   }
+  __syncthreads();
+  if ((int)threadIdx.x >= nsee) return;
+  double fr[4];   // the folded values
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if (q >= nvals) break;
+    double x[kWaves];
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) x[i] = sm[q][i];
+#pragma unroll
+    for (int i = 1; i < kWaves; ++i) x[0] = SUM ? x[0] + x[i] : amax(x[0], x[i]);
+    fr[q] = x[0];
+  }
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (q < nvals) out[(size_t)t * ostride + q] = fr[q];
+  }
+  if (!ga.ig) return;
+  // the gate's norms that this fold wrote: its values, not the loads made
+  // before it
+  const bool norms = out == ga.out, change = out == ga.outc;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if (q >= nvals) break;
+    if (norms) gpre.o[q] = fr[q];
+    if (change && q < 2) gpre.oc[q] = fr[q];
+  }
+  const GateWords wv = item_gate_check(ga.ig + gpre.gslot, gpre, threadIdx.x == 0);
+  if (inst0 == gpre.inst) {
+    DevLevel& d = ga.Lt[threadIdx.x];
+    if (wv.stop >= 0) d.stop = wv.stop;
+    if (wv.warm >= 0) d.warm = wv.warm;
+    if (wv.skipc >= 0) d.skipc = wv.skipc;
+    if (wv.pflip) d.pcur = pcur0 ^ 1;
+  }
+  set_words(ga.Lt, ga.nL, gpre.inst, wv, threadIdx.x + kFinBlock, kFinBlock);
 }
 
 // ---------------------------------------------------------------------------
@@ -3581,7 +3599,8 @@ void launch_finalize(const LaunchList& ll, const double* partial, int nvals, int
                      int ostride, hipStream_t s, const GateArgs* gate) {
   GateArgs ga{};
   if (gate) ga = *gate;
-  LAUNCH(k_finalize, ll.nitems, kFinBlock, LIST_ARGS(ll), nvals, op_sum, partial, out, ostride, ga, ll);
+  if (op_sum) LAUNCH(k_finalize<true>, ll.nitems, kFinBlock, LIST_ARGS(ll), nvals, partial, out, ostride, ga, ll);
+  else LAUNCH(k_finalize<false>, ll.nitems, kFinBlock, LIST_ARGS(ll), nvals, partial, out, ostride, ga, ll);
 }
 void launch_from_fortran(const DevLevel* L, const LaunchList& ll, const PtrList& ptr, int which,
                          int add_fold, hipStream_t s) {
