@@ -57,6 +57,7 @@ struct DevLevel : LevelHead {
   int gslot;                 // the instance's slot in the per-instance gate array
   unsigned mhx, mny;         // ceil(2^32/hx), ceil(2^32/ny) (0 for a divisor of 1): e/hx = umulhi(e, mhx)
                              // exactly while e*hx < 2^32 (the coarse tail's small levels)
+  void* w;                   // the black cells between two paired point sweeps (rb_pair), or null
   int bcx0, bcx1, bcy0, bcy1, bcz0, bcz1;   // boundary codes (prolongation ghosts)
   double vsum;               // finest: sum of cell volumes
   double vrsum;              // finest: sum of V*rho
@@ -265,6 +266,18 @@ inline int rb_march_planes(int hx, int ny, int nz) {
     if (nz >= K && (long long)hx * ny * ((nz + K - 1) / K) >= (1 << 18)) return K;
   return 0;
 }
+// Whole point sweeps (red, then black) of levels with a buffer w for the
+// black cells, in pairs: back 0 leaves the black cells in w, back 1 brings
+// them back to u.  rb_pair: whether a level's sweeps run so, as slabs of tz
+// planes (0: they do not) in `blocks` blocks; every item of a launch has that
+// tz and hx <= hx_max.
+constexpr int kPairY = 4;
+struct RbPair {
+  int tz, blocks;
+};
+RbPair rb_pair(bool fp64, int hx, int ny, int nz);
+void launch_rb_pair(bool fp64, const DevLevel* L, const LaunchList& ll, int zero_guess, int back,
+                    int tz, int hx_max, hipStream_t s);
 // z-line sweeps run 64 columns per workgroup and 'segs' = ceil(nz_max/kZSeg)
 // waves (segments of kZSeg cells) per column group; every item of one
 // launch must have nz <= segs*kZSeg.

@@ -406,6 +406,133 @@ __global__ __launch_bounds__(kBlock) void k_rb_march(const DevLevel* __restrict_
   }
 }
 
+// Both half-sweeps of a point sweep in one launch.  A workgroup takes kPairY
+// rows by TZ planes of whole x rows: it updates their red cells and those of
+// the rows and planes around them (whose owners do the same sums) into LDS,
+// then its black cells from there.  Other workgroups still read the old black
+// values, so the new ones go to another buffer: `back` 0 reads them from u and
+// writes w, 1 the other way; a level's sweeps run in such pairs.  Red cells
+// are written to u, and no workgroup reads them from memory.
+//
+// Small levels are bound by launches: a half-sweep of 64^3 in FP64 takes 2.4
+// us and the gap to the next 1, a whole sweep here 4.1 (solve 4500 -> 4100
+// us).  Larger ones are bound by the cache's traffic: b once and u read and
+// written once, for half of u four times and b once: at 256x64x256 in FP32
+// 17.2 -> 13.0 us.
+//
+// Thread (m, row) owns a position of row j0 - 1 + row, both halves, and
+// marches in z as k_rb_march does, so a red cell costs six loads and no z
+// coefficient (a thread per cell with all of its own loads took 4.4 us at
+// 64^3, 24 at 256x64x256).  kPairY 2, 6, 8 and TZ 8 were slower on both (64^3:
+// 4370, 4235, 4450 us and, spilling, 6490).
+template <class T, int TZ>
+__global__ __launch_bounds__(1024) void k_rb_pair(const DevLevel* __restrict__ Lt, LIST_PARAMS,
+                                                  int zero_guess, int back, LaunchList ll) {
+  constexpr int TY = kPairY;
+  extern __shared__ unsigned char lds_raw[];
+  const sp<kS, T> red = (sp<kS, T>)(sp<kS, unsigned char>)lds_raw;
+  const Work wk = work_item(ln, lnb, li0, ll);
+  const DevLevel& D = Lt[wk.idx];
+  void* wp = D.w;
+  pin_s(wp);
+  const LevelHead L = level_head(D);
+  if (level_off(L)) return;
+  const bool nbr = !(zero_flags(L, zero_guess) & 1);
+  const int hx = L.hx, ny = L.ny, nz = L.nz, nx = L.nx;
+  const int nty = (ny + TY - 1) / TY;
+  const int bz = wk.lb / nty, j0 = (wk.lb - bz * nty) * TY, k0 = bz * TZ;
+  const int row = gm_div(threadIdx.x, L.gmhx, L.gshx), m = threadIdx.x - row * hx, dy = row - 1;
+  const bool act = row < TY + 2;
+  auto wrap = [](int a, int n) { return a < 0 ? a + n : a >= n ? a - n : a; };
+  const int j = act ? wrap(j0 + dy, ny) : 0, jm = wrap(j - 1, ny), jp = wrap(j + 1, ny);
+  const bool own = act && dy >= 0 && dy < TY && j0 + dy < ny;
+  const sp<kG, const T> co = coefs<T>(L);
+  const sp<kG, const T> cy = co + 3 * nx;
+  const sp<kG, const T> cz = cy + 3 * ny;
+  const auto u = gfield<T>(L.u);
+  const auto f = gfield<const T>((const void*)L.f);
+  const sp<kG, const T> ub = gfield<const T>((const void*)(back ? wp : L.u));
+  const sp<kG, T> wb = gfield<T>(back ? L.u : wp);
+  // the thread's two columns, of half h: i = 2m + b with b = (h + j) & 1
+  const int b0 = j & 1, b1 = b0 ^ 1;
+  const int mm = m == 0 ? hx - 1 : m - 1, mp = m == hx - 1 ? 0 : m + 1;
+  const int ml[2] = {b0 ? m : mm, b0 ? mm : m}, mr[2] = {b0 ? mp : m, b0 ? m : mp};
+  const T wxl[2] = {co[2 * m + b0], co[2 * m + b1]}, wxr[2] = {co[nx + 2 * m + b0], co[nx + 2 * m + b1]};
+  const T dxx[2] = {co[2 * nx + 2 * m + b0], co[2 * nx + 2 * m + b1]};
+  const T wys = cy[j], wyn = cy[ny + j], dyy = cy[2 * ny + j];
+  auto at = [&](int k, int h, int jj, int q) { return ((k * ny + jj) * 2 + h) * hx + q; };
+  // red plane s of the march is plane k0 - 1 + s, black plane s k0 + s; the
+  // half of a plane is its number's (k0 is even)
+  auto plane = [&](int s) { return wrap(k0 - 1 + s, nz); };
+  auto value = [&](int h, T fv, T zm_, T zp_, T zd, T xl, T xr, T ys, T yn, T zm, T zp) {
+    const T d = (zd + dyy) + dxx[h];
+    T a = wxl[h] * xl + wxr[h] * xr;
+    a += wys * ys;
+    a += wyn * yn;
+    a += zm_ * zm;
+    a += zp_ * zp;
+    return over(fv - a, d);
+  };
+  constexpr int NR = TZ + 2;
+  T wzm[NR], wzp[NR], dzz[NR];
+  T fv[NR], xl[NR], xr[NR], ys[NR], yn[NR], zc[NR + 2], fb[TZ];
+  // (behind a wall of an odd nz the far plane counts as the number the march
+  // gives it: whatever half that names meets a zero coupling)
+  auto hr = [](int s) { return (s + 1) & 1; };   // half of red plane s
+#pragma unroll
+  for (int s = 0; s < NR; ++s) {
+    const int k = plane(s);
+    wzm[s] = cz[k];
+    wzp[s] = cz[nz + k];
+    dzz[s] = cz[2 * nz + k];
+  }
+  if (act) {
+#pragma unroll
+    for (int s = 0; s < NR; ++s) {
+      const int k = plane(s), h = hr(s);
+      fv[s] = f[at(k, h, j, m)];
+      if (nbr) {
+        xl[s] = ub[at(k, h ^ 1, j, ml[h])];
+        xr[s] = ub[at(k, h ^ 1, j, mr[h])];
+        ys[s] = ub[at(k, h ^ 1, jm, m)];
+        yn[s] = ub[at(k, h ^ 1, jp, m)];
+        zc[s + 2] = ub[at(wrap(k + 1, nz), h, j, m)];
+      }
+    }
+    if (nbr) {
+      zc[0] = ub[at(wrap(plane(0) - 1, nz), hr(0), j, m)];
+      zc[1] = ub[at(plane(0), hr(1), j, m)];
+    }
+    if (own) {
+#pragma unroll
+      for (int s = 0; s < TZ; ++s) fb[s] = f[at(min(k0 + s, nz - 1), (s + 1) & 1, j, m)];
+    }
+#pragma unroll
+    for (int s = 0; s < NR; ++s) {
+      const int h = hr(s);
+      const T v = nbr ? value(h, fv[s], wzm[s], wzp[s], dzz[s], xl[s], xr[s], ys[s], yn[s], zc[s], zc[s + 2])
+                      : over(fv[s], (dzz[s] + dyy) + dxx[h]);
+      red[(s * (TY + 2) + row) * hx + m] = v;
+      fv[s] = v;
+    }
+  }
+  __syncthreads();
+  if (!own) return;
+  // the red cells are stored here: a barrier waits for stores
+#pragma unroll
+  for (int s = 0; s < TZ; ++s)
+    if (k0 + s < nz) u[at(k0 + s, s & 1, j, m)] = fv[s + 1];
+  auto rd = [&](int s, int r, int q) { return red[(s * (TY + 2) + r) * hx + q]; };
+#pragma unroll
+  for (int s = 0; s < TZ; ++s) {
+    if (k0 + s >= nz) break;
+    const int h = (s + 1) & 1;
+    wb[at(k0 + s, h, j, m)] =
+        value(h, fb[s], wzm[s + 1], wzp[s + 1], dzz[s + 1], rd(s + 1, row, ml[h]), rd(s + 1, row, mr[h]),
+              rd(s + 1, row - 1, m), rd(s + 1, row + 1, m), rd(s, row, m), rd(s + 2, row, m));
+  }
+}
+
 // ---------------------------------------------------------------------------
 // z-line red-black Gauss-Seidel half-sweep (mgMK/mg_relax.F90:423-600, LJ):
 // the columns (i,j) of one colour ((i+j)&1 == parity) solve their
@@ -3310,6 +3437,38 @@ void launch_rb_march(bool fp64, const DevLevel* L, const LaunchList& ll, int par
     if (planes == 8) RM(float, 8); else if (planes == 4) RM(float, 4); else RM(float, 2);
   }
 #undef RM
+}
+RbPair rb_pair(bool fp64, int hx, int ny, int nz) {
+  // Whole rows in a workgroup of at most 1024 threads, and halos that wrap
+  // at most once.
+  if ((kPairY + 2) * hx > 1024 || ny < kPairY || nz < 4) return {0, 0};
+  // Three fields (u, w, b) that stay in the cache: past that the sweep waits
+  // for HBM and the halos' extra reads lose (12 cycles of FP64 256x128x128
+  // 2692 -> 2605 us, of 256x256x128 4158 -> 4486; FP32 256^3 4725 -> 4483,
+  // 256x512x256 9598 -> 10117).
+  if (2ll * hx * ny * nz > (fp64 ? 1ll << 22 : 1ll << 24)) return {0, 0};
+  // Slabs of four planes, or of two where four leave CUs idle (32^3 FP64 932
+  // -> 904 us, 64x32x32 FP32 1042 -> 1010; at 64^3, with as many workgroups
+  // as CUs, 650 against 654).
+  const int rows = (ny + kPairY - 1) / kPairY;
+  const int tz = rows * ((nz + 3) / 4) < device_cus() ? 2 : 4;
+  return {tz, rows * ((nz + tz - 1) / tz)};
+}
+void launch_rb_pair(bool fp64, const DevLevel* L, const LaunchList& ll, int zero_guess, int back,
+                    int tz, int hx_max, hipStream_t s) {
+  const int threads = ((kPairY + 2) * hx_max + 63) & ~63;
+  const size_t lds = (size_t)(kPairY + 2) * (tz + 2) * hx_max * (fp64 ? 8 : 4);
+#define RB(T, TZ)                                                                                \
+  hipLaunchKernelGGL((k_rb_pair<T, TZ>), dim3(ll.nblocks), dim3(threads), lds, s, L, LIST_ARGS(ll), \
+                     zero_guess, back, ll)
+  if (fp64) {
+    if (tz == 2) RB(double, 2);
+    else RB(double, 4);
+  } else {
+    if (tz == 2) RB(float, 2);
+    else RB(float, 4);
+  }
+#undef RB
 }
 void launch_rb_point(bool fp64, const DevLevel* L, const LaunchList& ll, int parity, int zero_guess,
                      hipStream_t s) {

@@ -566,6 +566,20 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
       break;
     }
   }
+  // point sweeps in pairs on the levels cycled by launches (without the
+  // buffer a level's half-sweeps run one by one)
+  for (int l = 0; cfg.smoother != AMG_SMOOTHER_LJ && l < I->lc(); ++l) {
+    DevLevel& d = newL[l];
+    if (std::max(I->pre[l], I->post[l]) < 2 || !rb_pair(I->fp64, d.hx, d.ny, d.nz).tz) continue;
+    d.w = I->mem.alloc((size_t)d.ncell * w);
+    if (!d.w) {
+      (void)hipGetLastError();
+      continue;
+    }
+    // its red cells stay zero: with an odd nz a sweep reads some (the far
+    // side of a wall, times a zero coupling)
+    launch_zero((double*)d.w, (int)((size_t)d.ncell * w / sizeof(double)), stream);
+  }
   // projection metrics
   {
     const HostLevel& F = I->H.lv[0];
@@ -840,11 +854,18 @@ void Context::vcycle(const std::vector<Instance*>& S, bool fp64) {
     for (Instance* I : S)
       if (dpt < I->lc()) maxs = std::max(maxs, pre ? I->pre[dpt] : I->post[dpt]);
     for (int s = 0; s < maxs; ++s) {
-      std::vector<Item> items;
+      std::vector<Item> items, pairs[2];
       for (Instance* I : S) {
         if (dpt >= I->lc()) continue;
         if (s >= (pre ? I->pre[dpt] : I->post[dpt])) continue;
         const int li = I->lev[dpt];
+        const DevLevel& d = hL[li];
+        // sweeps s and s+1 as a pair (an odd last sweep: half by half)
+        if (d.w && (s & 1 || s + 1 < (pre ? I->pre[dpt] : I->post[dpt]))) {
+          const RbPair rp = rb_pair(fp64, d.hx, d.ny, d.nz);
+          pairs[rp.tz == 2 ? 0 : 1].push_back({li, rp.blocks});
+          continue;
+        }
         items.push_back({li, blocks_smooth(hL[li])});
       }
       // from a zero initial guess: the red pass sees zero everywhere, the
@@ -854,6 +875,13 @@ void Context::vcycle(const std::vector<Instance*>& S, bool fp64) {
       const int dyn = (pre && dpt == 0 && !fp64 && any_pair) ? kZgDyn : 0;
       half(items, 0, (zero_first && s == 0) ? 3 | dyn : 0);
       half(items, 1, (zero_first && s == 0) ? 2 | dyn : 0);
+      for (int q = 0; q < 2; ++q)
+        for_lists(pairs[q], [&](const LaunchList& ll, int, int) {
+          int hx = 0;
+          for (int t = 0; t < ll.nitems; ++t) hx = std::max(hx, hL[ll.items[t]].hx);
+          launch_rb_pair(fp64, L, ll, (zero_first && s == 0) ? 3 | dyn : 0, s & 1, q == 0 ? 2 : 4, hx,
+                         stream);
+        });
     }
   };
   for (int dpt = 0; dpt < maxL0; ++dpt) {
