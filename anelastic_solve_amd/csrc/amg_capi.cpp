@@ -39,10 +39,10 @@ FlowGrid flow_grid(const Instance* I) {
   G.nz = F.nz;
   const Axis* ax[3] = {&F.ax, &F.ay, &F.az};
   for (int d = 0; d < 3; ++d) {
-    G.dxc[d] = ax[d]->dxc;
-    G.dxe[d] = ax[d]->dxe;
+    G.dxc[d] = ax[d]->dxc.data();
+    G.dxe[d] = ax[d]->dxe.data();
   }
-  G.rho = F.rho;
+  G.rho = F.rho.data();
   return G;
 }
 
@@ -462,7 +462,7 @@ int amg_cn_advance_device(amg_handle h, const double* veltemp1, double* veltemp2
   }
   const std::vector<double> table = cn_table(rows, G.nx, G.ny, rkdt);
   std::memcpy(h->h_cn, table.data(), sizeof(double) * table.size());
-  AMG_HIP(hipMemcpyAsync(h->d_cn, h->h_cn, sizeof(double) * table.size(), hipMemcpyHostToDevice, s));
+  launch_cn_table(h->h_cn, h->d_cn, (int)table.size(), s);
   const double *rho, *rdxc, *rdyc, *rdzc, *rdxe, *rdye, *rdze;
   metric_ptrs(h->I, &rho, &rdxc, &rdyc, &rdzc, &rdxe, &rdye, &rdze);
   launch_cn_column(veltemp1, veltemp2, p, h->d_cn, rdxe, rdye, G.nx, G.ny, G.nz, f1, f2, f3, rkdt, var,

@@ -12,11 +12,11 @@
 namespace amg {
 
 // Ghost-inclusive 1-D metrics of the finest grid (length n+2 per direction,
-// direction 0/1/2 = x/y/z) and rho(z).
+// direction 0/1/2 = x/y/z) and rho(z), as the instance's hierarchy holds them.
 struct FlowGrid {
   int nx = 0, ny = 0, nz = 0;
-  std::vector<double> dxc[3], dxe[3];
-  std::vector<double> rho;
+  const double *dxc[3], *dxe[3];
+  const double* rho;
 };
 
 // One face's bound_update rule with its products value*metric precomputed.
@@ -61,6 +61,8 @@ int plan_cn(const FlowGrid& G, int var, double rkdt, double rRe, double rPr, dou
 bool cn_segmented(int nx, int ny, int nz);
 std::vector<double> cn_table(const std::vector<CnRow>& rows, int nx, int ny, double rkdt);
 size_t cn_table_doubles(int nz);   // at most
+// n doubles of it from pinned host memory to the device.
+void launch_cn_table(const double* host, double* table, int n, hipStream_t s);
 void launch_cn_column(const double* v1, double* v2, const double* p, const double* T,
                       const double* rdxe, const double* rdye, int nx, int ny, int nz, double f1,
                       double f2, double f3, double rkdt, int var, hipStream_t s);

@@ -577,6 +577,14 @@ const VClass kClasses[] = {
     {"scal1temp", 8, 0, 1, 0, 0, 0, -1, 0},
 };
 
+// The step's table from pinned host memory: as a kernel it costs a launch; the
+// runtime's copy of the same few KB took the host and the stream 5 us more.
+__global__ __launch_bounds__(kFlowBlock) void k_cn_table(const double* __restrict__ host,
+                                                         double* __restrict__ table, int n) {
+  const int e = blockIdx.x * kFlowBlock + threadIdx.x;
+  if (e < n) table[e] = host[e];
+}
+
 }  // namespace
 
 int plan_ghost(const FlowGrid& G, const char* vtype, const amg_flowbc& bc, GhostPlan* out,
@@ -593,7 +601,7 @@ int plan_ghost(const FlowGrid& G, const char* vtype, const amg_flowbc& bc, Ghost
   const int n[3] = {G.nx, G.ny, G.nz};
   const int mk[3] = {c->mx, c->my, c->mz};
   for (int d = 0; d < 3; ++d) {
-    const std::vector<double>& dt = mk[d] ? G.dxc[d] : G.dxe[d];
+    const double* dt = mk[d] ? G.dxc[d] : G.dxe[d];
     const int l = c->l;
     auto TB = [&](int f) { return bc.tb[d + 3 * (f - 1) + 6 * (l - 1)]; };
     auto VB = [&](int f) { return bc.vb[d + 3 * (f - 1) + 6 * (l - 1)]; };
@@ -666,9 +674,9 @@ void launch_flow_ghost(double* const* a, const GhostPlan* P, int nf, int nx, int
 int plan_cn(const FlowGrid& G, int var, double rkdt, double rRe, double rPr, double rSc,
             const amg_flowbc& bc, std::vector<CnRow>* rows, std::string* err) {
   const int nz = G.nz;
-  const std::vector<double>& r = G.rho;
-  const std::vector<double>& dzc = G.dxc[2];
-  const std::vector<double>& dze = G.dxe[2];
+  const double* r = G.rho;
+  const double* dzc = G.dxc[2];
+  const double* dze = G.dxe[2];
   if (var != 1 && var != 2 && var != 3 && var != 5 && var != 8) {
     *err = "ABORTING ADVANCE CN, VARID IS NOT VALID";
     return -1;
@@ -856,6 +864,10 @@ std::vector<double> cn_table(const std::vector<CnRow>& rows, int nx, int ny, dou
   }
   t.insert(t.end(), back.begin(), back.end());
   return t;
+}
+
+void launch_cn_table(const double* host, double* table, int n, hipStream_t s) {
+  hipLaunchKernelGGL(k_cn_table, dim3(cdiv(n, kFlowBlock)), dim3(kFlowBlock), 0, s, host, table, n);
 }
 
 void launch_cn_column(const double* v1, double* v2, const double* p, const double* T,

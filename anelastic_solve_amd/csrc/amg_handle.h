@@ -24,8 +24,8 @@ void metric_ptrs(const Instance* I, const double** rho, const double** rdxc, con
                  const double** rdze);
 
 // The divergence report of dns/Routines.F90:123-173 with its block
-// partials and results in `partial` (4 * divergence_blocks + 4 doubles on
-// the handle's device); synchronous.
+// partials in `partial` (kDivVals * divergence_blocks doubles on the handle's
+// device); synchronous.
 int divergence_report(amg_handle h, const double* U, const double* V, const double* W,
                       double* div, double* partial, double* avg, double* maxabs, int loc[3]);
 

@@ -83,7 +83,8 @@ def _is_torch(x):
 
 
 def _dev_ptr(t, grid_shape, name):
-    if tuple(t.shape) != tuple(grid_shape) or not t.is_contiguous() or str(t.dtype) != "torch.float64":
+    import torch
+    if tuple(t.shape) != tuple(grid_shape) or not t.is_contiguous() or t.dtype != torch.float64:
         raise ValueError(f"{name}: need a contiguous float64 tensor of shape {grid_shape}")
     if not t.is_cuda:
         raise ValueError(f"{name}: expected a device tensor")
