@@ -202,13 +202,24 @@ struct Nb {
   int c, xm, xp, ym, yp, zm, zp;
 };
 
+// The planes a cell of plane k is coupled to.  Past a wall the coupling is
+// zero, but what it multiplies has to be finite: a plane in which the column's
+// cell has the other colour, so that a half-sweep from zero reads what the
+// half-sweep before it wrote.  nz - 1 and 0 are that for an even nz; for an
+// odd one (walls on both sides) it is the plane next to the wall.
+__device__ __forceinline__ int z_below(int k, int nz) {
+  return k > 0 ? k - 1 : (nz & 1) ? min(1, nz - 1) : nz - 1;
+}
+__device__ __forceinline__ int z_above(int k, int nz) {
+  return k < nz - 1 ? k + 1 : (nz & 1) ? max(nz - 2, 0) : 0;
+}
 __device__ __forceinline__ Nb neighbours(const LevelHead& L, int i, int j, int k) {
   const int hx = L.hx, ny = L.ny, nz = L.nz;
   const int col = (i + j) & 1, oth = col ^ 1, m = i >> 1, r = i & 1;
   int ml = m - 1 + r; if (ml < 0) ml = hx - 1;
   int mr = m + r;     if (mr >= hx) mr = 0;
   const int jm = (j == 0) ? ny - 1 : j - 1, jp = (j == ny - 1) ? 0 : j + 1;
-  const int km = (k == 0) ? nz - 1 : k - 1, kp = (k == nz - 1) ? 0 : k + 1;
+  const int km = z_below(k, nz), kp = z_above(k, nz);
   Nb n;
   n.c = cidx(m, j, k, col, hx, ny);
   const int ro = cidx(0, j, k, oth, hx, ny);
@@ -375,13 +386,13 @@ __global__ __launch_bounds__(kBlock) void k_rb_march(const DevLevel* __restrict_
       xr[s] = u[at(k, o, j, mr[h])];
       ys[s] = u[at(k, o, jm, m)];
       yn[s] = u[at(k, o, jp, m)];
-      zp[s] = u[at(k == nz - 1 ? 0 : k + 1, h, j, m)];
+      zp[s] = u[at(z_above(k, nz), h, j, m)];
     }
   }
   if (nbr) {
     // below the slab's first two planes
     const int h0 = (parity + k0) & 1;
-    zm01[0] = u[at(k0 == 0 ? nz - 1 : k0 - 1, h0, j, m)];
+    zm01[0] = u[at(z_below(k0, nz), h0, j, m)];
     zm01[1] = u[at(k0, h0 ^ 1, j, m)];
   }
 #pragma unroll
@@ -461,9 +472,22 @@ __global__ __launch_bounds__(1024) void k_rb_pair(const DevLevel* __restrict__ L
   const T dxx[2] = {co[2 * nx + 2 * m + b0], co[2 * nx + 2 * m + b1]};
   const T wys = cy[j], wyn = cy[ny + j], dyy = cy[2 * ny + j];
   auto at = [&](int k, int h, int jj, int q) { return ((k * ny + jj) * 2 + h) * hx + q; };
-  // red plane s of the march is plane k0 - 1 + s, black plane s k0 + s; the
-  // half of a plane is its number's (k0 is even)
-  auto plane = [&](int s) { return wrap(k0 - 1 + s, nz); };
+  // red plane s of the march is plane k0 - 1 + s = pk[s + 1], black plane s
+  // k0 + s; the half of a plane is its number's (k0 is even).  Planes outside
+  // are wrapped, or with an odd nz (walls) mirrored: of the same half either
+  // way, as z_below.
+  constexpr int NR = TZ + 2;
+  int pk[NR + 2];
+#pragma unroll
+  for (int t = 0; t < NR + 2; ++t) pk[t] = k0 - 2 + t;
+  if (k0 == 0 || k0 + TZ + 1 >= nz) {
+    const bool odd = nz & 1;
+#pragma unroll
+    for (int t = 0; t < NR + 2; ++t) {
+      const int k = pk[t], lo = odd ? -k : k + nz, hi = odd ? max(2 * (nz - 1) - k, 0) : k - nz;
+      pk[t] = k < 0 ? lo : k < nz ? k : hi;
+    }
+  }
   auto value = [&](int h, T fv, T zm_, T zp_, T zd, T xl, T xr, T ys, T yn, T zm, T zp) {
     const T d = (zd + dyy) + dxx[h];
     T a = wxl[h] * xl + wxr[h] * xr;
@@ -473,15 +497,12 @@ __global__ __launch_bounds__(1024) void k_rb_pair(const DevLevel* __restrict__ L
     a += zp_ * zp;
     return over(fv - a, d);
   };
-  constexpr int NR = TZ + 2;
   T wzm[NR], wzp[NR], dzz[NR];
   T fv[NR], xl[NR], xr[NR], ys[NR], yn[NR], zc[NR + 2], fb[TZ];
-  // (behind a wall of an odd nz the far plane counts as the number the march
-  // gives it: whatever half that names meets a zero coupling)
   auto hr = [](int s) { return (s + 1) & 1; };   // half of red plane s
 #pragma unroll
   for (int s = 0; s < NR; ++s) {
-    const int k = plane(s);
+    const int k = pk[s + 1];
     wzm[s] = cz[k];
     wzp[s] = cz[nz + k];
     dzz[s] = cz[2 * nz + k];
@@ -489,19 +510,19 @@ __global__ __launch_bounds__(1024) void k_rb_pair(const DevLevel* __restrict__ L
   if (act) {
 #pragma unroll
     for (int s = 0; s < NR; ++s) {
-      const int k = plane(s), h = hr(s);
+      const int k = pk[s + 1], h = hr(s);
       fv[s] = f[at(k, h, j, m)];
       if (nbr) {
         xl[s] = ub[at(k, h ^ 1, j, ml[h])];
         xr[s] = ub[at(k, h ^ 1, j, mr[h])];
         ys[s] = ub[at(k, h ^ 1, jm, m)];
         yn[s] = ub[at(k, h ^ 1, jp, m)];
-        zc[s + 2] = ub[at(wrap(k + 1, nz), h, j, m)];
+        zc[s + 2] = ub[at(pk[s + 2], h, j, m)];
       }
     }
     if (nbr) {
-      zc[0] = ub[at(wrap(plane(0) - 1, nz), hr(0), j, m)];
-      zc[1] = ub[at(plane(0), hr(1), j, m)];
+      zc[0] = ub[at(pk[0], hr(0), j, m)];
+      zc[1] = ub[at(pk[1], hr(1), j, m)];
     }
     if (own) {
 #pragma unroll

@@ -572,13 +572,7 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
     DevLevel& d = newL[l];
     if (std::max(I->pre[l], I->post[l]) < 2 || !rb_pair(I->fp64, d.hx, d.ny, d.nz).tz) continue;
     d.w = I->mem.alloc((size_t)d.ncell * w);
-    if (!d.w) {
-      (void)hipGetLastError();
-      continue;
-    }
-    // its red cells stay zero: with an odd nz a sweep reads some (the far
-    // side of a wall, times a zero coupling)
-    launch_zero((double*)d.w, (int)((size_t)d.ncell * w / sizeof(double)), stream);
+    if (!d.w) (void)hipGetLastError();
   }
   // projection metrics
   {
