@@ -490,6 +490,7 @@ int amg_batch_create(int n, const amg_config* cfg, const amg_grid* grids, amg_ba
   amg_batch_s* b = new amg_batch_s();
   amg_config c = *cfg;
   c.use_graph = 0;
+  b->ctx.many = n > 1;
   int rc = b->ctx.init(c);
   for (int i = 0; i < n && rc == AMG_OK; ++i) {
     Instance* I = nullptr;

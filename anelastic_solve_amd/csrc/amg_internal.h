@@ -55,6 +55,7 @@ struct DevLevel : LevelHead {
   int nullsp;                // the operator is singular (periodic/Neumann): constants in the null space
   int pairok;                // the instance may pair cycles (mixed, residual stop rule)
   int gslot;                 // the instance's slot in the per-instance gate array
+  int mk;                    // planes of a slab of the finest-level stencil kernels
   unsigned mhx, mny;         // ceil(2^32/hx), ceil(2^32/ny) (0 for a divisor of 1): e/hx = umulhi(e, mhx)
                              // exactly while e*hx < 2^32 (the coarse tail's small levels)
   void* w;                   // the black cells between two paired point sweeps (rb_pair), or null
@@ -386,14 +387,13 @@ size_t tail_lds_limit();
 //                   of 'link', with b' = b - bshift; {max|r|, max|e|, max|u2|}
 constexpr int kFinePer = 8;
 // The FP64 finest-level stencil kernels (residual, defect, correct+defect)
-// march in z over slabs of kMarchK planes: blocks per item =
-// cdiv(2*hx*ny, kBlock) * cdiv(nz, kMarchK), one partial per block.
-#ifndef AMG_MARCHK
-#define AMG_MARCHK 16
-#endif
-constexpr int kMarchK = AMG_MARCHK;
-inline long long march_blocks(int hx, int ny, int nz) {
-  return ((2LL * hx * ny + kBlock - 1) / kBlock) * ((nz + kMarchK - 1) / kMarchK);
+// march in z over slabs of DevLevel::mk planes: blocks per item =
+// cdiv(2*hx*ny, kBlock) * cdiv(nz, planes), one partial per block.  A slab is
+// kMarchK planes, of a level solved by itself march_planes().
+constexpr int kMarchK = 16;
+int march_planes(int hx, int ny, int nz);
+inline long long march_blocks(int hx, int ny, int nz, int planes) {
+  return ((2LL * hx * ny + kBlock - 1) / kBlock) * ((nz + planes - 1) / planes);
 }
 void launch_residual_max(const DevLevel* L, const LaunchList& ll, double* partial, hipStream_t s);
 void launch_change_max(const DevLevel* L, const LaunchList& ll, double* partial, hipStream_t s);
@@ -443,7 +443,7 @@ void launch_finalize(const LaunchList& ll, const double* partial, int nvals, int
 // per item in 'ptr') and the FP64 finest level.
 // from_fortran: dst = (which==0 ? u : f) = src interior (+ bcfold if add_fold)
 // wsum:         {sum V x} (x = u or f), or {sum V rho} when which == 2;
-//               march_blocks per item (z slabs of kMarchK planes)
+//               march_blocks per item of kMarchK planes
 // to_fortran:   dst interior = u, or u - (c[item]/vrsum) rho(z) for singular
 //               items when c is given (c: the sums of launch_wsum)
 // ingest:       f = rhs interior + bcfold, u = phi interior, and one partial

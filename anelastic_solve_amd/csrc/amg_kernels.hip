@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstddef>
+#include <type_traits>
 
 namespace amg {
 namespace {
@@ -2285,7 +2286,7 @@ __global__ __launch_bounds__(kBlock) void k_change_max(const DevLevel* __restric
 }
 
 // FP64 finest-level stencil kernels, marching in z.  A thread owns one
-// position col = (j*2 + colour)*hx + m of a plane and walks kMarchK planes,
+// position col = (j*2 + colour)*hx + m of a plane and walks D.mk planes,
 // keeping the centre values at k-1, k, k+1 in registers: every value of the
 // iterate is read from memory once per slab (plus one halo plane at each
 // slab end), the four in-plane neighbours come from the cache, and the
@@ -2367,13 +2368,14 @@ __device__ __forceinline__ void fine_march(sp<kG, const double> __restrict__ u,
   auto step = [&](int k, const Plane& cur) {
     const int pbk = k * plane;
     const double vp = sum(cur.pu, cur.pe);
-    double s = wxm * sum(cur.xm, cur.xme) + wxp * sum(cur.xp, cur.xpe);
-    s += wym * sum(cur.ym, cur.yme);
-    s += wyp * sum(cur.yp, cur.ype);
-    s += cz[k] * vm;
-    s += cz[nz + k] * vp;
+    // explicit fma: a residual is the same bits whatever slab it is in
+    double s = fm(wxp, sum(cur.xp, cur.xpe), wxm * sum(cur.xm, cur.xme));
+    s = fm(wym, sum(cur.ym, cur.yme), s);
+    s = fm(wyp, sum(cur.yp, cur.ype), s);
+    s = fm(cz[k], vm, s);
+    s = fm(cz[nz + k], vp, s);
     const double diag = (cz[2 * nz + k] + dxy_y) + dxy_x;
-    const double res = cur.fb - (s + diag * vc);
+    const double res = cur.fb - fm(diag, vc, s);
     // the shifted b (FP64: the V-cycle's finest right-hand side) and the
     // FP32 defect are read by later kernels only
     if constexpr (SHIFT && MODE == kResMax) st_row_nt<double>(f + pbk, dc, cur.fb);
@@ -2404,20 +2406,28 @@ __device__ __forceinline__ void fine_march(sp<kG, const double> __restrict__ u,
   // no register copies at a loop back edge (they would wait for the loads in
   // flight) and no load is sunk past a branch toward its use.
   constexpr int D = kFineDepth;
-  if (k1 - k0 == kMarchK) {
+  auto slab = [&](auto planes) {
+    constexpr int K = decltype(planes)::value;
     Plane R[D];
 #pragma unroll
     for (int s = 0; s < D - 1; ++s) R[s] = load(k0 + s);
 #pragma unroll
-    for (int s = 0; s < kMarchK; ++s) {
-      if (s + D - 1 < kMarchK) R[(s + D - 1) % D] = load(k0 + s + D - 1);
+    for (int s = 0; s < K; ++s) {
+      if (s + D - 1 < K) R[(s + D - 1) % D] = load(k0 + s + D - 1);
       // keep the prefetch ahead of the arithmetic: the scheduler would
       // otherwise move the loads toward their use
       __builtin_amdgcn_sched_barrier(0);
       step(k0 + s, R[s % D]);
     }
+  };
+  if (k1 - k0 == kMarchK) {
+    slab(std::integral_constant<int, kMarchK>());
+  } else if (k1 - k0 == 4) {
+    slab(std::integral_constant<int, 4>());
+  } else if (k1 - k0 == 2) {
+    slab(std::integral_constant<int, 2>());
   } else {
-    // the short last slab when nz is not a multiple of kMarchK
+    // other lengths: a short last slab
     Plane a = load(k0);
     for (int k = k0; k < k1; ++k) {
       const Plane n = load(min(k + 1, k1 - 1));
@@ -2443,8 +2453,8 @@ __global__ __launch_bounds__(kBlock) void k_fine(DevLevel* __restrict__ Lt, LIST
   const float* e32 = D.e32;
   float* r32 = D.r32;
   double bshift = D.bshift, vsum = D.vsum;
-  int nullsp = D.nullsp;
-  pin_s(e32, r32, bshift, vsum, nullsp);
+  int nullsp = D.nullsp, mk = D.mk;
+  pin_s(e32, r32, bshift, vsum, nullsp, mk);
   const LevelHead L = level_head(D);
   if (level_off(L)) return;
   // the first cycle of a pair: no correction (its gate reads no norms)
@@ -2458,7 +2468,7 @@ __global__ __launch_bounds__(kBlock) void k_fine(DevLevel* __restrict__ Lt, LIST
   const int lb = wk.lb;
   const int bk = lb / ncb, bc = lb - bk * ncb;
   const int col = bc * kBlock + threadIdx.x;
-  const int k0 = bk * kMarchK, k1 = min(k0 + kMarchK, nz);
+  const int k0 = bk * mk, k1 = min(k0 + mk, nz);
   double v[NV];
 #pragma unroll
   for (int q = 0; q < NV; ++q) v[q] = 0.0;
@@ -3742,6 +3752,17 @@ size_t tail_lds_limit() {
   return limit;
 }
 // (k_fine takes the table writable: the mixed first defect records bshift)
+int march_planes(int hx, int ny, int nz) {
+  // Slabs of 16 planes re-read the fewest planes; where they make fewer
+  // workgroups than the device has CUs, shorter ones (a 64^3 residual has 64
+  // workgroups of 16 planes: FP64 solve 4170 us, with 256 of four 3977;
+  // 64x48x32 673 -> 655).  Past that, shorter slabs lose (256x64x256, 1024
+  // workgroups of 16: 774 us, of four 808; 20 solves of up to 64x64x64 in the
+  // same launches 3720, each with its own rule 3990).
+  for (int K : {kMarchK, 4})
+    if (march_blocks(hx, ny, nz, K) >= device_cus()) return K;
+  return 2;
+}
 void launch_residual_max(const DevLevel* L, const LaunchList& ll, double* partial, hipStream_t s) {
   LAUNCH((k_fine<kResMax, false>), ll.nblocks, kBlock, const_cast<DevLevel*>(L), LIST_ARGS(ll), nullptr,
          partial, ll);

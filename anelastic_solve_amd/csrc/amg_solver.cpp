@@ -74,7 +74,7 @@ void DevArena::release() {
 size_t partial_blocks(const Instance& I) {
   const HostLevel& F = I.H.lv[0];
   const long long n = F.ncell();
-  long long b = march_blocks(F.nx / 2, F.ny, F.nz);
+  long long b = march_blocks(F.nx / 2, F.ny, F.nz, march_planes(F.nx / 2, F.ny, F.nz));
   b = std::max(b, (long long)cdiv(n, (long long)kBlock * kFinePer));
   b = std::max(b, (long long)cdiv(n, (long long)kBlock * kWsumPer));
   b = std::max(b, (long long)cdiv(n, kBlock));
@@ -309,6 +309,7 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
     d.inst = I->id;
     d.gslot = I->gslot;
     d.ncell = (int)H.ncell();
+    d.mk = many ? kMarchK : march_planes(d.hx, d.ny, d.nz);
     d.link = -1;
     d.bcx0 = I->H.bc[0][0]; d.bcx1 = I->H.bc[0][1];
     d.bcy0 = I->H.bc[1][0]; d.bcy1 = I->H.bc[1][1];
@@ -993,7 +994,7 @@ std::vector<Item> march_items(const Context& C, const std::vector<Instance*>& S,
   for (Instance* I : S) {
     const int li = current ? I->fine[I->cur] : I->fine[0];
     const DevLevel& d = C.hL[li];
-    items.push_back({li, (int)march_blocks(d.hx, d.ny, d.nz)});
+    items.push_back({li, (int)march_blocks(d.hx, d.ny, d.nz, d.mk)});
   }
   return items;
 }
@@ -1101,7 +1102,7 @@ const double* Context::null_sums(const std::vector<Instance*>& S) {
   for (Instance* I : S) {
     any = any || I->H.singular;
     const int li = I->fine[0];   // the device's pcur picks the current buffer
-    sums.push_back({li, (int)march_blocks(hL[li].hx, hL[li].ny, hL[li].nz)});
+    sums.push_back({li, (int)march_blocks(hL[li].hx, hL[li].ny, hL[li].nz, kMarchK)});
   }
   if (!any) return nullptr;
   double* c = d_out + kOutRegion * 3;
@@ -1441,7 +1442,7 @@ int Context::run_kernel(Instance* I, int which, int level, int reps, double* byt
     if (r222) which = which == 16 ? 17 : 9;   // the z-march restriction (17: with rskip)
   } else if (which == 3) {
     const DevLevel& fd = hL[I->fine[I->cur]];
-    items.push_back({I->fine[I->cur], (int)march_blocks(fd.hx, fd.ny, fd.nz)});
+    items.push_back({I->fine[I->cur], (int)march_blocks(fd.hx, fd.ny, fd.nz, fd.mk)});
     b = fp64 ? 16.0 * d.ncell : 32.0 * d.ncell;
   } else if (which == 7 || which == 8) {
     if (!zline || d.nz > (fp64 ? kTailNz64 : kTailNz)) {

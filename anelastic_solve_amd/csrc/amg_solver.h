@@ -110,6 +110,7 @@ struct Context {
   hipGraphExec_t gchain[3] = {};
   void drop_graphs();
   bool graph_ok = true;
+  bool many = false;             // launches hold many instances (set before the first is added)
 
   int init(const amg_config& c);
   ~Context();

@@ -25,6 +25,7 @@ CASES = [
     ((64, 42, 34), WALLS, (6, 2, 2), 2, 2),                 # two rows and two planes left over
     ((64, 60, 21), WALLS, (6, 3, 1), 3, 2),                 # odd nz; a single sweep after the pair
     ((48, 72, 56), PERIODIC_XY, (4, 3, 4), 1, 4),           # no pair before, two after
+    ((128, 64, 38), WALLS, (6, 4, 2), 2, 2),                # the residual's slabs of 4 planes, 2 left over
     ((336, 32, 40), WALLS, (4, 4, 4), 2, 3),                # hx = 168
     ((352, 32, 40), WALLS, (5, 4, 4), 2, 2),                # hx = 176: the finest level unpaired
 ]
