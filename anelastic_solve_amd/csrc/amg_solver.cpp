@@ -420,7 +420,8 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
     if (I->post[l] >= 1 && x.fx == 2 && x.fy == 2 && x.fz == 2)
       x.skip = !line ? kXferSkipPoint : ents[l].pz ? kXferSkipLineWrap : kXferSkipLine;
     x.rskip = kXferSkipNone;
-    if (I->pre[l] >= 1 && restrict222_ok(ents[l], ents[l + 1], x) && !(line && ents[l].pz))
+    if (I->pre[l] >= 1 && (restrict222_ok(ents[l], ents[l + 1], x) || restrict_quad_ok(ents[l + 1], x)) &&
+        !(line && ents[l].pz))
       x.rskip = line ? kXferSkipLine : kXferSkipPoint;
     x.pmx = gm_magic((unsigned)prolong_duals_dir(ents[l + 1].nx, x.fx, ents[l].px), &x.psx);
     x.pmy = gm_magic((unsigned)prolong_duals_dir(ents[l + 1].ny, x.fy, ents[l].py), &x.psy);
@@ -887,18 +888,22 @@ void Context::vcycle(const std::vector<Instance*>& S, bool fp64) {
         zero.push_back({I->lev[dpt], cdiv(hL[I->lev[dpt]].ncell, kBlock)});
     for_lists(zero, [&](const LaunchList& ll, int, int) { launch_fill_zero(fp64, L, ll, stream); });
     smooth(dpt, true, zero_first);
-    std::vector<Item> items, items222;
+    std::vector<Item> items, quads, items222;
     for (Instance* I : S) {
       if (dpt >= I->lc()) continue;
       const int xi = I->xf[dpt];
       const DevLevel& C = hL[I->lev[dpt + 1]];
       if (restrict222_ok(hL[I->lev[dpt]], C, hX[xi])) items222.push_back({xi, restrict222_blocks(C)});
+      else if (restrict_quad_ok(C, hX[xi])) quads.push_back({xi, restrict_quad_blocks(C)});
       else items.push_back({xi, cdiv(C.ncell, kBlock)});
     }
     // the residuals the pre-smoothing's last half-sweep solved are taken as
     // zero (DevXfer::rskip)
     for_lists(items222, [&](const LaunchList& ll, int, int) {
       launch_restrict222(fp64, L, dX, ll, stream, true);
+    });
+    for_lists(quads, [&](const LaunchList& ll, int, int) {
+      launch_restrict_quad(fp64, L, dX, ll, stream, true);
     });
     for_lists(items, [&](const LaunchList& ll, int, int) {
       launch_restrict(fp64, L, dX, ll, stream);
@@ -1411,6 +1416,7 @@ int Context::run_kernel(Instance* I, int which, int level, int reps, double* byt
   std::vector<Item> items;
   double b = 0.0;
   int form = 0;
+  bool quad = false;
   if (which >= 10 && which <= 13) {
     // the z-line half-sweep in a given form: 10/11 short, 12/13 lean (red/black)
     if (!zline || (fp64 && which < 12)) {
@@ -1433,11 +1439,13 @@ int Context::run_kernel(Instance* I, int which, int level, int reps, double* byt
     const DevXfer& xf = hX[I->xf[level]];
     const bool restr = which == 1 || which == 16;
     const bool r222 = restr && restrict222_ok(d, c, xf);
+    quad = restr && !r222 && restrict_quad_ok(c, xf);
     const int nc = restr ? c.ncell : prolong_duals(d, c, xf);
-    items.push_back({I->xf[level], r222 ? restrict222_blocks(c) : cdiv(nc, kBlock)});
+    items.push_back({I->xf[level], r222 ? restrict222_blocks(c)
+                                  : quad ? restrict_quad_blocks(c) : cdiv(nc, kBlock)});
     double fine = 2.0;
     if (which == 15 && xf.skip != kXferSkipNone) fine = 1.0;
-    if (which == 16 && r222 && xf.rskip != kXferSkipNone) fine = 1.5;
+    if (which == 16 && (r222 || quad) && xf.rskip != kXferSkipNone) fine = 1.5;
     b = (fine + 0.125) * w * d.ncell;
     if (r222) which = which == 16 ? 17 : 9;   // the z-march restriction (17: with rskip)
   } else if (which == 3) {
@@ -1482,6 +1490,8 @@ int Context::run_kernel(Instance* I, int which, int level, int reps, double* byt
         else rb_launches(items, fp64, par, zg);
       } else if (which == 7 || which == 8) {
         launch_zline_col(fp64, dL, ll, which == 8 ? 1 : 0, 0, stream);
+      } else if ((which == 1 || which == 16) && quad) {
+        launch_restrict_quad(fp64, dL, dX, ll, stream, which == 16);
       } else if (which == 1 || which == 16) {
         launch_restrict(fp64, dL, dX, ll, stream);
       } else if (which == 9 || which == 17) {
