@@ -3082,11 +3082,13 @@ __global__ __launch_bounds__(kBlock) void k_ghost_fill(double* __restrict__ a, i
 // Projection step (dns/NSsolver.F90:2204-2219, :2057-2082; dns/Routines.F90:123-144).
 //
 // The source and the divergence march in z: a thread owns one position of a
-// plane and kProjK planes, so W below a plane is the value it has just used
-// (with one cell per thread the plane below was read by another XCD, a second
-// time from memory) and the position is divided once per slab.  Bound by
+// plane and kProjK planes (the source of a small grid two), so W below a
+// plane is the value it has just used (with one cell per thread the plane
+// below was read by another XCD, a second time from memory) and the position
+// is divided once per slab.  Bound by
 // memory: at 512x256x256 the source takes 216 us (271 with one cell per
 // thread) for 1.09 GB.
+template <int K>
 __global__ __launch_bounds__(kBlock) void k_psource(const double* __restrict__ U,
                                                     const double* __restrict__ V,
                                                     const double* __restrict__ W,
@@ -3102,13 +3104,13 @@ __global__ __launch_bounds__(kBlock) void k_psource(const double* __restrict__ U
   if (pos >= sxy) return;
   const int j = pos / sx, i = pos - j * sx;
   const bool in = i > 0 && j > 0 && i <= nx && j <= ny;
-  const int k0 = bk * kProjK, ic = in ? i : 1, jc = in ? j : 1;
+  const int k0 = bk * K, ic = in ? i : 1, jc = in ? j : 1;
   const size_t c0 = (size_t)jc * sx + ic;               // a ghost column reads the first interior one
   const double rx = rdxc[ic], ry = rdyc[jc];
-  double u[kProjK], um[kProjK], v[kProjK], vm[kProjK], w[kProjK + 1];
+  double u[K], um[K], v[K], vm[K], w[K + 1];
   w[0] = W[(size_t)max(k0 - 1, 0) * sxy + c0];
 #pragma unroll
-  for (int q = 0; q < kProjK; ++q) {
+  for (int q = 0; q < K; ++q) {
     const size_t e = (size_t)min(k0 + q, nz + 1) * sxy + c0;
     u[q] = U[e];
     um[q] = U[e - 1];
@@ -3117,7 +3119,7 @@ __global__ __launch_bounds__(kBlock) void k_psource(const double* __restrict__ U
     w[q + 1] = W[e];
   }
 #pragma unroll
-  for (int q = 0; q < kProjK; ++q) {
+  for (int q = 0; q < K; ++q) {
     const int k = k0 + q;
     if (k > nz + 1) break;
     double r = 0.0;
@@ -3901,8 +3903,15 @@ void launch_ghost_fill(double* a, int nx, int ny, int nz, const GhostBC& bc, hip
 void launch_psource(const double* U, const double* V, const double* W, double* SRC, const double* rho,
                     const double* rdxc, const double* rdyc, const double* rdzc, int nx, int ny, int nz,
                     double rdt, hipStream_t s) {
-  LAUNCH(k_psource, nb((size_t)(nx + 2) * (ny + 2)) * nb(nz + 2, kProjK), kBlock, U, V, W, SRC, rho,
-         rdxc, rdyc, rdzc, nx, ny, nz, rdt);
+  const unsigned plane = nb((size_t)(nx + 2) * (ny + 2));
+  // Slabs of kProjK planes where they fill the device several times over;
+  // smaller grids are bound by a thread's chain and take two planes (call at
+  // 64x48x32 20.9 -> 19.6 us, 160x112x80 27.0 -> 25.6; 256^3 123.5 against
+  // 130.2 with two).
+  const bool full = plane * nb(nz + 2, kProjK) >= 4096;
+  const unsigned blocks = plane * nb(nz + 2, full ? kProjK : 2);
+  if (full) LAUNCH(k_psource<kProjK>, blocks, kBlock, U, V, W, SRC, rho, rdxc, rdyc, rdzc, nx, ny, nz, rdt);
+  else LAUNCH(k_psource<2>, blocks, kBlock, U, V, W, SRC, rho, rdxc, rdyc, rdzc, nx, ny, nz, rdt);
 }
 void launch_pgrad(const double* p, double* U, double* V, double* W, const double* rho,
                   const double* rdxe, const double* rdye, const double* rdze, int nx, int ny, int nz,
