@@ -568,13 +568,22 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
       break;
     }
   }
-  // point sweeps in pairs on the levels cycled by launches (without the
-  // buffer a level's half-sweeps run one by one)
-  for (int l = 0; cfg.smoother != AMG_SMOOTHER_LJ && l < I->lc(); ++l) {
-    DevLevel& d = newL[l];
-    if (std::max(I->pre[l], I->post[l]) < 2 || !rb_pair(I->fp64, d.hx, d.ny, d.nz).tz) continue;
-    d.w = I->mem.alloc((size_t)d.ncell * w);
-    if (!d.w) (void)hipGetLastError();
+  // point sweeps in pairs on the levels cycled by launches: one buffer for all
+  // of them, of the largest's size (the first), as a level's pairs bring its
+  // black cells back before the next level's begin.  Without it the
+  // half-sweeps run one by one.
+  if (cfg.smoother != AMG_SMOOTHER_LJ) {
+    void* wb = nullptr;
+    for (int l = 0; l < I->lc(); ++l) {
+      DevLevel& d = newL[l];
+      if (std::max(I->pre[l], I->post[l]) < 2 || !rb_pair(I->fp64, d.hx, d.ny, d.nz).tz) continue;
+      if (!wb) wb = I->mem.alloc((size_t)d.ncell * w);
+      if (!wb) {
+        (void)hipGetLastError();
+        break;
+      }
+      d.w = wb;
+    }
   }
   // projection metrics
   {
