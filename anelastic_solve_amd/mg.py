@@ -82,9 +82,16 @@ def _is_torch(x):
     return type(x).__module__.startswith("torch")
 
 
+_FLOAT64 = None      # torch.float64, kept from the first tensor on
+
+
 def _dev_ptr(t, grid_shape, name):
-    import torch
-    if tuple(t.shape) != tuple(grid_shape) or not t.is_contiguous() or t.dtype != torch.float64:
+    global _FLOAT64
+    if _FLOAT64 is None:
+        import torch
+        _FLOAT64 = torch.float64
+    # 0.1 us; with an import statement in every call 0.23, a smallest psource 0.4 of its 19 us more
+    if t.dtype != _FLOAT64 or tuple(t.shape) != tuple(grid_shape) or not t.is_contiguous():
         raise ValueError(f"{name}: need a contiguous float64 tensor of shape {grid_shape}")
     if not t.is_cuda:
         raise ValueError(f"{name}: expected a device tensor")
