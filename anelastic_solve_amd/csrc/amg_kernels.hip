@@ -3082,8 +3082,8 @@ __global__ __launch_bounds__(kBlock) void k_ghost_fill(double* __restrict__ a, i
 // Projection step (dns/NSsolver.F90:2204-2219, :2057-2082; dns/Routines.F90:123-144).
 //
 // The source and the divergence march in z: a thread owns one position of a
-// plane and kProjK planes (the source of a small grid two), so W below a
-// plane is the value it has just used (with one cell per thread the plane
+// plane and kProjK planes (the source of a small grid two or one), so W below
+// a plane is the value it has just used (with one cell per thread the plane
 // below was read by another XCD, a second time from memory) and the position
 // is divided once per slab.  Bound by
 // memory: at 512x256x256 the source takes 216 us (271 with one cell per
@@ -3904,14 +3904,19 @@ void launch_psource(const double* U, const double* V, const double* W, double* S
                     const double* rdxc, const double* rdyc, const double* rdzc, int nx, int ny, int nz,
                     double rdt, hipStream_t s) {
   const unsigned plane = nb((size_t)(nx + 2) * (ny + 2));
-  // Slabs of kProjK planes where they fill the device several times over;
-  // smaller grids are bound by a thread's chain and take two planes (call at
-  // 64x48x32 20.9 -> 19.6 us, 160x112x80 27.0 -> 25.6; 256^3 123.5 against
-  // 130.2 with two).
-  const bool full = plane * nb(nz + 2, kProjK) >= 4096;
-  const unsigned blocks = plane * nb(nz + 2, full ? kProjK : 2);
-  if (full) LAUNCH(k_psource<kProjK>, blocks, kBlock, U, V, W, SRC, rho, rdxc, rdyc, rdzc, nx, ny, nz, rdt);
-  else LAUNCH(k_psource<2>, blocks, kBlock, U, V, W, SRC, rho, rdxc, rdyc, rdzc, nx, ny, nz, rdt);
+  // Slabs of kProjK planes where they fill the device several times over (256^3
+  // 123.5 us a call, with two planes 130.2).  Smaller grids are bound by a
+  // thread's chain and take two planes, or one up to four workgroups per CU.
+  // The kernel with one cell per thread and no march, with one plane, with two:
+  // 24x24x14 2.68, 2.64, 2.80 us; 128x24x46 (672 workgroups of one plane) 3.40,
+  // 3.24, 3.28; 96x96x64 (2508) 6.20, 5.32, 4.88; 160x112x80 11.96, 9.08, 8.64.
+  const int K = plane * nb(nz + 2, kProjK) >= 4096 ? kProjK : plane * (unsigned)(nz + 2) > 1024 ? 2 : 1;
+  const unsigned blocks = plane * nb(nz + 2, K);
+#define PS(K) LAUNCH(k_psource<K>, blocks, kBlock, U, V, W, SRC, rho, rdxc, rdyc, rdzc, nx, ny, nz, rdt)
+  if (K == kProjK) PS(kProjK);
+  else if (K == 2) PS(2);
+  else PS(1);
+#undef PS
 }
 void launch_pgrad(const double* p, double* U, double* V, double* W, const double* rho,
                   const double* rdxe, const double* rdye, const double* rdze, int nx, int ny, int nz,
