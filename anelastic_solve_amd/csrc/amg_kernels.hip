@@ -116,17 +116,23 @@ __device__ __forceinline__ int xcd_swizzle(int b, int n) {
   return x * q + min(x, rem) + idx;
 }
 
-// Reciprocal for the line solves: the hardware rcp (1 ulp) in FP32, a
-// correctly rounded division in FP64.
+// Reciprocal for the line solves: the hardware rcp (1 ulp) in FP32, 1.0 / x in
+// FP64: the hardware's 24-bit estimate, two Newton steps, which leave it within
+// 1 ulp, and a third, which then rounds it correctly (Markstein's theorem); the
+// fixup gives the special arguments what the division does.  It equals the
+// division in all of 1e11 arguments tried, random ones and the 2^34 significands
+// next to 1 and to 2 (two steps differ in 6 of the last), and in zeros,
+// infinities, NaN, subnormal arguments and subnormal results.
+//
+// A z-line sweep has a chain of kZSeg of them per segment.  Half-sweeps with
+// the division, with three steps, with two: 64^3 7.03, 6.87, 6.83 us, 128^3
+// 10.0, 9.64, 9.50, 256^3 44.4, 43.3, 43.0.
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-// FP64: the hardware's 24-bit estimate and two Newton steps, within 1 ulp
-// wherever x and its reciprocal are normal.  A z-line sweep has a chain of
-// kZSeg dependent reciprocals per segment: with the division in its place a
-// 64^3 half-sweep took 7.4 us instead of 6.8, a 128^3 one 10.1 instead of 9.5.
 __device__ __forceinline__ double rcp(double x) {
   double r = __builtin_amdgcn_rcp(x);
-  r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
-  return __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+  return __builtin_amdgcn_div_fixup(r, x, 1.0);
 }
 
 // Fused multiply-add a*b + c, written out where several kernels have to
