@@ -58,7 +58,8 @@ struct DevLevel : LevelHead {
   int mk;                    // planes of a slab of the finest-level stencil kernels
   unsigned mhx, mny;         // ceil(2^32/hx), ceil(2^32/ny) (0 for a divisor of 1): e/hx = umulhi(e, mhx)
                              // exactly while e*hx < 2^32 (the coarse tail's small levels)
-  void* w;                   // the black cells between two paired point sweeps (rb_pair), or null
+  void* w[2];                // the black cells between two paired point sweeps (rb_pair) while
+                             // pcur is 0, 1, or null
   int bcx0, bcx1, bcy0, bcy1, bcz0, bcz1;   // boundary codes (prolongation ghosts)
   double vsum;               // finest: sum of cell volumes
   double vrsum;              // finest: sum of V*rho
@@ -267,7 +268,7 @@ inline int rb_march_planes(int hx, int ny, int nz) {
     if (nz >= K && (long long)hx * ny * ((nz + K - 1) / K) >= (1 << 18)) return K;
   return 0;
 }
-// Whole point sweeps (red, then black) of levels with a buffer w for the
+// Whole point sweeps (red, then black) of levels with buffers w for the
 // black cells, in pairs: back 0 leaves the black cells in w, back 1 brings
 // them back to u.  rb_pair: whether a level's sweeps run so, as slabs of tz
 // planes (0: they do not) in `blocks` blocks; every item of a launch has that

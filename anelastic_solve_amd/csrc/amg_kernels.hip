@@ -451,10 +451,11 @@ __global__ __launch_bounds__(1024) void k_rb_pair(const DevLevel* __restrict__ L
   const sp<kS, T> red = (sp<kS, T>)(sp<kS, unsigned char>)lds_raw;
   const Work wk = work_item(ln, lnb, li0, ll);
   const DevLevel& D = Lt[wk.idx];
-  void* wp = D.w;
-  pin_s(wp);
+  void *w0 = D.w[0], *w1 = D.w[1];
+  pin_s(w0, w1);
   const LevelHead L = level_head(D);
   if (level_off(L)) return;
+  void* const wp = L.pcur ? w1 : w0;
   const bool nbr = !(zero_flags(L, zero_guess) & 1);
   const int hx = L.hx, ny = L.ny, nz = L.nz, nx = L.nx;
   const int nty = (ny + TY - 1) / TY;

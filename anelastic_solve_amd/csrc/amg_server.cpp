@@ -355,6 +355,7 @@ int amg_server_create(const amg_config* cfg, double hbm_budget_bytes, int max_sl
   c.use_graph = 0;
   c.verbose = 0;
   s->ctx.many = true;
+  s->ctx.budgeted = true;
   const int rc = s->ctx.init(c);
   if (rc != AMG_OK) {
     delete s;

@@ -568,21 +568,27 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
       break;
     }
   }
-  // point sweeps in pairs on the levels cycled by launches: one buffer for all
-  // of them, of the largest's size (the first), as a level's pairs bring its
-  // black cells back before the next level's begin.  Without it the
-  // half-sweeps run one by one.
+  // point sweeps in pairs on the levels cycled by launches.  A level's pairs
+  // bring its black cells back before the next level's begin, so one buffer
+  // does for all, and a V-cycle leaves an FP64 field of the finest level idle:
+  // of a mixed solve the pressure buffer that its next correction writes, of an
+  // FP64 one the previous iterate -- unless the solve reports relmax, which
+  // compares with it.  Then the buffer is the instance's own, or where the
+  // memory is budgeted there is none and the half-sweeps run one by one.
   if (cfg.smoother != AMG_SMOOTHER_LJ) {
-    void* wb = nullptr;
+    void* own[2] = {fA.u2, I->fp64 ? fA.u2 : fA.u};
+    const bool taken = I->fp64 && cfg.report_relmax;
+    if (taken) own[0] = own[1] = nullptr;
     for (int l = 0; l < I->lc(); ++l) {
       DevLevel& d = newL[l];
       if (std::max(I->pre[l], I->post[l]) < 2 || !rb_pair(I->fp64, d.hx, d.ny, d.nz).tz) continue;
-      if (!wb) wb = I->mem.alloc((size_t)d.ncell * w);
-      if (!wb) {
-        (void)hipGetLastError();
-        break;
+      if (taken && !own[0] && !budgeted) {
+        own[0] = own[1] = I->mem.alloc((size_t)d.ncell * w);   // the first is the largest
+        if (!own[0]) (void)hipGetLastError();
       }
-      d.w = wb;
+      if (!own[0]) break;
+      d.w[0] = own[0];
+      d.w[1] = own[1];
     }
   }
   // projection metrics
@@ -866,7 +872,7 @@ void Context::vcycle(const std::vector<Instance*>& S, bool fp64) {
         const int li = I->lev[dpt];
         const DevLevel& d = hL[li];
         // sweeps s and s+1 as a pair (an odd last sweep: half by half)
-        if (d.w && (s & 1 || s + 1 < (pre ? I->pre[dpt] : I->post[dpt]))) {
+        if (d.w[0] && (s & 1 || s + 1 < (pre ? I->pre[dpt] : I->post[dpt]))) {
           const RbPair rp = rb_pair(fp64, d.hx, d.ny, d.nz);
           pairs[rp.tz == 2 ? 0 : 1].push_back({li, rp.blocks});
           continue;

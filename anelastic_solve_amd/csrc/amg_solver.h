@@ -111,6 +111,7 @@ struct Context {
   void drop_graphs();
   bool graph_ok = true;
   bool many = false;             // launches hold many instances (set before the first is added)
+  bool budgeted = false;         // instances keep to the server's estimate of their memory
 
   int init(const amg_config& c);
   ~Context();
