@@ -134,7 +134,7 @@ int amg::divergence_report(amg_handle h, const double* U, const double* V, const
   const int nx = h->I->nx, ny = h->I->ny, nz = h->I->nz;
   const double *dxc = rdze + nz + 2, *dyc = dxc + nx + 2, *dzc = dyc + ny + 2;
   hipStream_t s = h->ctx.stream;
-  double* o = h->ctx.h_out;
+  double* o = h->ctx.h_div;
   launch_divergence(U, V, W, div, rdxc, rdyc, rdzc, dxc, dyc, dzc, nx, ny, nz, partial, s);
   launch_divergence_finalize(partial, divergence_blocks(nx, ny, nz), o, s);
   AMG_HIP(hipGetLastError());

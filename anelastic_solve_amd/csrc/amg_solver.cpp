@@ -26,7 +26,7 @@ inline int cdiv(long long a, long long b) { return (int)((a + b - 1) / b); }
 
 // d_out/h_out hold four regions of kOutRegion doubles: [0] per-instance norms
 // (4 per instance), [1] unused, [2] relmax changes (2 per instance),
-// [3] weighted sums (1 per instance).
+// [3] weighted sums (1 per instance); behind h_out's, h_div.
 constexpr size_t kOutRegion = (size_t)kMaxInstances * 4;
 
 // Launch fn(ll, item_offset, block_offset) over chunks of at most kMaxItems items.
@@ -120,7 +120,8 @@ int Context::init(const amg_config& c) {
   }
   AMG_HIP(hipGetDevice(&device));
   AMG_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-  AMG_HIP(hipHostMalloc((void**)&h_out, sizeof(double) * kOutRegion * 4, hipHostMallocDefault));
+  AMG_HIP(hipHostMalloc((void**)&h_out, sizeof(double) * (kOutRegion * 4 + kDivVals), hipHostMallocDefault));
+  h_div = h_out + kOutRegion * 4;
   AMG_HIP(hipMalloc((void**)&d_out, sizeof(double) * kOutRegion * 4));
   AMG_HIP(hipMalloc((void**)&d_igate, sizeof(ItemGate) * kMaxInstances));
   AMG_HIP(hipHostMalloc((void**)&h_igate, sizeof(ItemGate) * kMaxInstances, hipHostMallocDefault));

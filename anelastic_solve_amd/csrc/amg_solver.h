@@ -102,6 +102,7 @@ struct Context {
   size_t cap_partial = 0;
   double* d_out = nullptr;       // per-item results
   double* h_out = nullptr;       // pinned mirror
+  double* h_div = nullptr;       // the divergence report's results, apart from a solve's (pinned)
   ItemGate* d_igate = nullptr;   // per-instance gates, kMaxInstances
   ItemGate* h_igate = nullptr;   // and their pinned mirror
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
