@@ -81,26 +81,30 @@ size_t partial_blocks(const Instance& I) {
   return (size_t)b + 1;
 }
 
-size_t cycle_bytes(const Instance& I, const std::vector<DevXfer>& X) {
-  // X: the instance's own transfers, X[l] from level l to level l+1
+size_t cycle_bytes(const Instance& I, const std::vector<DevLevel>& D, const std::vector<DevXfer>& X) {
+  // D, X: the instance's own levels and transfers, X[l] from level l to l+1
   const double w = I.fp64 ? 8.0 : 4.0;
   double b = 0.0;
   const int L = (int)I.H.lv.size();
   // levels with smoothing and transfers: above the direct level, or every
-  // level but the coarsest; a direct level reads f and writes u.  The
-  // restriction reads u and b (2w per fine cell, w/8 written); the
-  // prolongation reads and writes u (2w, w/8 read), or half of it when the
-  // level's post-smoothing rewrites the other half (DevXfer::skip, 2:2:2);
-  // the marching restriction skips b and the outside neighbours of the
-  // cells whose residual the pre-smoothing solved (DevXfer::rskip: w/2
-  // less).  Both apply to the V-cycle's own transfers, above the coarse tail.
+  // level but the coarsest; a direct level reads f and writes u.  A sweep's two
+  // half-sweeps each read half of b and of u and write half of u (3w per cell);
+  // point sweeps run in pairs (DevLevel::w) read b and half of u and write u
+  // (2.5w), an odd last one half by half.  The restriction reads u and b (2w
+  // per fine cell, w/8 written), or half of b and, of the other half, what
+  // the first half's stencils need (w/2 less) when the pre-smoothing solved the
+  // residuals of the rest (DevXfer::rskip); the prolongation reads and writes u
+  // (2w, w/8 read), or half of it when the level's post-smoothing rewrites the
+  // other half (DevXfer::skip, 2:2:2).  Both apply to the V-cycle's own
+  // launches, above the coarse tail.
   const int top = I.ld >= 0 ? I.ld : L - 1;
   for (int l = 0; l < top; ++l) {
     const DevXfer& x = X[(size_t)l];
     const bool cyc = l < I.lc();
     const double xfer = (cyc && x.rskip != kXferSkipNone ? 1.625 : 2.125) +
                         (cyc && x.skip != kXferSkipNone ? 1.125 : 2.125);
-    b += w * (double)I.H.lv[l].ncell() * (3.0 * (I.pre[l] + I.post[l]) + xfer);
+    auto sweeps = [&](int n) { return 3.0 * n - (cyc && D[(size_t)l].w[0] ? 0.5 * (n & ~1) : 0.0); };
+    b += w * (double)I.H.lv[l].ncell() * (sweeps(I.pre[l]) + sweeps(I.post[l]) + xfer);
   }
   if (I.ld >= 0) b += 2.0 * w * (double)I.H.lv[I.ld].ncell();
   const double n0 = (double)I.H.lv[0].ncell();
@@ -607,7 +611,7 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
     if (!I->d_met) return fail();
     AMG_HIP(hipMemcpy(I->d_met, m.data(), m.size() * 8, hipMemcpyHostToDevice));
   }
-  I->bytes_per_cycle = cycle_bytes(*I, newX);
+  I->bytes_per_cycle = cycle_bytes(*I, newL, newX);
   I->bytes_corr = (size_t)((I->fp64 ? 16.0 : 32.0) * (double)I->H.lv[0].ncell());
   I->bytes_vcycle = I->bytes_per_cycle - I->bytes_corr;
   // paired cycles: mixed precision, the residual stop rule, and a finest
