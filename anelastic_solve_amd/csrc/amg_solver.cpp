@@ -1446,6 +1446,22 @@ int Context::run_kernel(Instance* I, int which, int level, int reps, double* byt
     form = which < 12 ? 1 : 2;
     which = (which & 1) ? 4 : 0;
   }
+  if (which == 18) {
+    // the coarse tail of levels whose columns share one matrix
+    if (I->ld >= 0 || I->tail_line == 0 || level != I->l0) {
+      set_error("amg_run_kernel: 18 is the line tail, from the first level that it cycles");
+      return AMG_EINVAL;
+    }
+    LaunchList ll;
+    std::memset(&ll, 0, sizeof ll);
+    ll.nitems = ll.nblocks = 1;
+    ll.items[0] = I->tail;
+    ll.prefix[1] = 1;
+    for (int r = 0; r < reps; ++r) launch_tail_line(dL, dT, ll, I->tail_line, stream);
+    AMG_HIP(hipGetLastError());
+    if (bytes) *bytes = 2.0 * w * d.ncell;
+    return AMG_OK;
+  }
   if (which == 0 || which == 4 || which == 6) {
     items.push_back({I->lev[level], zline ? cdiv((long long)d.hx * d.ny, 64)
                                           : cdiv((long long)d.hx * d.ny * d.nz, kBlock)});

@@ -298,8 +298,11 @@ int amg_server_drain(amg_server s);
  *             rewrites without reading them
  *         16: the V-cycle's residual + restriction level -> level+1, which
  *             takes as zero the residuals that the level's last
- *             pre-smoothing half-sweep (black) solved (marching restriction
- *             only; otherwise as 1)
+ *             pre-smoothing half-sweep (black) solved (2:2:2 marching or
+ *             four-lane restriction; otherwise as 1)
+ *         18: the coarse tail of levels whose columns share one matrix: one
+ *             sub-V-cycle from zero of 'level' and below in one launch
+ *             (AMG_EINVAL unless the V-cycle runs such a tail from 'level' on)
  * Returns the kernel's algorithmic bytes per launch.  The caller times the
  * stream (amg_stream) with its own events. */
 int amg_run_kernel(amg_handle h, int which, int level, int precision, int reps, double* bytes);
