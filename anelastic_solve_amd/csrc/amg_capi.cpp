@@ -460,7 +460,7 @@ int amg_cn_advance_device(amg_handle h, const double* veltemp1, double* veltemp2
     AMG_HIP(hipMalloc((void**)&h->d_cn, most));
     AMG_HIP(hipHostMalloc((void**)&h->h_cn, most, hipHostMallocDefault));
   }
-  const std::vector<double> table = cn_table(rows, G.nx, G.ny, rkdt);
+  const std::vector<double> table = cn_table(rows, G.nx, G.ny);
   std::memcpy(h->h_cn, table.data(), sizeof(double) * table.size());
   launch_cn_table(h->h_cn, h->d_cn, (int)table.size(), s);
   const double *rho, *rdxc, *rdyc, *rdzc, *rdxe, *rdye, *rdze;

@@ -59,7 +59,7 @@ int plan_cn(const FlowGrid& G, int var, double rkdt, double rRe, double rPr, dou
 // The table a launch reads, as doubles: the rows themselves for the serial
 // kernel, or the segmented kernel's (cn_segmented).
 bool cn_segmented(int nx, int ny, int nz);
-std::vector<double> cn_table(const std::vector<CnRow>& rows, int nx, int ny, double rkdt);
+std::vector<double> cn_table(const std::vector<CnRow>& rows, int nx, int ny);
 size_t cn_table_doubles(int nz);   // at most
 // n doubles of it from pinned host memory to the device.
 void launch_cn_table(const double* host, double* table, int n, hipStream_t s);

@@ -414,20 +414,23 @@ __global__ __launch_bounds__(kFlowBlock) void k_cn_column(const double* __restri
 //   forward   G_k = G'_k + PF_k G_{r0-1},  PF_k = prod_{i=r0..k} ap_i,          G' from G_{r0-1} = 0,
 //   backward  x_k = x'_k + QB_k x_{r1},    QB_k = prod_{i=k..r1-1} (-c_i/bp_i), x' from x_{r1} = 0.
 // Each wave solves its segment, the segments' end values are chained through
-// LDS (a scan over at most 16 segments), and each row adds its carry term: the
-// serial kernel's result to rounding (its products of constants are made once,
-// and multiply-adds are fused).  The wall rows 0 and nz+1 are constant rows:
-// their right-hand sides are numbers.  Every load comes before the first
-// barrier and every store after the last, so the column is rewritten in place.
+// LDS (a scan over at most 16 segments), and each row adds its carry term.  The
+// right-hand side is the serial kernel's, operation for operation (with products
+// of constants made once and fused multiply-adds it was nearer to the exact
+// value, 1.5e-16 against 1.6e-16, but further from the reference's evaluation:
+// 1.9e-16); the solve is the serial kernel's to rounding.  The wall rows 0 and
+// nz+1 are constant rows: their right-hand sides are numbers.  Every load comes
+// before the first barrier and every store after the last, so the column is
+// rewritten in place.
 //
 // It reads and writes each value once (24 B/cell, 32 with the pressure) and
 // is bound by memory as long as two 1024-lane workgroups share a CU, one's
 // loads under the other's chains: hence at most 64 registers, which is why the
 // table's backward part goes through LDS and rows are addressed as a scalar
 // row offset plus one lane offset (raw buffers).  256^3 u with the pressure
-// (549 MB): 135 us; 161 with 86 registers and one workgroup per CU.
+// (549 MB): 136 us; 161 with 86 registers and one workgroup per CU.
 constexpr int kCnSeg = 16;     // rows per wave and waves per column group, at most
-constexpr int kCnFwd = 6;      // table words of a row: e1 e2 ap pz cval kind
+constexpr int kCnFwd = 9;      // table words of a row: c1 m1 c2 m2 m3 pz ap cval kind
 constexpr int kCnBack = 4;     // and of its backward part: PF 1/bp c QB
 struct CnEnds {
   double g0, c0, rb0;          // row 0: right-hand side, -c/bp of its super-diagonal, 1/bp
@@ -440,7 +443,8 @@ __global__ __launch_bounds__(1024, 8) void k_cn_seg(const double* __restrict__ v
                                                     const double* __restrict__ T,
                                                     const double* __restrict__ rdxe,
                                                     const double* __restrict__ rdye, int nx, int ny,
-                                                    int nz, int S, double f1, double f23, double rkdt) {
+                                                    int nz, int S, double f1, double f2, double f3,
+                                                    double rkdt, double h) {
   constexpr int N = kCnSeg;
   __shared__ double gend[N][64], xfirst[N][64], xtop[64], back[N][N * kCnBack];
   const int lane = threadIdx.x;
@@ -468,7 +472,7 @@ __global__ __launch_bounds__(1024, 8) void k_cn_seg(const double* __restrict__ v
   };
   const unsigned bl = (unsigned)(j * (nx + 2) + i) * 8u;
   const unsigned bn = bl + (PV == 1 ? 8u : (unsigned)(nx + 2) * 8u);   // the pressure's x or y neighbour
-  const double dm = PV == 1 ? rkdt * rdxe[i] : (PV == 2 ? rkdt * rdye[j] : 0.0);
+  const double dm = PV == 1 ? rdxe[i] : (PV == 2 ? rdye[j] : 0.0);
   // row q of the segment is q+1 rows past the buffers' start; rows past the
   // segment repeat its last row's upper neighbour
   auto row = [&](int q) { return (unsigned)min(q + 1, nz + 2 - r0) * plane; };
@@ -489,14 +493,13 @@ __global__ __launch_bounds__(1024, 8) void k_cn_seg(const double* __restrict__ v
 #pragma unroll
     for (int q = 0; q < m; ++q) {
       const double* R = T + kCnFwd * min(r0 + c0 + q, nz + 1);
-      // the increments first, so that the field's own value is rounded once
-      double r = f23 * a1[q];
-      if constexpr (PV == 1 || PV == 2) r = __builtin_fma(-dm, pb[q] - pa[q], r);
-      if constexpr (PV == 3) r = __builtin_fma(-R[3], pa[q + 1] - pa[q], r);
-      r = __builtin_fma(R[0], v[q + 2] - v[q + 1], r);
-      r = __builtin_fma(-R[1], v[q + 1] - v[q], r);
-      r = __builtin_fma(f1, v[q + 1], r);
-      G[c0 + q] = R[5] != 0.0 ? R[4] : r;
+      // the serial kernel's operations in their order
+      double r = f1 * v[q + 1] + f2 * a1[q] * f3;
+      if constexpr (PV == 1 || PV == 2) r = r - rkdt * (pb[q] - pa[q]) * dm;
+      if constexpr (PV == 3) r = r - rkdt * (pa[q + 1] - pa[q]) * R[5];
+      const double tv = R[0] * (v[q + 2] - v[q + 1]) * R[1] - R[2] * (v[q + 1] - v[q]) * R[3];
+      r = r + h * tv * R[4];
+      G[c0 + q] = R[8] != 0.0 ? R[7] : r;
     }
   };
   if (len == N) {
@@ -510,7 +513,7 @@ __global__ __launch_bounds__(1024, 8) void k_cn_seg(const double* __restrict__ v
 #pragma unroll
   for (int q = 0; q < N; ++q)
     if (q < len) {
-      g = __builtin_fma(T[kCnFwd * (r0 + q) + 2], g, G[q]);
+      g = __builtin_fma(T[kCnFwd * (r0 + q) + 6], g, G[q]);
       G[q] = g;
     }
   gend[w][lane] = g;
@@ -824,7 +827,7 @@ size_t cn_table_doubles(int nz) {
                   kCnFwd * (size_t)(nz + 2) + sizeof(CnEnds) / 8 + kCnSeg * kCnSeg * kCnBack);
 }
 
-std::vector<double> cn_table(const std::vector<CnRow>& rows, int nx, int ny, double rkdt) {
+std::vector<double> cn_table(const std::vector<CnRow>& rows, int nx, int ny) {
   const int nz = (int)rows.size() - 2;
   std::vector<double> t;
   if (!cn_segmented(nx, ny, nz)) {
@@ -832,12 +835,8 @@ std::vector<double> cn_table(const std::vector<CnRow>& rows, int nx, int ny, dou
     std::memcpy(t.data(), rows.data(), sizeof(CnRow) * rows.size());
     return t;
   }
-  // products of constants in extended precision, rounded once
-  typedef long double ld;
-  const ld h = (ld)rkdt * 0.5;
   for (const CnRow& R : rows) {
-    const double fwd[kCnFwd] = {(double)(h * R.c1 * R.m1 * R.m3), (double)(h * R.c2 * R.m2 * R.m3), R.ap,
-                                rkdt * R.pz, R.cval, R.kind ? 1.0 : 0.0};
+    const double fwd[kCnFwd] = {R.c1, R.m1, R.c2, R.m2, R.m3, R.pz, R.ap, R.cval, R.kind ? 1.0 : 0.0};
     t.insert(t.end(), fwd, fwd + kCnFwd);
   }
   const CnRow &B = rows.front(), &E = rows.back();
@@ -849,7 +848,7 @@ std::vector<double> cn_table(const std::vector<CnRow>& rows, int nx, int ny, dou
   for (int r0 = 1, w = 0; r0 <= nz; r0 += S, ++w) {
     const int len = std::min(S, nz + 1 - r0);
     double* b = back.data() + (size_t)w * kCnSeg * kCnBack;
-    ld pf = 1.0, qb = 1.0;
+    long double pf = 1.0, qb = 1.0;   // (products in extended precision, rounded once)
     for (int q = 0; q < len; ++q) {
       const CnRow& R = rows[r0 + q];
       pf = R.ap * pf;
@@ -858,7 +857,7 @@ std::vector<double> cn_table(const std::vector<CnRow>& rows, int nx, int ny, dou
       b[q * kCnBack + 2] = R.c;
     }
     for (int q = len - 1; q >= 0; --q) {
-      qb = -((ld)rows[r0 + q].c / rows[r0 + q].bp) * qb;
+      qb = -((long double)rows[r0 + q].c / rows[r0 + q].bp) * qb;
       b[q * kCnBack + 3] = (double)qb;
     }
   }
@@ -874,11 +873,11 @@ void launch_cn_column(const double* v1, double* v2, const double* p, const doubl
                       const double* rdxe, const double* rdye, int nx, int ny, int nz, double f1,
                       double f2, double f3, double rkdt, int var, hipStream_t s) {
   const int pv = (p != nullptr && var <= 3) ? var : 0;
+  const double h = rkdt * 0.5;
   if (cn_segmented(nx, ny, nz)) {
     const int S = (nz + kCnSeg - 1) / kCnSeg, P = (nz + S - 1) / S;
     const dim3 g(cdiv((long long)nx * ny, 64)), b(64, P);
-    const double f23 = f2 * f3;
-#define CS(V) hipLaunchKernelGGL(k_cn_seg<V>, g, b, 0, s, v1, v2, p, T, rdxe, rdye, nx, ny, nz, S, f1, f23, rkdt)
+#define CS(V) hipLaunchKernelGGL(k_cn_seg<V>, g, b, 0, s, v1, v2, p, T, rdxe, rdye, nx, ny, nz, S, f1, f2, f3, rkdt, h)
     if (pv == 1) CS(1);
     else if (pv == 2) CS(2);
     else if (pv == 3) CS(3);
@@ -886,7 +885,6 @@ void launch_cn_column(const double* v1, double* v2, const double* p, const doubl
 #undef CS
     return;
   }
-  const double h = rkdt * 0.5;
   const CnRow* R = reinterpret_cast<const CnRow*>(T);
   const dim3 g(cdiv((long long)nx * ny, kFlowBlock)), b(kFlowBlock);
 #define CC(V) hipLaunchKernelGGL(k_cn_column<V>, g, b, 0, s, v1, v2, p, R, rdxe, rdye, nx, ny, nz, f1, f2, f3, rkdt, h)
