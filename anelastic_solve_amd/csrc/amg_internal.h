@@ -358,10 +358,12 @@ void launch_coarse(bool fp64, const DevLevel* L, const LaunchList& ll, hipStream
 // rows or modes, one workgroup each (a level of 64^3 fills the device with
 // 256): 'planes' has nz*ny/kDirectCols blocks per item, 'slabs'
 // nx*ny/kDirectCols; lds = the largest direct_lds() of the items.
-// direct_fits: a plane's operands (the plane, the y matrix, 16 columns of the
-// x matrix) and the z pass's are at most one CU's LDS.  (A larger FP32 level
-// fits -- 128^3 does -- but its passes take longer than the levels they would
-// replace.)
+// direct_fits: a plane, the y matrix and 16 columns of the x matrix, and the
+// z pass's matrices, together take no more than one CU's LDS.  The passes hold
+// less there (direct_lds), so this bounds their work, not their memory; past it
+// the direct solve wins and loses (us per cycle, cycled on against direct; z-line,
+// point smoother): FP64 128x128x16 189, 154 and 146, 145; FP64 256x64x16 203, 187
+// and 156, 169; FP32 256x128x8 118, 131 and 122, 144.
 constexpr long long kDirectCells = 1 << 18;
 constexpr int kDirectCols = 16;
 constexpr int kDirectMaxNz = 64;

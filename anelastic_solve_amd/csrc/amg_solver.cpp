@@ -538,7 +538,7 @@ int Context::add_instance(const amg_grid& g, Instance** out, Hierarchy* built) {
   // separable direct solve of the first level below the finest, above the
   // coarse tail (the tail solves small levels in one launch), that the
   // direct solve takes: at most kDirectCells cells, nx and ny multiples of
-  // 16, nz <= kDirectMaxNz, direct_fits; the levels below it
+  // 16, nz <= kDirectMaxNz, direct_fits (amg_internal.h); the levels below it
   // are not cycled.  A mixed solve computes it in FP32 (its tables are
   // FP32), an FP64 one in FP64.
   if (cfg.coarse_direct != 0) {
