@@ -428,7 +428,7 @@ __global__ __launch_bounds__(kFlowBlock) void k_cn_column(const double* __restri
 // loads under the other's chains: hence at most 64 registers, which is why the
 // table's backward part goes through LDS and rows are addressed as a scalar
 // row offset plus one lane offset (raw buffers).  256^3 u with the pressure
-// (549 MB): 136 us; 161 with 86 registers and one workgroup per CU.
+// (549 MB): 135 us; 161 with 86 registers and one workgroup per CU.
 constexpr int kCnSeg = 16;     // rows per wave and waves per column group, at most
 constexpr int kCnFwd = 9;      // table words of a row: c1 m1 c2 m2 m3 pz ap cval kind
 constexpr int kCnBack = 4;     // and of its backward part: PF 1/bp c QB

@@ -3624,9 +3624,9 @@ void launch_zline(bool fp64, const DevLevel* L, const LaunchList& ll, int parity
   //   takes the short form, FP64 (which the short form leaves no registers)
   //   the lean one;
   // - more: blocks pair up on the CUs, the lean form's registers allowing.
-  //   FP64 needs the 32-column shape for that (256^3 48.1 -> 42.9 us, 4.18 ->
+  //   FP64 needs the 32-column shape for that (256^3 48.4 -> 42.9 us, 4.16 ->
   //   4.69 TB/s, where the lone 16-wave group of a CU loaded and solved in
-  //   turn; 512x256x128 41.4 -> 40.2; of 140 groups 11.2 -> 12.0).
+  //   turn; 512x256x128 41.0 -> 40.4; of 140 groups 11.2 -> 12.0).
   const int cus = device_cus();
   const bool few = form == 0 && segs >= 2 && 2 * ll.nblocks <= cus;
   const bool many = form == 0 && ll.nblocks > cus;

@@ -105,6 +105,7 @@ int amg_server_s::bind(Member& m) {
     return n;
   };
   // the hierarchy's size is known only after building it; estimate from the grid
+  // (an upper bound as long as fields are what Context::budgeted leaves)
   const double ncell = (double)m.grid.nx * m.grid.ny * m.grid.nz;
   const double w = ctx.cfg.precision == AMG_FP64 ? 8.0 : 4.0;
   const double est = ncell * (8.0 / 7.0) * w * 2.5 + ncell * 8.0 * (ctx.cfg.precision == AMG_FP64 ? 1.0 : 3.0);
