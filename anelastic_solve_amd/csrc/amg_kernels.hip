@@ -891,8 +891,8 @@ __global__ __launch_bounds__(H ? 512 : 1024, LEAN ? 32 / (int)sizeof(T) : (H ? 2
 
 // ---------------------------------------------------------------------------
 // The FP32 half-sweep of a level whose columns all have the same x/y diagonal
-// share (both horizontal axes uniform, no wall in them): every column then
-// has the same matrix, so the pivots, the segments' coupling solutions and
+// share (both horizontal axes uniform, periodic or with Dirichlet walls): every
+// column then has the same matrix, so the pivots, the segments' coupling solutions and
 // the whole cyclic reduction of the interface matrix are the same numbers in
 // every column.  They are computed once, when the level is built
 // (k_zline_table), with the operations of zline_group, and the sweep keeps
